@@ -55,7 +55,8 @@ bool valid_bc(int b) { return b >= MMF_BC_FREE_FLOW && b <= MMF_BC_PERIODIC; }
 // 2D order 1 from 2^18 cells (64^2 56 vs 28 us per step, 512^2 equal, 1024^2
 // 137 vs 188), 3D order 1 from 2^20 (32^3 273 vs 37 us, 96^3 319 vs 193,
 // 128^3 271 vs 379), 2D order 2 from 2^20 (below it the tile kernel, then the
-// gather kernel).
+// gather kernel).  Order-1 grids without ghost cells or per-face conditions go
+// to the brick kernel below brick_auto_max.
 bool use_march(const mmf_ctx *ctx) {
   if (ctx->kernel == mmf::KERNEL_GATHER || !mmf::march_shape_supported(ctx->g, ctx->shape)) return false;
   if (ctx->kernel == mmf::KERNEL_AUTO) {
@@ -75,12 +76,29 @@ bool tile_applies(const mmf_ctx *ctx) {
 // 146, the tile kernel's fixed per-block latency no longer hidden).
 constexpr int64_t TILE_AUTO_MAX_N = (int64_t)1 << 18;
 
+// AUTO takes the brick kernel for order-1 grids below this size (us per step,
+// gather / best marching shape / brick; MI355X).  3D: 32^3 37 / 36 / 23, 64^3
+// 65 / 57 / 48, 100 x 90 x 84 173 / 163 / 108, 168 x 133 x 32 156 / 104 / 98,
+// but 128^3 385 / 155 / 225: the marching kernel builds fewer halo tuples.
+// 2D: 64^2 29 / 76 / 19, 500 x 400 55 / 57 / 31.  Strips without a reflecting
+// x border or a body march without branches and issue fewer instructions per
+// cell: with several grids in flight 1000 x 600 takes 43 us per step against
+// 46 (alone 79 against 60), so they keep their sizes; the others (1448^2,
+// reflecting, 316 / 167; 1024^2 with a cylinder 168 / 107) go to the bricks.
+int64_t brick_auto_max(const GridDev &g) {
+  if (g.dim == 3) return (int64_t)1 << 20;
+  const bool flat_strips = !g.flags && (g.periodic[0] || (g.bc[0] == MMF_BC_FREE_FLOW && g.bc[1] == MMF_BC_FREE_FLOW));
+  return (int64_t)1 << (flat_strips ? 18 : 22);
+}
+
 // The stage kernel of the next launches.  With the learned reconstruction on:
 // the tile kernel, or (GATHER) the face-state + flux kernel pair.
 int kernel_used(const mmf_ctx *ctx) {
   if (ctx->learn_on) return ctx->kernel == mmf::KERNEL_GATHER ? mmf::KERNEL_GATHER : mmf::KERNEL_TILE;
   if (ctx->kernel == mmf::KERNEL_TILE) return tile_applies(ctx) ? mmf::KERNEL_TILE : mmf::KERNEL_GATHER;
   if (ctx->kernel == mmf::KERNEL_AUTO && tile_applies(ctx) && ctx->g.N < TILE_AUTO_MAX_N) return mmf::KERNEL_TILE;
+  if (ctx->kernel == mmf::KERNEL_AUTO && ctx->g.N < brick_auto_max(ctx->g) && mmf::brick_supported(ctx->g))
+    return mmf::KERNEL_BRICK;
   return use_march(ctx) ? mmf::KERNEL_MARCH : mmf::KERNEL_GATHER;
 }
 
@@ -106,6 +124,8 @@ int launch_stage_on(mmf_ctx *ctx, int stage, int mode, double *U, double *R, dou
     plain.blend = 1.0;
     e = mmf::launch_stage_learned(ctx->g, ctx->learn_on ? ctx->learn : plain, stage, mode, U, R, W, R, W, U, ctx->dctrl,
                                   ctx->stream);
+  } else if (kind == mmf::KERNEL_BRICK) {
+    e = mmf::launch_stage_brick(ctx->g, stage, mode, U, R, W, R, W, U, ctx->dctrl, ctx->stream);
   } else if (kind == mmf::KERNEL_MARCH) {
     e = mmf::launch_stage_march(ctx->g, ctx->shape, stage, mode, U, R, W, R, W, U, ctx->dctrl, ctx->stream);
   } else {
@@ -369,7 +389,7 @@ int mmf_set_march_blocks(mmf_ctx *ctx, int32_t blocks) {
 
 int mmf_get_kernel(const mmf_ctx *ctx, int32_t *kind, int32_t *tile_rows, int32_t *chunk) {
   if (!ctx) return MMF_ERR_INVALID;
-  if (kind) *kind = kernel_used(ctx);
+  if (kind) *kind = (kernel_used(ctx) == mmf::KERNEL_BRICK) ? (int)mmf::KERNEL_GATHER : kernel_used(ctx);
   if (tile_rows) *tile_rows = ctx->shape.ty;
   // 0: the planes of all tiles spread evenly over the blocks (3D order 1)
   if (chunk) *chunk = (ctx->shape.seg_blocks > 0 && ctx->g.dim == 3 && ctx->g.order == 1) ? 0 : ctx->shape.chunk;
@@ -878,7 +898,8 @@ int ensure_tiles(mmf_ctx *ctx) {
 }
 
 int ensure_lam(mmf_ctx *ctx) {
-  const bool early = kernel_used(ctx) == mmf::KERNEL_MARCH && mmf::march_early(ctx->g);
+  const int used = kernel_used(ctx);
+  const bool early = (used == mmf::KERNEL_MARCH && mmf::march_early(ctx->g)) || used == mmf::KERNEL_BRICK;
   if (!early) {
     ctx->lam_valid = false;
     return MMF_OK;
@@ -897,9 +918,10 @@ int enqueue_steps(mmf_ctx *ctx, int64_t nsteps) {
       int rc = launch_stage_timed(ctx, stage, mmf::MODE_STEP);
       if (rc != MMF_OK) return rc;
     }
-    // the tile kernel's and the 3D marching kernel's stage-3 launches advance the time themselves
+    // the tile, brick and 3D marching kernels' stage-3 launches advance the time themselves
     const int used = kernel_used(ctx);
-    if (used == mmf::KERNEL_TILE || (used == mmf::KERNEL_MARCH && ctx->g.dim == 3)) continue;
+    if (used == mmf::KERNEL_TILE || used == mmf::KERNEL_BRICK || (used == mmf::KERNEL_MARCH && ctx->g.dim == 3))
+      continue;
     hipError_t e = mmf::launch_advance(ctx->dctrl, ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, e, "advance kernel");
   }

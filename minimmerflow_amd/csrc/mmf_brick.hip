@@ -1,0 +1,387 @@
+// mmf_brick.hip -- order-1 stage kernel of small and ordinary grids (gfx950).
+//
+// A block owns a brick of BX x BY x BZ cells, one thread per cell, and the
+// brick's one-cell halo, at most one halo cell per thread.  Every thread
+// loads its cell and its halo cell at once (no load waits for another: the
+// per-cell gather kernel it replaces here spent most of a launch on a chain of
+// dependent neighbour loads and 64-bit index divisions, and built the flux
+// tuple of every neighbour again: seven tuples per 3D cell instead of two),
+// builds both flux tuples -- every division and the square root of the
+// reference's per-face evaluation -- into LDS, and after one barrier evaluates
+// the faces of its cell from the neighbours' slots.  A border face's halo slot
+// holds the virtual state's tuple, so the faces have no border branches.  The
+// tuples are the unit of work, so the brick needs no march and no second
+// barrier, and a launch is one pass of about one load latency, two tuples and
+// 2 DIM faces.
+//
+// dt is known before stage 1 (Ctrl::lam_now, as in the marching kernel):
+// stage 1 writes W1 = U + dt R / V, stage 3 gathers the next step's maximum
+// and closes the step, so a step is three launches.
+//
+// Each cell's residual is summed in the reference's face order: results equal
+// the gather kernel's and the oracle's bit for bit.
+#include <hip/hip_runtime.h>
+
+#include "mmf_device.hpp"
+#include "mmf_internal.hpp"
+#include "mmf_stage.hpp"
+
+namespace mmf {
+
+namespace {
+
+constexpr int NTUP = 11;  // c[5], vel[3], p, a, H
+
+template <int NS>
+__device__ __forceinline__ void put_tup(double *lds, int slot, const Tup &t) {
+#pragma unroll
+  for (int k = 0; k < NF; ++k) lds[k * NS + slot] = t.c[k];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) lds[(5 + a) * NS + slot] = t.vel[a];
+  lds[8 * NS + slot] = t.p;
+  lds[9 * NS + slot] = t.a;
+  lds[10 * NS + slot] = t.H;
+}
+
+template <int NS>
+__device__ __forceinline__ void get_tup(const double *lds, int slot, Tup &t) {
+#pragma unroll
+  for (int k = 0; k < NF; ++k) t.c[k] = lds[k * NS + slot];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) t.vel[a] = lds[(5 + a) * NS + slot];
+  t.p = lds[8 * NS + slot];
+  t.a = lds[9 * NS + slot];
+  t.H = lds[10 * NS + slot];
+}
+
+__device__ __forceinline__ unsigned long long wave_max(unsigned long long b) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const unsigned long long o = __shfl_xor(b, off, 64);
+    b = (o > b) ? o : b;
+  }
+  return b;
+}
+
+}  // namespace
+
+// MASK: the grid has cell flags (every fluid cell solved).  P2: A and V are
+// powers of two (the faces hand over unscaled sums, scaled once at the update;
+// the same doubles).
+template <int DIM, int BX, int BY, int BZ, int STAGE, bool MASK, bool P2>
+__global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X, const double *U, double *out,
+                                                      Ctrl *ctrl, int mode, int nbx, int nby) {
+  constexpr int NT = BX * BY * BZ;
+  constexpr int HX = BY * BZ, HY = BX * BZ, HZ = (DIM == 3) ? BX * BY : 0;
+  constexpr int XM = NT, XP = XM + HX, YM = XP + HX, YP = YM + HY, ZM = YP + HY, ZP = ZM + HZ;
+  constexpr int H = 2 * (HX + HY + HZ);
+  constexpr int NS = NT + H;
+  constexpr int NW = (NT + 63) / 64;
+  static_assert(H <= NT, "one halo cell per thread");
+  __shared__ double lds[NTUP * NS];
+  __shared__ uint8_t lfl[MASK ? NS : 1];
+  __shared__ unsigned int sneg[NW];
+  __shared__ unsigned long long red[2 * NW];
+
+  const int tid = threadIdx.x;
+  const bool step = mode == MODE_STEP;
+  const int tile = xcd_range((int)blockIdx.x, (int)gridDim.x);
+  const int bz = (DIM == 3) ? tile / (nbx * nby) : 0;
+  const int by = (tile / nbx) % nby, bx = tile % nbx;
+  const int nx = (int)g.n[0], ny = (int)g.n[1], nz = (DIM == 3) ? (int)g.n[2] : 1;
+  const int x0 = bx * BX, y0 = by * BY, z0 = bz * BZ;
+  const int w = (nx - x0 < BX) ? nx - x0 : BX;
+  const int h = (ny - y0 < BY) ? ny - y0 : BY;
+  const int d = (DIM == 3) ? ((nz - z0 < BZ) ? nz - z0 : BZ) : 1;
+  auto index = [&](int x, int y, int z) { return (uint32_t)x + (uint32_t)nx * ((uint32_t)y + (uint32_t)ny * (uint32_t)z); };
+
+  const int lx = tid % BX, ly = (tid / BX) % BY, lz = (DIM == 3) ? tid / (BX * BY) : 0;
+  const bool valid = lx < w && ly < h && lz < d;
+  const uint32_t idx = valid ? index(x0 + lx, y0 + ly, z0 + lz) : index(x0, y0, z0);
+
+  // this thread's halo cell (hside: the side it lies on, -1 for none); across
+  // a non-periodic border the inner cell, whose virtual state it builds
+  int hside = -1;
+  bool hborder = false;
+  uint32_t hidx = idx;
+  if (tid < H) {
+    const int s = XM + tid;
+    int i, j, k = 0;  // position in the brick, the outer coordinate one off it
+    if (s < YM) {
+      const int r = (s < XP) ? s - XM : s - XP;
+      hside = (s < XP) ? 0 : 1;
+      i = (s < XP) ? -1 : w;
+      j = r % BY;
+      k = r / BY;
+    } else if (s < ZM || DIM == 2) {
+      const int r = (s < YP) ? s - YM : s - YP;
+      hside = (s < YP) ? 2 : 3;
+      j = (s < YP) ? -1 : h;
+      i = r % BX;
+      k = r / BX;
+    } else {
+      const int r = (s < ZP) ? s - ZM : s - ZP;
+      hside = (s < ZP) ? 4 : 5;
+      k = (s < ZP) ? -1 : d;
+      i = r % BX;
+      j = r / BX;
+    }
+    const int a = hside >> 1;
+    if ((a == 0 || i < w) && (a == 1 || j < h) && (a == 2 || k < d)) {
+      int q[3] = {x0 + i, y0 + j, z0 + k};
+      const int n[3] = {nx, ny, nz};
+#pragma unroll
+      for (int b = 0; b < DIM; ++b) {
+        if (q[b] >= 0 && q[b] < n[b]) continue;
+        if (g.periodic[b]) q[b] += (q[b] < 0) ? n[b] : -n[b];
+        else {
+          hborder = true;
+          q[b] += (q[b] < 0) ? 1 : -1;
+        }
+      }
+      hidx = index(q[0], q[1], q[2]);
+    } else {
+      hside = -1;
+    }
+  }
+
+  // every load of the launch, none dependent on another
+  const int64_t fs = g.fs;
+  double Xc[NF], Xh[NF], Uc[NF];
+#pragma unroll
+  for (int k = 0; k < NF; ++k) Xc[k] = X[k * fs + idx];
+#pragma unroll
+  for (int k = 0; k < NF; ++k) Xh[k] = X[k * fs + hidx];
+#pragma unroll
+  for (int k = 0; k < NF; ++k) Uc[k] = (STAGE >= 2) ? U[k * fs + idx] : 0.0;
+  uint8_t fc = CELL_FLUID | CELL_SOLVED, fh = CELL_FLUID | CELL_SOLVED;
+  if (MASK) {
+    fc = g.flags[idx];
+    fh = g.flags[hidx];
+  }
+  const bool run = !step || ctrl->t < ctrl->tmax;  // main.cpp:377 loop guard
+  const double dt = step ? step_dt_early(ctrl) : 0.0;
+
+  const bool solved = valid && (!MASK || (fc & CELL_SOLVED));
+  double lam = 0.0;  // stage maximum: the larger side of every face (euler.cpp:232-234)
+  Tup Tc;
+  make_tup(Xc, Tc);
+  put_tup<NS>(lds, tid, Tc);
+  bool neg_here = valid && tup_negative(Tc);
+  if (solved) {
+    // every cell has faces along every axis
+    double um = fabs(Tc.vel[0]);
+#pragma unroll
+    for (int a = 1; a < DIM; ++a) um = lam_acc(um, fabs(Tc.vel[a]));
+    lam = um + Tc.a;
+  }
+  if (MASK) lfl[tid] = fc;
+  if (hside >= 0) {
+    const int a = hside >> 1;
+    if (hborder) {  // euler.cpp:261-376
+      double v[NF];
+      border_state(g, hside, a, Xh, v);
+#pragma unroll
+      for (int k = 0; k < NF; ++k) Xh[k] = v[k];
+    }
+    Tup Th;
+    make_tup(Xh, Th);
+    put_tup<NS>(lds, XM + tid, Th);
+    neg_here = neg_here || tup_negative(Th);
+    if (MASK) lfl[XM + tid] = fh;
+    if (hborder && (!MASK || (fh & CELL_SOLVED))) {
+      const double ua = (a == 0) ? Th.vel[0] : (a == 1) ? Th.vel[1] : Th.vel[2];
+      lam = lam_acc(lam, fabs(ua) + Th.a);
+    }
+  }
+  // a state with negative pressure or density somewhere in the block: its
+  // faces are then counted (below) instead of every face always
+  const unsigned long long nb = __ballot(neg_here);
+  if ((tid & 63) == 0) sneg[tid >> 6] = nb != 0;
+  __syncthreads();
+
+  unsigned int anyneg = 0;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) anyneg |= sneg[i];
+
+  double lam_nx = 0.0;
+  NegCount neg;
+  if (solved) {
+    const int slot_m[3] = {lx > 0 ? tid - 1 : XM + ly + BY * lz, ly > 0 ? tid - BX : YM + lx + BX * lz,
+                           lz > 0 ? tid - BX * BY : ZM + lx + BX * ly};
+    const int slot_p[3] = {lx + 1 < w ? tid + 1 : XP + ly + BY * lz, ly + 1 < h ? tid + BX : YP + lx + BX * lz,
+                           lz + 1 < d ? tid + BX * BY : ZP + lx + BX * ly};
+    // the neighbour's tuple across a face; a fluid-solid face's virtual state
+    // is the reflected own state (main.cpp:271-275, euler.cpp:347-356)
+    auto across = [&](int slot, int a, Tup &N) {
+      if (MASK && ((lfl[slot] ^ fc) & CELL_FLUID)) {
+        double v[NF];
+        reflect_axis(Tc.c, a, v);
+        make_tup(v, N);
+        return true;
+      }
+      get_tup<NS>(lds, slot, N);
+      return false;
+    };
+    const double halfA = P2 ? 1.0 : g.halfA;
+    const int qc[3] = {x0 + lx, y0 + ly, z0 + lz};
+    double rhs[NF] = {0., 0., 0., 0., 0.};  // euler.cpp:142-148
+    bool wall_any = false;
+#pragma unroll
+    for (int a = 0; a < DIM; ++a) {
+      double Fm[NF], Fp[NF];
+      {
+        Tup N;
+        const bool wall = across(slot_m[a], a, N);
+        const double l = face_flux_area(N, Tc, a, P2, g.A, halfA, Fm);
+        if (MASK && wall) lam = lam_acc(lam, l);
+        wall_any = wall_any || wall;
+      }
+      {
+        Tup N;
+        const bool wall = across(slot_p[a], a, N);
+        const double l = face_flux_area(Tc, N, a, P2, g.A, halfA, Fp);
+        if (MASK && wall) lam = lam_acc(lam, l);
+        wall_any = wall_any || wall;
+      }
+      if (g.periodic[a] && qc[a] == (int)g.n[a] - 1) {
+        // the wrap face is first in the reference-order face list
+#pragma unroll
+        for (int k = 0; k < NF; ++k) { rhs[k] -= Fp[k]; rhs[k] += Fm[k]; }
+      } else {
+#pragma unroll
+        for (int k = 0; k < NF; ++k) { rhs[k] += Fm[k]; rhs[k] -= Fp[k]; }
+      }
+    }
+    if (anyneg || wall_any) {
+      // once per face, as the reference evaluates it: every upper face, and
+      // the lower ones that no solved cell has as its upper face
+#pragma unroll
+      for (int a = 0; a < DIM; ++a) {
+        Tup N;
+        const bool border = !g.periodic[a] && qc[a] == 0;
+        const bool wall = across(slot_m[a], a, N);
+        if (border || wall || (MASK && !(lfl[slot_m[a]] & CELL_SOLVED))) neg.add(N, Tc);
+        across(slot_p[a], a, N);
+        neg.add(Tc, N);
+      }
+    }
+
+    double nu[NF];
+#pragma unroll
+    for (int k = 0; k < NF; ++k) {
+      const double r = P2 ? g.halfA * rhs[k] : rhs[k];
+      GridDev gp = g;
+      gp.pow2V = P2;
+      nu[k] = (STAGE == 1) ? (step ? Tc.c[k] + div_vol(gp, dt * r) : r) : rk_update<STAGE>(gp, Uc[k], Tc.c[k], r, dt);
+      if (run) out[k * fs + idx] = nu[k];
+    }
+    if (STAGE == 3) {
+      // the next step's stage-1 maximum: this cell's, and the virtual states
+      // its border and wall faces will have
+      lam_nx = cell_max_eig<DIM>(nu);
+#pragma unroll
+      for (int a = 0; a < DIM; ++a) {
+        bool refl = false;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int slot = s ? slot_p[a] : slot_m[a];
+          const bool border = !g.periodic[a] && (s ? qc[a] == (int)g.n[a] - 1 : qc[a] == 0);
+          if (border) {
+            const int bc = g.bc[2 * a + s];
+            refl = refl || bc == BC_REFLECTING || bc == BC_WALL;
+            if (bc == BC_DIRICHLET) lam_nx = lam_acc(lam_nx, fabs(lds[(5 + a) * NS + slot]) + lds[9 * NS + slot]);
+          } else if (MASK) {
+            refl = refl || !(lfl[slot] & CELL_FLUID);
+          }
+        }
+        if (refl) {
+          double v[NF];
+          Tup V;
+          reflect_axis(nu, a, v);
+          make_tup(v, V);
+          lam_nx = lam_acc(lam_nx, fabs(V.vel[a]) + V.a);
+        }
+      }
+    }
+  } else if (MASK && valid && run && STAGE != 3) {
+    // unsolved (solid) cells: a residual of zero
+    GridDev gp = g;
+    gp.pow2V = P2;
+#pragma unroll
+    for (int k = 0; k < NF; ++k)
+      out[k * fs + idx] = (STAGE == 1) ? (step ? Xc[k] + div_vol(gp, dt * 0.0) : 0.0) : Uc[k];
+  }
+
+  if (!run) return;  // uniform over the grid: t does not change before the step closes
+  if (anyneg || MASK) neg.flush(ctrl, tid);
+  const unsigned long long ml = wave_max(dbits(lam));
+  const unsigned long long mn = (STAGE == 3 && step) ? wave_max(dbits(lam_nx)) : 0ull;
+  if ((tid & 63) == 0) {
+    red[tid >> 6] = ml;
+    red[NW + (tid >> 6)] = mn;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    unsigned long long m = red[0], n = red[NW];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) {
+      m = (red[i] > m) ? red[i] : m;
+      n = (red[NW + i] > n) ? red[NW + i] : n;
+    }
+    stage_max_put(ctrl, step ? STAGE - 1 : 3, m);
+    if (STAGE == 3 && step) lam_put(ctrl, n);
+  }
+  if (STAGE == 3 && step) close_step<true>(ctrl, tid);
+}
+
+template <int DIM, int BX, int BY, int BZ, bool MASK, bool P2>
+static hipError_t launch_brick_p(const GridDev &g, int stage, int mode, const double *U, const double *R,
+                                 const double *W, double *oR, double *oW, double *oU, Ctrl *ctrl, hipStream_t s) {
+  const int nbx = (int)((g.n[0] + BX - 1) / BX), nby = (int)((g.n[1] + BY - 1) / BY);
+  const int nbz = (int)((g.n[2] + BZ - 1) / BZ);
+  const dim3 grid((unsigned)nbx * nby * nbz), block(BX * BY * BZ);
+  // stage 2 reads the W1 that stage 1 wrote into R's buffer
+  switch (stage) {
+    case 1:
+      hipLaunchKernelGGL((k_brick<DIM, BX, BY, BZ, 1, MASK, P2>), grid, block, 0, s, g, U, U, oR, ctrl, mode, nbx, nby);
+      break;
+    case 2:
+      hipLaunchKernelGGL((k_brick<DIM, BX, BY, BZ, 2, MASK, P2>), grid, block, 0, s, g, R, U, oW, ctrl, mode, nbx, nby);
+      break;
+    default:
+      hipLaunchKernelGGL((k_brick<DIM, BX, BY, BZ, 3, MASK, P2>), grid, block, 0, s, g, W, U, oU, ctrl, mode, nbx, nby);
+  }
+  return hipGetLastError();
+}
+
+bool brick_supported(const GridDev &g) {
+  return g.order == 1 && !g.bslot && (g.flags == nullptr || g.ghost_free) && g.N < BRICK_MAX_CELLS;
+}
+
+template <int DIM, int BX, int BY, int BZ>
+static hipError_t launch_brick_s(const GridDev &g, int stage, int mode, const double *U, const double *R,
+                                 const double *W, double *oR, double *oW, double *oU, Ctrl *ctrl, hipStream_t s) {
+  const bool p2 = g.pow2A && g.pow2V;
+  if (g.flags)
+    return p2 ? launch_brick_p<DIM, BX, BY, BZ, true, true>(g, stage, mode, U, R, W, oR, oW, oU, ctrl, s)
+              : launch_brick_p<DIM, BX, BY, BZ, true, false>(g, stage, mode, U, R, W, oR, oW, oU, ctrl, s);
+  return p2 ? launch_brick_p<DIM, BX, BY, BZ, false, true>(g, stage, mode, U, R, W, oR, oW, oU, ctrl, s)
+            : launch_brick_p<DIM, BX, BY, BZ, false, false>(g, stage, mode, U, R, W, oR, oW, oU, ctrl, s);
+}
+
+// 3D: 8 x 8 x 4 cells, 256 of them with exactly 256 halo cells: two tuples per
+// thread, 45 KB of LDS (three blocks per CU).  16 x 8 x 4, 8 x 8 x 8 and 16 x
+// 16 x 4 build fewer halo tuples (1.9, 1.75, 1.6 per cell) but put fewer
+// blocks on the chip: 32^3 27 / 28 / 36 against 23 us per step, 100 x 90 x 84
+// 159 / 112 / 140 against 108.
+// 2D: 16 x 16 cells (1.25 tuples per cell) once that gives every CU a block,
+// 8 x 8 below: 500 x 400 30.8 against 33.8 us per step, 64^2 20.2 against 19.1.
+hipError_t launch_stage_brick(const GridDev &g, int stage, int mode, const double *U, const double *R, const double *W,
+                              double *oR, double *oW, double *oU, Ctrl *ctrl, hipStream_t s) {
+  if (g.dim == 3) return launch_brick_s<3, 8, 8, 4>(g, stage, mode, U, R, W, oR, oW, oU, ctrl, s);
+  if (g.N >= (1 << 16)) return launch_brick_s<2, 16, 16, 1>(g, stage, mode, U, R, W, oR, oW, oU, ctrl, s);
+  return launch_brick_s<2, 8, 8, 1>(g, stage, mode, U, R, W, oR, oW, oU, ctrl, s);
+}
+
+}  // namespace mmf

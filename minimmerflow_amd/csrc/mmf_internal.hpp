@@ -59,7 +59,8 @@ __host__ __device__ inline int march_tile_of_block(int b, int nblk) {
 }
 
 // Stage-kernel variants.
-enum KernelKind { KERNEL_AUTO = 0, KERNEL_GATHER = 1, KERNEL_MARCH = 2, KERNEL_TILE = 3 };
+// KERNEL_BRICK is AUTO's choice only; at the C-ABI it reports as GATHER.
+enum KernelKind { KERNEL_AUTO = 0, KERNEL_GATHER = 1, KERNEL_MARCH = 2, KERNEL_TILE = 3, KERNEL_BRICK = 4 };
 
 // Launch shape of the marching kernel (tile rows and march chunk).
 struct MarchShape {
@@ -142,6 +143,13 @@ inline OutputLayout output_layout(int64_t N) {
 // (MMF_OK or the status mmf_create would return); no flags, field stride =
 // cells rounded up to 64.
 int grid_from_desc(const mmf_grid_desc *d, GridDev &g);
+
+// Order-1 brick kernel (mmf_brick.hip): without per-face conditions, every
+// fluid cell solved, 32-bit cell indices.
+constexpr int64_t BRICK_MAX_CELLS = (int64_t)1 << 28;
+bool brick_supported(const GridDev &g);
+hipError_t launch_stage_brick(const GridDev &g, int stage, int mode, const double *U, const double *R, const double *W,
+                              double *oR, double *oW, double *oU, Ctrl *ctrl, hipStream_t s);
 
 // Kernel launchers (mmf_kernels.hip).  All enqueue on 'stream'.
 hipError_t launch_stage(const GridDev &g, int stage, int mode, const double *U, const double *R, const double *W,

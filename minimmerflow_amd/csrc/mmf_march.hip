@@ -186,25 +186,6 @@ __device__ __forceinline__ double virtual_face(const GridDev &g, const double *b
   return lam;
 }
 
-// The largest of a cell's per-axis eigenvalues |u_a| + sqrt(gamma T)
-// (euler.cpp:57-66 for n = +-e_a) with four divisions instead of the tuple's
-// seven, the same double: a correctly rounded division is odd in its
-// divisor and non-decreasing in its dividend, so max_a |fl(m_a / rho)| =
-// fl(max_a |m_a| / |rho|), and fl(x + a) is non-decreasing in x; T is
-// cons2prim's (utils.cpp:48-63) to the bit.  A NaN momentum wins the u64
-// maximum and stays NaN.
-template <int DIM>
-__device__ __forceinline__ double cell_max_eig(const double *c) {
-  double m = fabs(c[FID_RHO_U]);
-#pragma unroll
-  for (int a = 1; a < DIM; ++a) m = lam_acc(m, fabs(c[FID_RHO_U + a]));
-  const double umax = m / fabs(c[FID_RHO]);
-  const double K = (c[FID_RHO_U] * c[FID_RHO_U] + c[FID_RHO_V] * c[FID_RHO_V] + c[FID_RHO_W] * c[FID_RHO_W]) /
-                   (c[FID_RHO] * c[FID_RHO]);
-  const double T = (2.0 * c[FID_RHO_E] / c[FID_RHO] - K) / (2.0 / (GAMMA - 1.0));
-  return umax + sqrt(GAMMA * T);
-}
-
 }  // namespace
 
 // One block's march over tile 'tile' (x, y tile and chunk).  MASK: the cell

@@ -13,6 +13,13 @@ namespace mmf {
 // division sequence.
 __device__ __forceinline__ double div_vol(const GridDev &g, double x) { return g.pow2V ? x * g.invV : x / g.V; }
 
+// Tile of block b of n: consecutive blocks go to the 8 XCDs in turn; each XCD
+// takes a contiguous range of tiles (any n), whose halos meet in its L2.
+__device__ __forceinline__ int xcd_range(int b, int n) {
+  const int q = n / 8, r = n % 8, x = b % 8;
+  return x * q + (x < r ? x : r) + b / 8;
+}
+
 // Linear index of this block in its grid.
 __device__ __forceinline__ unsigned int block_linear() {
   return blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
@@ -191,6 +198,25 @@ __device__ __forceinline__ void block_lam_to(Ctrl *ctrl, double v, int tid) {
     for (int w = 1; w < (NT + 63) / 64; ++w) m = (red[w] > m) ? red[w] : m;
     lam_put(ctrl, m);
   }
+}
+
+// The largest of a cell's per-axis eigenvalues |u_a| + sqrt(gamma T)
+// (euler.cpp:57-66 for n = +-e_a) with four divisions instead of the tuple's
+// seven, the same double: a correctly rounded division is odd in its
+// divisor and non-decreasing in its dividend, so max_a |fl(m_a / rho)| =
+// fl(max_a |m_a| / |rho|), and fl(x + a) is non-decreasing in x; T is
+// cons2prim's (utils.cpp:48-63) to the bit.  A NaN momentum wins the u64
+// maximum and stays NaN.
+template <int DIM>
+__device__ __forceinline__ double cell_max_eig(const double *c) {
+  double m = fabs(c[FID_RHO_U]);
+#pragma unroll
+  for (int a = 1; a < DIM; ++a) m = lam_acc(m, fabs(c[FID_RHO_U + a]));
+  const double umax = m / fabs(c[FID_RHO]);
+  const double K = (c[FID_RHO_U] * c[FID_RHO_U] + c[FID_RHO_V] * c[FID_RHO_V] + c[FID_RHO_W] * c[FID_RHO_W]) /
+                   (c[FID_RHO] * c[FID_RHO]);
+  const double T = (2.0 * c[FID_RHO_E] / c[FID_RHO] - K) / (2.0 / (GAMMA - 1.0));
+  return umax + sqrt(GAMMA * T);
 }
 
 // Neighbour of cell q along axis a (dir +-1); false outside a non-periodic border.
