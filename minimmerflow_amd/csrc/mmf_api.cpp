@@ -220,6 +220,7 @@ int grid_from_desc(const mmf_grid_desc *d, GridDev &g) {
   int e2 = 0;
   g.pow2V = std::frexp(g.V, &e2) == 0.5 ? 1 : 0;
   g.invV = 1.0 / g.V;
+  g.quotV = g.V > 0x1p-100 && g.V < 0x1p100 ? 1 : 0;
   g.pow2A = std::frexp(g.A, &e2) == 0.5 ? 1 : 0;
   g.halfA = 0.5 * g.A;
   return MMF_OK;

@@ -165,7 +165,7 @@ __global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X
   const bool solved = valid && (!MASK || (fc & CELL_SOLVED));
   double lam = 0.0;  // stage maximum: the larger side of every face (euler.cpp:232-234)
   Tup Tc;
-  make_tup(Xc, Tc);
+  make_tup_fast(Xc, Tc);
   put_tup<NS>(lds, tid, Tc);
   bool neg_here = valid && tup_negative(Tc);
   if (solved) {
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X
       for (int k = 0; k < NF; ++k) Xh[k] = v[k];
     }
     Tup Th;
-    make_tup(Xh, Th);
+    make_tup_fast(Xh, Th);
     put_tup<NS>(lds, XM + tid, Th);
     neg_here = neg_here || tup_negative(Th);
     if (MASK) lfl[XM + tid] = fh;
@@ -268,18 +268,29 @@ __global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X
     }
 
     double nu[NF];
+    if (P2) {
 #pragma unroll
-    for (int k = 0; k < NF; ++k) {
-      const double r = P2 ? g.halfA * rhs[k] : rhs[k];
-      GridDev gp = g;
-      gp.pow2V = P2;
-      nu[k] = (STAGE == 1) ? (step ? Tc.c[k] + div_vol(gp, dt * r) : r) : rk_update<STAGE>(gp, Uc[k], Tc.c[k], r, dt);
-      if (run) out[k * fs + idx] = nu[k];
+      for (int k = 0; k < NF; ++k) rhs[k] = g.halfA * rhs[k];
+    }
+    if (STAGE == 1 && !step) {
+#pragma unroll
+      for (int k = 0; k < NF; ++k) nu[k] = rhs[k];
+    } else {
+      double x[NF], q[NF];
+#pragma unroll
+      for (int k = 0; k < NF; ++k) x[k] = dt * rhs[k];
+      div_vol5<P2>(g, x, q);
+#pragma unroll
+      for (int k = 0; k < NF; ++k) nu[k] = rk_update_q<STAGE>(Uc[k], Tc.c[k], q[k]);
+    }
+    if (run) {
+#pragma unroll
+      for (int k = 0; k < NF; ++k) out[k * fs + idx] = nu[k];
     }
     if (STAGE == 3) {
       // the next step's stage-1 maximum: this cell's, and the virtual states
       // its border and wall faces will have
-      lam_nx = cell_max_eig<DIM>(nu);
+      lam_nx = cell_max_eig_fast<DIM>(nu);
 #pragma unroll
       for (int a = 0; a < DIM; ++a) {
         bool refl = false;

@@ -138,6 +138,100 @@ __device__ __forceinline__ void make_tup(const double *c, Tup &t) {
   make_tup_prim(c, prim, t);
 }
 
+// ---------------------------------------------------------------------------
+// Correctly rounded quotients that share a reciprocal.
+//
+// A correctly rounded FP64 division is 11 instructions here (scale both
+// operands, hardware reciprocal, two Newton steps, product, remainder, fused
+// correction, fix-up).  The reciprocal and its Newton steps depend on the
+// divisor alone, and scaling and fix-up only act near the ends of the exponent
+// range, so inside it a further quotient by the same divisor is three
+// instructions, the same operations on the same operands: the same double
+// (compared with a / b, K / b^2, sqrt and the two constants on 10^9 operands
+// each, mantissas at both ends of their range among them).  The stage kernels
+// issue FP64 instructions three quarters of the time, and a flux tuple's seven
+// divisions were two thirds of it (145 issue slots, 85 this way).
+// ---------------------------------------------------------------------------
+
+// The reciprocal that quot() takes for divisor b.
+__device__ __forceinline__ double quot_rcp(double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+  return __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+}
+
+// a / b from y = quot_rcp(b) (or the rounded 1 / b).
+__device__ __forceinline__ double quot(double a, double b, double y) {
+  const double q = a * y;
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+
+// Operands whose exponent is at least this keep every remainder exact (a
+// zero's counts as 0; infinities and NaN are found in the result).
+constexpr int QUOT_MIN_EXP = -900;
+
+__device__ __forceinline__ int min_exp(double a, double b) {
+  const int x = __builtin_amdgcn_frexp_exp(a), y = __builtin_amdgcn_frexp_exp(b);
+  return x < y ? x : y;
+}
+
+__device__ __forceinline__ bool quot_divisor(double b) {
+  return (unsigned)(__builtin_amdgcn_frexp_exp(b) + 100) <= 200u;
+}
+
+__device__ __forceinline__ bool finite_bits(double x) {
+  return !__builtin_amdgcn_class(x, 0x207);  // neither NaN nor an infinity (3 = both NaN kinds, 4, 0x200)
+}
+
+// sqrt(x) for 2^-700 < x < inf: the library's steps without its range scaling.
+__device__ __forceinline__ double sqrt_normal(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double s = x * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, s, 0.5);
+  h = __builtin_fma(h, r, h);
+  s = __builtin_fma(s, r, s);
+  s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
+  return __builtin_fma(__builtin_fma(-s, s, x), h, s);
+}
+
+// T of cons2prim and sqrt(gamma T), y = quot_rcp(rho); false where an operand
+// is outside the ranges above (K, 2 E and T; the divisor and the result are
+// the caller's).
+__device__ __forceinline__ bool temperature_quot(const double *c, double y, double &T, double &a) {
+  constexpr double c5 = 2.0 / (GAMMA - 1.0);
+  const double K = c[FID_RHO_U] * c[FID_RHO_U] + c[FID_RHO_V] * c[FID_RHO_V] + c[FID_RHO_W] * c[FID_RHO_W];
+  const double r2 = c[FID_RHO] * c[FID_RHO];
+  double y2 = y * y;
+  y2 = __builtin_fma(y2, __builtin_fma(-r2, y2, 1.0), y2);
+  T = quot(quot(2.0 * c[FID_RHO_E], c[FID_RHO], y) - quot(K, r2, y2), c5, 1.0 / c5);
+  a = sqrt_normal(GAMMA * T);
+  return (min_exp(K, c[FID_RHO_E]) >= QUOT_MIN_EXP) & (T > 0x1p-700);
+}
+
+// make_tup with shared reciprocals; false: c is outside their range and t is
+// not the tuple.
+__device__ __forceinline__ bool make_tup_quot(const double *c, Tup &t) {
+  const double rho = c[FID_RHO];
+  const double y = quot_rcp(rho);
+  double T;
+  bool ok = temperature_quot(c, y, T, t.a);
+#pragma unroll
+  for (int k = 0; k < NF; ++k) t.c[k] = c[k];
+#pragma unroll
+  for (int b = 0; b < 3; ++b) t.vel[b] = quot(c[FID_RHO_U + b], rho, y);
+  t.p = rho * T;
+  const double vel2 = t.vel[0] * t.vel[0] + t.vel[1] * t.vel[1] + t.vel[2] * t.vel[2];
+  const double eto = quot(t.p, GAMMA - 1., 1.0 / (GAMMA - 1.)) + 0.5 * rho * vel2;
+  t.H = eto + t.p;
+  const int e = min_exp(c[FID_RHO_U], c[FID_RHO_V]), ew = __builtin_amdgcn_frexp_exp(c[FID_RHO_W]);
+  return ok & ((e < ew ? e : ew) >= QUOT_MIN_EXP) & quot_divisor(rho) & finite_bits(t.H);
+}
+
+// make_tup, the division sequences only where the quotients do not apply.
+__device__ __forceinline__ void make_tup_fast(const double *c, Tup &t) {
+  if (__builtin_expect(!make_tup_quot(c, t), 0)) make_tup(c, t);
+}
+
 // Mirror of the velocity component along axis a (euler.cpp:318-337 with
 // n = +-e_a: u - 2 (u.n) n), reflecting and wall BC (euler.cpp:347-356).
 __device__ __forceinline__ void reflect_axis(const double *cons, int a, double *out) {

@@ -26,6 +26,7 @@ struct GridDev {
   int32_t ghost_free;    // with flags: every fluid cell is solved (no ghost cells)
   double invV;         // 1/V, used only when V is a power of two (x/V == x*invV exactly)
   int32_t pow2V;
+  int32_t quotV;       // invV and V are inside the range of quot() (mmf_device.hpp)
   int32_t pow2A;       // A is a power of two: A*(0.5*x) == (0.5*A)*x exactly
   double halfA;        // 0.5*A
   // 3D marching kernel on a grid with flags: per block, its tile, with

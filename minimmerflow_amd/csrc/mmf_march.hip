@@ -350,6 +350,22 @@ __device__ __forceinline__ void march_block(const GridDev &g, StageIn<STAGE> in,
     return l;
   };
 
+  // a cell's stage update: stage 1 writes the residual itself unless it is a
+  // step's with early dt
+  auto update = [&](const double *c, const double *u, const double *rhs, double *nu) {
+    if (STAGE == 1 && !w1) {
+#pragma unroll
+      for (int k = 0; k < NF; ++k) nu[k] = rhs[k];
+    } else {
+      double x[NF], q[NF];
+#pragma unroll
+      for (int k = 0; k < NF; ++k) x[k] = dt * rhs[k];
+      div_vol5<P2>(g, x, q);
+#pragma unroll
+      for (int k = 0; k < NF; ++k) nu[k] = rk_update_q<STAGE>(u[k], c[k], q[k]);
+    }
+  };
+
   Tup Tc;  // tuple of this column's cell in plane m
   uint8_t fc = CELL_FLUID | CELL_SOLVED;
   uint8_t fb = CELL_FLUID | CELL_SOLVED;  // the cell below plane m (MASK)
@@ -381,7 +397,7 @@ __device__ __forceinline__ void march_block(const GridDev &g, StageIn<STAGE> in,
       double Xh[NF];
       Tup Th;
       src.load(gp, dt, hcol + (uint32_t)m0 * sm, Xh);
-      make_tup(Xh, Th);
+      make_tup_fast(Xh, Th);
       tup_store<PS>(lds, hslot, Th);
       if (MASK) lfl[hslot] = g.flags[hcol + (uint32_t)m0 * sm];
     }
@@ -472,7 +488,7 @@ __device__ __forceinline__ void march_block(const GridDev &g, StageIn<STAGE> in,
         {
           double X[NF];
           pf.state(gp, dt, X);
-          make_tup(X, Tn);
+          make_tup_fast(X, Tn);
           tup_store<PS>(Ln, myslot, Tn);
           const uint32_t p2 = (m + 2 < m1) ? (uint32_t)(m + 2) : (have_beyond ? beyond : (uint32_t)(m + 1));
           pf.issue(src, col + p2 * sm);
@@ -501,15 +517,16 @@ __device__ __forceinline__ void march_block(const GridDev &g, StageIn<STAGE> in,
           neg.add(Tc, Tn);
           lam_max = lam_acc(lam_max, l);
         }
-        double nu[NF];
+        double nu[NF], rhs[NF];
 #pragma unroll
         for (int k = 0; k < NF; ++k) {
-          double rhs = (acc[k] + AFlo[k]) - AFhi[k];
-          if (P2) rhs = rhs_scale * rhs;
-          nu[k] = w1 ? Tc.c[k] + div_vol(gp, dt * rhs) : rk_update<STAGE>(gp, Ucur[k], Tc.c[k], rhs, dt);
-          outf.put(k, idx, nu[k]);
+          rhs[k] = (acc[k] + AFlo[k]) - AFhi[k];
+          if (P2) rhs[k] = rhs_scale * rhs[k];
         }
-        if (EARLY && STAGE == 3) lam_nx = lam_acc(lam_nx, cell_max_eig<DIM>(nu));
+        update(Tc.c, Ucur, rhs, nu);
+#pragma unroll
+        for (int k = 0; k < NF; ++k) outf.put(k, idx, nu[k]);
+        if (EARLY && STAGE == 3) lam_nx = lam_acc(lam_nx, cell_max_eig_fast<DIM>(nu));
 #pragma unroll
         for (int k = 0; k < NF; ++k) AFlo[k] = AFhi[k];
         Tc = Tn;
@@ -521,7 +538,7 @@ __device__ __forceinline__ void march_block(const GridDev &g, StageIn<STAGE> in,
           double Xh[NF];
           Tup Th;
           ph.state(gp, dt, Xh);
-          make_tup(Xh, Th);
+          make_tup_fast(Xh, Th);
           tup_store<PS>(Ln, hslot, Th);
           if (m + 2 < m1) ph.issue(src, hcol + (uint32_t)(m + 2) * sm);
         }
@@ -558,7 +575,7 @@ __device__ __forceinline__ void march_block(const GridDev &g, StageIn<STAGE> in,
 #pragma unroll
         for (int k = 0; k < NF; ++k) Unext[k] = pf.a[k];
       }
-      make_tup(X, Tn);
+      make_tup_fast(X, Tn);
       bad_n = tup_negative(Tn);
       fn = ff;
       if (in_chunk) {
@@ -570,7 +587,7 @@ __device__ __forceinline__ void march_block(const GridDev &g, StageIn<STAGE> in,
       double Xh[NF];
       Tup Th;
       ph.state(gp, dt, Xh);
-      make_tup(Xh, Th);
+      make_tup_fast(Xh, Th);
       tup_store<PS>(Ln, hslot, Th);
       if (MASK) LFn[hslot] = fh;
     }
@@ -662,16 +679,17 @@ __device__ __forceinline__ void march_block(const GridDev &g, StageIn<STAGE> in,
         // the periodic top cell: its upper face (the wrap face) precedes its
         // lower face in the reference's face list
         const bool wrap_top = top_wrap_here && m == nm - 1;
-        double nu[NF];
+        double nu[NF], rhs[NF];
 #pragma unroll
         for (int k = 0; k < NF; ++k) {
-          double rhs = wrap_top ? (acc[k] - AFhi[k]) + AFlo[k] : (acc[k] + AFlo[k]) - AFhi[k];
-          if (P2) rhs = rhs_scale * rhs;
-          nu[k] = w1 ? Tc.c[k] + div_vol(gp, dt * rhs) : rk_update<STAGE>(gp, Ucur[k], Tc.c[k], rhs, dt);
-          outf.put(k, idx, nu[k]);
+          rhs[k] = wrap_top ? (acc[k] - AFhi[k]) + AFlo[k] : (acc[k] + AFlo[k]) - AFhi[k];
+          if (P2) rhs[k] = rhs_scale * rhs[k];
         }
+        update(Tc.c, Ucur, rhs, nu);
+#pragma unroll
+        for (int k = 0; k < NF; ++k) outf.put(k, idx, nu[k]);
         if (EARLY && STAGE == 3) {
-          lam_nx = lam_acc(lam_nx, cell_max_eig<DIM>(nu));
+          lam_nx = lam_acc(lam_nx, cell_max_eig_fast<DIM>(nu));
           if (MASK || REFL) lam_nx = lam_acc(lam_nx, virtual_max_eig(gp, nu, LF, m, fb, fn, has_next));
         }
       } else if (STAGE != 3) {

@@ -79,11 +79,38 @@ struct Pf2 {
       }
     }
   }
+  template <bool P2>
   __device__ __forceinline__ void state(const GridDev &g, double dt, double *X) const {
+    if (STAGE == 2) {
+      double x[NF], q[NF];
 #pragma unroll
-    for (int k = 0; k < NF; ++k) X[k] = (STAGE == 2) ? a[k] + div_vol(g, dt * b[k]) : a[k];
+      for (int k = 0; k < NF; ++k) x[k] = dt * b[k];
+      div_vol5<P2>(g, x, q);
+#pragma unroll
+      for (int k = 0; k < NF; ++k) X[k] = a[k] + q[k];
+    } else {
+#pragma unroll
+      for (int k = 0; k < NF; ++k) X[k] = a[k];
+    }
   }
 };
+
+// A cell's stage update (stage 1 writes the residual).
+template <int STAGE, bool P2>
+__device__ __forceinline__ void row_update(const GridDev &g, double dt, const double *u, const double *c,
+                                           const double *rhs, double *nu) {
+  if (STAGE == 1) {
+#pragma unroll
+    for (int k = 0; k < NF; ++k) nu[k] = rhs[k];
+    return;
+  }
+  double x[NF], q[NF];
+#pragma unroll
+  for (int k = 0; k < NF; ++k) x[k] = dt * rhs[k];
+  div_vol5<P2>(g, x, q);
+#pragma unroll
+  for (int k = 0; k < NF; ++k) nu[k] = rk_update_q<STAGE>(u[k], c[k], q[k]);
+}
 
 __device__ __forceinline__ double vface(const GridDev &g, bool wall, int side, int a, const Tup &Fl, bool fluid_lower,
                                         double *AF, NegCount &neg, bool count) {
@@ -162,12 +189,12 @@ __device__ double march2d_item(const GridDev &g0, const In2<STAGE, P2> &in, cons
       Pf2<STAGE> p0;
       double X[NF];
       p0.issue(in, idx0);
-      p0.state(g, dt, X);
+      p0.template state<P2>(g, dt, X);
       if (STAGE == 2) {
 #pragma unroll
         for (int k = 0; k < NF; ++k) Ucur[k] = p0.a[k];
       }
-      make_tup(X, Tc);
+      make_tup_fast(X, Tc);
       bad_c = tup_negative(Tc);
       fc = cell_flags<MASK>(g, idx0);
       tstore(ldsb, lane, Tc);
@@ -190,7 +217,7 @@ __device__ double march2d_item(const GridDev &g0, const In2<STAGE, P2> &in, cons
         Tup Tp;
         const uint32_t pidx = col + (uint32_t)mprev * sm;
         in.state(g, dt, pidx, Xp);
-        make_tup(Xp, Tp);
+        make_tup_fast(Xp, Tp);
         const uint8_t fp = cell_flags<MASK>(g, pidx);
         // counted here: the item below does not count its chunk's top face
         if ((fp | fc) & CELL_SOLVED) {
@@ -241,12 +268,12 @@ __device__ double march2d_item(const GridDev &g0, const In2<STAGE, P2> &in, cons
     const bool build = (valid && has_next) || (halo && in_chunk);
     if (build) {
       double X[NF];
-      pf.state(g, dt, X);
+      pf.template state<P2>(g, dt, X);
       if (STAGE == 2) {
 #pragma unroll
         for (int k = 0; k < NF; ++k) Unext[k] = pf.a[k];
       }
-      make_tup(X, Tn);
+      make_tup_fast(X, Tn);
       bad_n = tup_negative(Tn);
       fn = ff;
       if (in_chunk) {
@@ -365,12 +392,15 @@ __device__ double march2d_item(const GridDev &g0, const In2<STAGE, P2> &in, cons
       if (fc & CELL_SOLVED) {
         // the periodic top cell: its upper face (the wrap face) comes first
         const bool wrap_top = top_wrap_here && m == nm - 1;
+        double rhs[NF], nu[NF];
 #pragma unroll
         for (int k = 0; k < NF; ++k) {
-          double rhs = wrap_top ? (acc[k] - AFhi[k]) + AFlo[k] : (acc[k] + AFlo[k]) - AFhi[k];
-          if (P2) rhs = rhs_scale * rhs;
-          outb[k * fs + idx] = rk_update<STAGE>(g, Ucur[k], Tc.c[k], rhs, dt);
+          rhs[k] = wrap_top ? (acc[k] - AFhi[k]) + AFlo[k] : (acc[k] + AFlo[k]) - AFhi[k];
+          if (P2) rhs[k] = rhs_scale * rhs[k];
         }
+        row_update<STAGE, P2>(g, dt, Ucur, Tc.c, rhs, nu);
+#pragma unroll
+        for (int k = 0; k < NF; ++k) outb[k * fs + idx] = nu[k];
       } else if (STAGE != 3) {
 #pragma unroll
         for (int k = 0; k < NF; ++k) outb[k * fs + idx] = (STAGE == 1) ? 0.0 : Ucur[k];
@@ -452,12 +482,12 @@ __device__ double march2d_item_flat(const GridDev &g0, const In2<STAGE, P2> &in,
     Pf2<STAGE> p0;
     double X[NF];
     p0.issue(in, idx0);
-    p0.state(g, dt, X);
+    p0.template state<P2>(g, dt, X);
     if (STAGE == 2) {
 #pragma unroll
       for (int k = 0; k < NF; ++k) Ucur[k] = p0.a[k];
     }
-    make_tup(X, Tc);
+    make_tup_fast(X, Tc);
     bad_c = tup_negative(Tc);
     tstore(ldsb, lane, Tc);
     if (valid) {
@@ -474,7 +504,7 @@ __device__ double march2d_item_flat(const GridDev &g0, const In2<STAGE, P2> &in,
         double Xp[NF];
         Tup Tp;
         in.state(g, dt, col + (uint32_t)mprev * sm, Xp);
-        make_tup(Xp, Tp);
+        make_tup_fast(Xp, Tp);
         // counted here: the item below does not count its chunk's top face
         l = face_flux_area(Tp, Tc, 1, P2, A, halfA, AFlo);
         if (tup_negative(Tp) | bad_c) neg.add(Tp, Tc);
@@ -507,12 +537,12 @@ __device__ double march2d_item_flat(const GridDev &g0, const In2<STAGE, P2> &in,
     double Unext[NF];
     if (has_next) {
       double X[NF];
-      pf.state(g, dt, X);
+      pf.template state<P2>(g, dt, X);
       if (STAGE == 2) {
 #pragma unroll
         for (int k = 0; k < NF; ++k) Unext[k] = pf.a[k];
       }
-      make_tup(X, Tn);
+      make_tup_fast(X, Tn);
       bad_n = tup_negative(Tn);
       if (in_chunk) tstore(Ln, lane, Tn);
     }
@@ -564,16 +594,16 @@ __device__ double march2d_item_flat(const GridDev &g0, const In2<STAGE, P2> &in,
 
     // ---- this cell is complete: its RK stage update ----
     const bool wrap_top = top_wrap_here && m == nm - 1;
-    double nu[NF];
+    double nu[NF], rhs[NF];
 #pragma unroll
     for (int k = 0; k < NF; ++k) {
       double acc = 0.0;  // first two contributions from zero: their order does not change the bits
       acc += AFx[k];
       acc -= AFup[k];
-      double rhs = wrap_top ? (acc - AFhi[k]) + AFlo[k] : (acc + AFlo[k]) - AFhi[k];
-      if (P2) rhs = rhs_scale * rhs;
-      nu[k] = rk_update<STAGE>(g, Ucur[k], Tc.c[k], rhs, dt);
+      rhs[k] = wrap_top ? (acc - AFhi[k]) + AFlo[k] : (acc + AFlo[k]) - AFhi[k];
+      if (P2) rhs[k] = rhs_scale * rhs[k];
     }
+    row_update<STAGE, P2>(g, dt, Ucur, Tc.c, rhs, nu);
     if (valid) {
 #pragma unroll
       for (int k = 0; k < NF; ++k) outb[k * fs + idx] = nu[k];
@@ -934,7 +964,7 @@ __global__ __launch_bounds__(W2O) void k_march2d_o2(GridDev g, const double *X, 
     ea = eb;
     eb = ec;
     ec = epf;
-    if (epf) pf.state(gg, dt, Xc);
+    if (epf) pf.template state<P2>(gg, dt, Xc);
     {
       bool e;
       const int r = row_of(c + 3, e);

@@ -13,6 +13,30 @@ namespace mmf {
 // division sequence.
 __device__ __forceinline__ double div_vol(const GridDev &g, double x) { return g.pow2V ? x * g.invV : x / g.V; }
 
+// The five x_k / V of a cell's update.  Where V is not a power of two they
+// share its reciprocal (quot(): five instead of fourteen issue slots each), the
+// division sequences only where an operand is outside its range.
+template <bool P2>
+__device__ __forceinline__ void div_vol5(const GridDev &g, const double *x, double *q) {
+  if (P2) {
+#pragma unroll
+    for (int k = 0; k < NF; ++k) q[k] = x[k] * g.invV;
+    return;
+  }
+  int e = __builtin_amdgcn_frexp_exp(x[0]);
+#pragma unroll
+  for (int k = 1; k < NF; ++k) {
+    const int ek = __builtin_amdgcn_frexp_exp(x[k]);
+    e = (ek < e) ? ek : e;
+  }
+#pragma unroll
+  for (int k = 0; k < NF; ++k) q[k] = __builtin_amdgcn_div_fixup(quot(x[k], g.V, g.invV), g.V, x[k]);
+  if (__builtin_expect(e < QUOT_MIN_EXP || !g.quotV, 0)) {
+#pragma unroll
+    for (int k = 0; k < NF; ++k) q[k] = x[k] / g.V;
+  }
+}
+
 // Tile of block b of n: consecutive blocks go to the 8 XCDs in turn; each XCD
 // takes a contiguous range of tiles (any n), whose halos meet in its L2.
 __device__ __forceinline__ int xcd_range(int b, int n) {
@@ -219,6 +243,21 @@ __device__ __forceinline__ double cell_max_eig(const double *c) {
   return umax + sqrt(GAMMA * T);
 }
 
+// cell_max_eig with the shared reciprocal of rho.
+template <int DIM>
+__device__ __forceinline__ double cell_max_eig_fast(const double *c) {
+  double m = fabs(c[FID_RHO_U]);
+#pragma unroll
+  for (int a = 1; a < DIM; ++a) m = lam_acc(m, fabs(c[FID_RHO_U + a]));
+  const double rho = fabs(c[FID_RHO]), y = quot_rcp(c[FID_RHO]);
+  double T, s;
+  const bool ok = temperature_quot(c, y, T, s);
+  const double l = quot(m, rho, fabs(y)) + s;
+  if (__builtin_expect(!(ok & (__builtin_amdgcn_frexp_exp(m) >= QUOT_MIN_EXP) & quot_divisor(rho) & finite_bits(l)), 0))
+    return cell_max_eig<DIM>(c);
+  return l;
+}
+
 // Neighbour of cell q along axis a (dir +-1); false outside a non-periodic border.
 __device__ __forceinline__ bool neighbour(const GridDev &g, const int64_t *q, int a, int dir, int64_t &nb) {
   int64_t v = q[a] + dir;
@@ -318,6 +357,14 @@ __device__ __forceinline__ double rk_update(const GridDev &g, double u, double x
   if (STAGE == 1) return rhs;
   if (STAGE == 2) return 0.75 * u + 0.25 * (x + div_vol(g, dt * rhs));
   return (1. / 3) * u + (2. / 3) * (x + div_vol(g, dt * rhs));
+}
+
+// The same from q = dt rhs / V (stage 1: W1 = U + q).
+template <int STAGE>
+__device__ __forceinline__ double rk_update_q(double u, double x, double q) {
+  if (STAGE == 1) return x + q;
+  if (STAGE == 2) return 0.75 * u + 0.25 * (x + q);
+  return (1. / 3) * u + (2. / 3) * (x + q);
 }
 
 }  // namespace mmf
