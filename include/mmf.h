@@ -85,12 +85,14 @@ int mmf_get_sizes(const mmf_ctx *ctx, int64_t *ncells, int64_t *ninterfaces);
 /* ---- stage-kernel selection ------------------------------------------------ */
 enum { MMF_KERNEL_AUTO = 0, MMF_KERNEL_GATHER = 1, MMF_KERNEL_MARCH = 2, MMF_KERNEL_TILE = 3 };
 /* GATHER: per-cell kernel, any grid.  MARCH: the marching LDS-tile kernels
- * (order 1; order 2 in 2D without bodies).  TILE: the 8x8 LDS tile kernel of
+ * (order 1; order 2 in 2D without bodies).  TILE: the 8x8 LDS tile kernels of
  * 2D order-2 grids without bodies (each face once, the step's time advance
  * in its last stage; also the learned reconstruction's kernel).  AUTO: TILE
- * for 2D order-2 grids without bodies below 2^18 cells; MARCH where it
- * applies from 2^18 cells (2D order 1) or 2^20 cells (3D order 1, 2D order
- * 2); else GATHER.  mmf_set_kernel refuses MARCH or TILE on a grid they do not
+ * for 2D order-2 grids without bodies; MARCH where it applies from 2^18 cells
+ * (2D order 1, strips that need no reflected state) or 2^20 cells (3D); else
+ * GATHER, which AUTO runs as LDS bricks (a thread per cell, every flux tuple
+ * once per brick) where they apply: 3D order 2 without bodies at any size,
+ * order 1 where every fluid cell is solved, border conditions per side.  mmf_set_kernel refuses MARCH or TILE on a grid they do not
  * apply to; bodies set afterwards make them fall back to GATHER.  tile_rows (3D: 4 or 8) and chunk (planes per block along the last axis)
  * shape the marching kernel; <= 0 keeps the default (3D order 1, 64 x 8
  * tiles: where the chunks would leave a partial round of blocks, the planes

@@ -54,9 +54,9 @@ bool valid_bc(int b) { return b >= MMF_BC_FREE_FLOW && b <= MMF_BC_PERIODIC; }
 // it a grid gives the marching kernels too few blocks or rows to march):
 // 2D order 1 from 2^18 cells (64^2 56 vs 28 us per step, 512^2 equal, 1024^2
 // 137 vs 188), 3D order 1 from 2^20 (32^3 273 vs 37 us, 96^3 319 vs 193,
-// 128^3 271 vs 379), 2D order 2 from 2^20 (below it the tile kernel, then the
-// gather kernel).  Order-1 grids without ghost cells or per-face conditions go
-// to the brick kernel below brick_auto_max.
+// 128^3 271 vs 379), 3D order 2 (with bodies) from 2^20.  Order-1 grids without
+// ghost cells or per-face conditions go to the brick kernel below
+// brick_auto_max, order-2 grids without bodies to the tile kind and the bricks.
 bool use_march(const mmf_ctx *ctx) {
   if (ctx->kernel == mmf::KERNEL_GATHER || !mmf::march_shape_supported(ctx->g, ctx->shape)) return false;
   if (ctx->kernel == mmf::KERNEL_AUTO) {
@@ -70,11 +70,19 @@ bool tile_applies(const mmf_ctx *ctx) {
   return ctx->g.dim == 2 && ctx->g.order == 2 && !ctx->g.flags && !ctx->g.bslot;
 }
 
-// AUTO takes the tile kernel for 2D order-2 grids below this size (measured on
-// MI355X, vortex: 128^2 25.7 vs 50.0 us per step for the gather kernel, 256^2
-// 48.5 vs 58.0; at 512^2 the gather and strip kernels are faster, 125-128 vs
-// 146, the tile kernel's fixed per-block latency no longer hidden).
-constexpr int64_t TILE_AUTO_MAX_N = (int64_t)1 << 18;
+// 2D order-2 grids above this size run the tile kind as 8 x 8 bricks of one wave
+// (mmf_brick_o2.hip) instead of 8 x 8 tiles of six: half the instructions per
+// cell, but a longer chain in each wave.  us per step alone / with three grids
+// in flight, six waves against one (MI355X, vortex): 64^2 25.5 / 9.8 and 27.9 /
+// 10.5, 128^2 25.7 / 11.3 and 27.7 / 11.1, 192^2 35 / 20 and 30 / 12, 256^2 48 /
+// 33 and 33 / 14; 512^2 128 (gather) and 69, 2048^2 1343 (strips) and 664.
+// 3D order 2 always takes the bricks: 32^3 66 (gather) and 37, 144^3 1357
+// (marching) and 594, 256^3 5207 and 3282.
+constexpr int64_t TILE_SIX_WAVES_MAX_N = (int64_t)1 << 14;
+
+bool o2_bricks(const GridDev &g) {
+  return mmf::brick_o2_supported(g) && (g.dim == 3 || g.N > TILE_SIX_WAVES_MAX_N);
+}
 
 // AUTO takes the brick kernel for order-1 grids below this size (us per step,
 // gather / best marching shape / brick; MI355X).  3D: 32^3 37 / 36 / 23, 64^3
@@ -96,7 +104,8 @@ int64_t brick_auto_max(const GridDev &g) {
 int kernel_used(const mmf_ctx *ctx) {
   if (ctx->learn_on) return ctx->kernel == mmf::KERNEL_GATHER ? mmf::KERNEL_GATHER : mmf::KERNEL_TILE;
   if (ctx->kernel == mmf::KERNEL_TILE) return tile_applies(ctx) ? mmf::KERNEL_TILE : mmf::KERNEL_GATHER;
-  if (ctx->kernel == mmf::KERNEL_AUTO && tile_applies(ctx) && ctx->g.N < TILE_AUTO_MAX_N) return mmf::KERNEL_TILE;
+  if (ctx->kernel == mmf::KERNEL_AUTO && tile_applies(ctx)) return mmf::KERNEL_TILE;
+  if (ctx->kernel == mmf::KERNEL_AUTO && ctx->g.dim == 3 && mmf::brick_o2_supported(ctx->g)) return mmf::KERNEL_BRICK;
   if (ctx->kernel == mmf::KERNEL_AUTO && ctx->g.N < brick_auto_max(ctx->g) && mmf::brick_supported(ctx->g))
     return mmf::KERNEL_BRICK;
   return use_march(ctx) ? mmf::KERNEL_MARCH : mmf::KERNEL_GATHER;
@@ -118,6 +127,8 @@ int launch_stage_on(mmf_ctx *ctx, int stage, int mode, double *U, double *R, dou
     e = mmf::launch_recon_learned(ctx->g, ctx->learn, stage, mode, U, R, W, ctx->dctrl, ctx->stream);
     if (e == hipSuccess)
       e = mmf::launch_flux_fs(ctx->g, ctx->learn, stage, mode, U, R, W, R, W, U, ctx->dctrl, ctx->stream);
+  } else if (!ctx->learn_on && (kind == mmf::KERNEL_TILE || kind == mmf::KERNEL_BRICK) && o2_bricks(ctx->g)) {
+    e = mmf::launch_stage_brick_o2(ctx->g, stage, mode, U, R, W, R, W, U, ctx->dctrl, ctx->stream);
   } else if (kind == mmf::KERNEL_TILE) {
     // one launch per stage, face states in LDS; plain face values without a network
     mmf::LearnRun plain{};
@@ -900,7 +911,8 @@ int ensure_tiles(mmf_ctx *ctx) {
 
 int ensure_lam(mmf_ctx *ctx) {
   const int used = kernel_used(ctx);
-  const bool early = (used == mmf::KERNEL_MARCH && mmf::march_early(ctx->g)) || used == mmf::KERNEL_BRICK;
+  const bool early = (used == mmf::KERNEL_MARCH && mmf::march_early(ctx->g)) ||
+                     (used == mmf::KERNEL_BRICK && ctx->g.order == 1);
   if (!early) {
     ctx->lam_valid = false;
     return MMF_OK;

@@ -152,6 +152,12 @@ bool brick_supported(const GridDev &g);
 hipError_t launch_stage_brick(const GridDev &g, int stage, int mode, const double *U, const double *R, const double *W,
                               double *oR, double *oW, double *oU, Ctrl *ctrl, hipStream_t s);
 
+// Order-2 brick kernel (mmf_brick_o2.hip): without bodies or per-face
+// conditions, 32-bit cell indices.
+bool brick_o2_supported(const GridDev &g);
+hipError_t launch_stage_brick_o2(const GridDev &g, int stage, int mode, const double *U, const double *R,
+                                 const double *W, double *oR, double *oW, double *oU, Ctrl *ctrl, hipStream_t s);
+
 // Kernel launchers (mmf_kernels.hip).  All enqueue on 'stream'.
 hipError_t launch_stage(const GridDev &g, int stage, int mode, const double *U, const double *R, const double *W,
                         double *out_R, double *out_W, double *out_U, Ctrl *ctrl, hipStream_t stream);

@@ -1,11 +1,12 @@
-"""The brick kernel (AUTO on small and ordinary order-1 grids) against the
-per-cell gather kernel: RHS, steps, time control, stage maxima and positivity
-counts, all bit for bit, on brick edges, remainders, one-cell grids, every
-border condition, periodic wraps and bodies."""
+"""The brick kernels (AUTO on small and ordinary order-1 grids and on order-2
+grids without a body) against the per-cell gather kernel: RHS, steps, time
+control, stage maxima and positivity counts, all bit for bit, on brick edges,
+remainders, one-cell grids, every border condition, periodic wraps and
+bodies."""
 import numpy as np
 import pytest
 
-from test_gpu_kernels import build, run_variant
+from test_gpu_kernels import build
 
 pytestmark = pytest.mark.gpu
 
@@ -32,12 +33,38 @@ CASES = [
 ]
 
 
+O2_CASES = [
+    ("3d o2 one cell", 3, (1, 1, 1), [0, 1, 2, 3, 0, 1]),
+    ("3d o2 one brick", 3, (8, 8, 4), [3, 0, 1, 2, 0, 3]),
+    ("3d o2 one past a brick", 3, (9, 9, 5), [1, 1, 0, 3, 2, 0]),
+    ("3d o2 two cells per axis, periodic", 3, (2, 2, 2), [4] * 6),
+    ("3d o2 thin, wraps inside a brick", 3, (3, 17, 2), [4, 4, 1, 0, 4, 4]),
+    ("3d o2 full bricks, periodic", 3, (16, 8, 12), [4] * 6),
+    ("3d o2 ragged", 3, (70, 13, 37), [0, 1, 2, 0, 1, 3]),
+    # 2D: one-wave bricks above 2^14 cells
+    ("2d o2 one past a brick", 2, (129, 137), [1, 2, 0, 3]),
+    ("2d o2 two columns, periodic", 2, (2, 8201), [4] * 4),
+    ("2d o2 one row", 2, (16385, 1), [0, 2, 1, 3]),
+    ("2d o2 large", 2, (530, 510), [3, 0, 4, 4]),
+]
+
+
+@pytest.mark.parametrize("name,dim,n,bc", O2_CASES, ids=[c[0] for c in O2_CASES])
+@pytest.mark.parametrize("negative", [False, True])
+def test_brick_order2_equals_gather(mmf, name, dim, n, bc, negative):
+    check(mmf, name, dim, n, bc, None, negative, 2)
+
+
 @pytest.mark.parametrize("name,dim,n,bc,body", CASES, ids=[c[0] for c in CASES])
 @pytest.mark.parametrize("negative", [False, True])
 def test_brick_equals_gather(mmf, name, dim, n, bc, body, negative):
+    check(mmf, name, dim, n, bc, body, negative, 1)
+
+
+def check(mmf, name, dim, n, bc, body, negative, order):
     info = np.zeros((6, 5))
     info[:] = [1.0, 0.3, -0.1, 0.05 if dim == 3 else 0.0, 1.0]
-    s, U = build(mmf, dim, list(n), bc, info, body, seed=len(name))
+    s, U = build(mmf, dim, list(n), bc, info, body, order=order, seed=len(name))
     if negative:  # density and energy negative: real sound speed, counted sides
         k = np.random.default_rng(3).integers(0, len(U), max(1, len(U) // 50))
         U = U.copy()
@@ -49,34 +76,36 @@ def test_brick_equals_gather(mmf, name, dim, n, bc, body, negative):
         s.reset_positivity_counters()
         s.set_kernel(kind)
         s.set_state(U)
-        first = s.compute_rhs()
-        counts = s.positivity_counters()
-        if negative:
-            s.advance(1)
-            out.append((first, counts, s.nonfinite_steps(), s.get_state()))
-        else:
-            out.append((first, counts, run_variant(mmf, s, U, kind)))
-    (Ra, ea), (Rb, eb) = out[0][0], out[1][0]
-    assert np.array_equal(Ra, Rb, equal_nan=True) and (ea == eb or (np.isnan(ea) and np.isnan(eb)))
-    assert out[0][1] == out[1][1]
-    if negative:
-        assert out[0][1][1] > 0 and out[0][2] == out[1][2]
-        assert np.array_equal(out[0][3], out[1][3], equal_nan=True)
-        return
-    a, b = out[0][2], out[1][2]
-    assert np.array_equal(a[0], b[0]) and a[1] == b[1]
-    assert np.array_equal(a[2], b[2]), "state after 3 steps"
+        rhs, eig = s.compute_rhs()
+        counts = [s.positivity_counters()]
+        s.advance(1 if negative else 3)
+        try:
+            t, dt, step, stages = s.time()
+            time = (t, dt, step, tuple(stages))
+        except mmf.MMFError:  # the flow itself left the positive states, with either kernel
+            time = s.nonfinite_steps()
+        counts.append(s.positivity_counters())
+        out.append((rhs, eig, s.get_state(), time, counts))
+    a, b = out
+    assert np.array_equal(a[0], b[0], equal_nan=True), "rhs"
+    assert a[1] == b[1] or (np.isnan(a[1]) and np.isnan(b[1])), "maximum eigenvalue"
+    assert np.array_equal(a[2], b[2], equal_nan=True), "state after the steps"
     assert a[3] == b[3], "time control and stage maxima"
-    assert a[4] == b[4], "positivity counts"
+    if negative:
+        assert a[4][0][1] > 0
+        assert a[4][0] == b[4][0], "positivity counts"
+    else:
+        assert a[4] == b[4], "positivity counts"
 
 
 def test_brick_steps_against_the_oracle(mmf, orc):
-    """64^2 and 20 x 18 x 12, reflecting and Dirichlet sides, four steps each."""
-    for dim, n, bc in ((2, [64, 64], [1, 1, 1, 1, 0, 0]), (3, [20, 18, 12], [3, 0, 1, 2, 0, 1])):
+    """64^2 and 20 x 18 x 12, reflecting and Dirichlet sides, orders 1 and 2, four steps each."""
+    for dim, n, bc, order in ((2, [64, 64], [1, 1, 1, 1, 0, 0], 1), (3, [20, 18, 12], [3, 0, 1, 2, 0, 1], 1),
+                              (2, [60, 52], [3, 1, 4, 4, 0, 0], 2), (3, [20, 18, 12], [3, 0, 1, 2, 0, 1], 2)):
         info = np.tile([1.0, 0.3, -0.1, 0.0, 1.0], (6, 1))
-        s, U = build(mmf, dim, n, bc, info, None, seed=9)
+        s, U = build(mmf, dim, n, bc, info, None, order=order, seed=9)
         h = 2.0 / max(n)
-        o = orc.Solver(orc.problem(orc.RADSOD, dim), 1, n, [-1.0, -1.0, -1.0], h, side_bc=bc, side_info=info)
+        o = orc.Solver(orc.problem(orc.RADSOD, dim), order, n, [-1.0, -1.0, -1.0], h, side_bc=bc, side_info=info)
         Uo, W, t = U.copy(), U.copy(), 0.0
         s.set_state(U)
         s.set_time(0.0, 10.0, 0.5)
