@@ -453,18 +453,12 @@ def run_learned(args, mmf):
 
 
 def mesh_bytes(fm):
-    """Algorithmic HBM bytes of one stage of the face-list kernels (axis-aligned
-    faces, a handful of areas: 12 B of geometry per face).  Face kernel: owner,
-    neighbour, kind (12 B) and A*F written (40 B) per face, the stage state read
-    once per cell (40 B).  Cell kernel: offset (4 B) and volume (8 B) per cell,
-    one 4 B incidence per face side, A*F read once per face (40 B), the RK
-    update's state traffic per cell (80 / 120 / 120 B for stages 1 / 2 / 3)."""
-    import numpy as np
-    F, N = fm.nfaces, fm.ncells
-    sides = int(2 * F - (fm.neigh < 0).sum())
-    face = 52.0 * F + 40.0 * N
-    cell = 12.0 * N + 4.0 * sides + 40.0 * F + BYTES_PER_CELL_STAGE * N
-    return face, cell
+    """Algorithmic HBM bytes of one stage of the face-list kernel (axis-aligned
+    faces, a handful of areas): offset (4 B), volume (8 B) and axes (1 B) per
+    cell, 8 B per incidence (face side), the RK stage's state traffic per cell
+    (80 / 120 / 120 B for stages 1 / 2 / 3)."""
+    sides = int(2 * fm.nfaces - (fm.neigh < 0).sum())
+    return 13.0 * fm.ncells + 8.0 * sides + BYTES_PER_CELL_STAGE * fm.ncells
 
 
 def cpu_baseline_mesh(fm, pb_o, budget_s=10.0, budget_mt=5.0):
@@ -521,7 +515,7 @@ def run_mesh(args, mmf):
     g.advance(args.steps)
     t, dt, step, _ = g.time()
     el = time.perf_counter() - t1
-    face_ms, cell_ms, stages = g.read_timing()
+    _, stage_ms, stages = g.read_timing()
     g.enable_timing(False)
     if step != args.warmup + args.steps:
         raise SystemExit("bench: only %d of %d steps were active" % (step, args.warmup + args.steps))
@@ -530,13 +524,11 @@ def run_mesh(args, mmf):
         raise SystemExit("bench: negative or non-finite states encountered (%d, %d, %d)" % npc)
     N = fm.ncells
     value = N * 3 * args.steps / el
-    fb, cb = mesh_bytes(fm)
-    fa, ca = face_ms / stages, cell_ms / stages
-    dom = "face" if fa >= ca else "cell"
-    achieved = (fb / (fa * 1e-3) if dom == "face" else cb / (ca * 1e-3)) / 1e9
+    sb, sa = mesh_bytes(fm), stage_ms / stages
+    achieved = sb / (sa * 1e-3) / 1e9
     workload = "octree_sod_3d_%d_order1" % n
-    log("timed %d steps in %.3f s: %.3f ms/step; face kernel %.4f ms (%.0f GB/s), cell kernel %.4f ms (%.0f GB/s)"
-        % (args.steps, el, el / args.steps * 1e3, fa, fb / fa / 1e6, ca, cb / ca / 1e6))
+    log("timed %d steps in %.3f s: %.3f ms/step; stage kernel %.4f ms (%.0f GB/s)"
+        % (args.steps, el, el / args.steps * 1e3, sa, achieved))
     cpu = None
     if not args.no_cpu_baseline:
         log("cpu baseline: oracle face-list loop ...")
@@ -561,8 +553,8 @@ def run_mesh(args, mmf):
                    "initial": "r<0.4: rho=1 p=1; else rho=0.125 p=0.1; u=0", "boundaries": "free flow",
                    "time": "SSP-RK3, CFL 0.5 (min cell size), fixed step count", "prewarm_steps": nprewarm,
                    "reconstruction": "order 1", "flux": "Rusanov", "t_after_timed_steps": t,
-                   "kernels_ms_per_stage": {"faces": fa, "cells": ca},
-                   "algorithmic_bytes_per_stage": {"faces": fb, "cells": cb},
+                   "kernel_ms_per_stage": sa,
+                   "algorithmic_bytes_per_stage": sb,
                    "parallelism": "single GPU"},
         "roofline": {
             "bound": "hbm",
@@ -571,10 +563,9 @@ def run_mesh(args, mmf):
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": load_traffic(workload),
-            "kernel": "k_mesh_%s (%s)" % (dom + "s", "per-interface flux, A*F per face" if dom == "face"
-                                          else "segmented sum in face order + RK update"),
-            "algorithmic_bytes_per_launch": fb if dom == "face" else cb,
-            "avg_launch_ms": fa if dom == "face" else ca,
+            "kernel": "k_mesh_stage (a cell's faces in order + RK update)",
+            "algorithmic_bytes_per_launch": sb,
+            "avg_launch_ms": sa,
         },
         "cpu_baseline": cpu,
     }

@@ -533,7 +533,8 @@ int mmf_mesh_get_time(mmf_mesh *m, double *t, double *dt, int64_t *step, double 
 /* negative p / rho face sides (euler.cpp:94-101) and steps that met a
  * non-finite state */
 int mmf_mesh_get_counters(mmf_mesh *m, int64_t *neg_p, int64_t *neg_rho, int64_t *nonfinite_steps);
-/* HIP-event timing of the face and cell kernels of every stage */
+/* HIP-event timing of every stage's kernel, in cell_ms (the cells evaluate
+ * their faces; face_ms is 0) */
 int mmf_mesh_enable_timing(mmf_mesh *m, int32_t on);
 int mmf_mesh_read_timing(mmf_mesh *m, double *face_ms, double *cell_ms, int64_t *stages);
 

@@ -290,7 +290,7 @@ __global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X
     if (STAGE == 3) {
       // the next step's stage-1 maximum: this cell's, and the virtual states
       // its border and wall faces will have
-      lam_nx = cell_max_eig_fast<DIM>(nu);
+      lam_nx = cell_max_eig<DIM>(nu);
 #pragma unroll
       for (int a = 0; a < DIM; ++a) {
         bool refl = false;

@@ -526,7 +526,7 @@ __device__ __forceinline__ void march_block(const GridDev &g, StageIn<STAGE> in,
         update(Tc.c, Ucur, rhs, nu);
 #pragma unroll
         for (int k = 0; k < NF; ++k) outf.put(k, idx, nu[k]);
-        if (EARLY && STAGE == 3) lam_nx = lam_acc(lam_nx, cell_max_eig_fast<DIM>(nu));
+        if (EARLY && STAGE == 3) lam_nx = lam_acc(lam_nx, cell_max_eig<DIM>(nu));
 #pragma unroll
         for (int k = 0; k < NF; ++k) AFlo[k] = AFhi[k];
         Tc = Tn;
@@ -689,7 +689,7 @@ __device__ __forceinline__ void march_block(const GridDev &g, StageIn<STAGE> in,
 #pragma unroll
         for (int k = 0; k < NF; ++k) outf.put(k, idx, nu[k]);
         if (EARLY && STAGE == 3) {
-          lam_nx = lam_acc(lam_nx, cell_max_eig_fast<DIM>(nu));
+          lam_nx = lam_acc(lam_nx, cell_max_eig<DIM>(nu));
           if (MASK || REFL) lam_nx = lam_acc(lam_nx, virtual_max_eig(gp, nu, LF, m, fb, fn, has_next));
         }
       } else if (STAGE != 3) {

@@ -3,21 +3,24 @@
 // any conforming or hanging-face mesh given as owner / neighbour / area /
 // normal per face and a volume per cell, order 1 (reconstruction.cpp:90-97).
 //
-// Two kernels per RK stage, no float atomics:
-//   k_mesh_faces  one thread per interface, in the caller's interface order:
-//                 coalesced SoA loads of the face's geometry and kind, the two
-//                 side states gathered from the SoA state, the boundary or
-//                 wall virtual state (euler.cpp:198-225), the Rusanov flux
-//                 (euler.cpp:42-73), A*F written per face (SoA), the face
-//                 eigenvalue into the stage maximum;
-//   k_mesh_cells  one thread per cell: a segmented sum over the cell's
-//                 incident faces in increasing face index (the order the
-//                 reference's interface loop reaches them, euler.cpp:153-247:
-//                 RHS -= A*F as owner, += A*F as neighbour), fused with the RK
-//                 stage update (main.cpp:409-495, per-cell volume).
-// The residual of every cell is summed in the reference's face order, so the
-// results are bitwise reproducible and equal to a serial interface loop over
-// the same face list.
+// One kernel per RK stage (k_mesh_stage), one thread per cell: the cell's
+// flux tuple once, then its incident faces in increasing face index (the order
+// the reference's interface loop reaches them, euler.cpp:153-247: RHS -= A*F
+// as owner, += A*F as neighbour), each from the other cell's state or the
+// border's or wall's virtual state (euler.cpp:198-225), and the stage update
+// with the cell's own volume (main.cpp:409-495).  An incidence is 8 bytes: the
+// other cell and the face's kind; the next incidence's state is loaded while
+// this one's flux is formed.  Both cells of a face evaluate it: a face kernel
+// writing A*F for a cell kernel to sum halves the fluxes, but the 40 bytes per
+// face it writes and the cell kernel reads twice cost more (us per step, with a
+// face kernel / without: 491,520 octree cells 188 / 116, 61,440 66 / 41, 7,680
+// 39 / 42; 3.9 million cells 1341 / 858).  What bounds it now is FP64 issue: 215
+// instructions per incidence, a third of them the other cell's tuple.
+//
+// dt is known before stage 1 (Ctrl::lam_now): stage 3 gathers the maximum of
+// the step that follows from the state it writes, and closes the step.  No
+// float atomics: every cell sums in the reference's face order, so the results
+// are bitwise reproducible and equal to a serial interface loop over the list.
 #include <hip/hip_runtime.h>
 
 #include "mmf_device.hpp"
@@ -35,154 +38,280 @@ __device__ __forceinline__ bool mesh_solved(const MeshDev &m, int64_t c) {
 
 // euler.cpp:261-376: the virtual state beyond a border or wall face, from the
 // fluid side's state and the normal pointing out of the fluid.
-__device__ __forceinline__ void mesh_bc_state(const MeshDev &m, int32_t kind, const double *n, const double *fluid,
+__device__ __forceinline__ void mesh_bc_state(const MeshDev &m, uint32_t kind, const double *n, const double *fluid,
                                               double *out) {
-  const int bc = (kind & MESH_KIND_BC_MASK) - 1;
+  const int bc = (int)(kind & MESH_KIND_BC_MASK) - 1;
   if (bc == BC_REFLECTING || bc == BC_WALL) {
     reflect_general(n, fluid, out);
   } else if (bc == BC_DIRICHLET) {
-    prim2cons(m.info + NF * (kind >> MESH_KIND_SLOT_SHIFT), out);
+    prim2cons(m.info + NF * ((kind >> MESH_KIND_SLOT_SHIFT) & 0xffff), out);
   } else {
 #pragma unroll
     for (int k = 0; k < NF; ++k) out[k] = fluid[k];
   }
 }
 
-__global__ __launch_bounds__(MB) void k_mesh_faces(MeshDev m, const double *__restrict__ X, double *__restrict__ AF,
-                                                   Ctrl *ctrl, int slot, int mode) {
-  if (mode == MODE_STEP && !(ctrl->t < ctrl->tmax)) return;  // main.cpp:377 loop guard
-  const int64_t f = (int64_t)blockIdx.x * MB + threadIdx.x;
-  double lam = 0.0;
-  int np = 0, nr = 0;
-  if (f < m.F) {
-    const int64_t o = m.owner[f], nb = m.neigh[f];
-    const bool os = mesh_solved(m, o);
-    const bool ns = nb >= 0 && mesh_solved(m, nb);
-    if (os || ns) {  // euler.cpp:181-183
-      const int32_t kind = m.kind[f];
-      const int32_t nc = (kind >> MESH_KIND_NRM_SHIFT) & 7;
-      double n[3];
-      if (nc == MESH_NRM_GENERAL) {
-        n[0] = m.normal[f];
-        n[1] = m.normal[m.F + f];
-        n[2] = m.normal[2 * m.F + f];
-      } else {  // +-e_a: the same doubles as the caller's (1 or -1, and +0)
-        n[0] = n[1] = n[2] = 0.0;
-        n[nc >> 1] = (nc & 1) ? -1.0 : 1.0;
-      }
-      double L[NF], R[NF];
-      if ((kind & MESH_KIND_BC_MASK) == 0) {
-#pragma unroll
-        for (int k = 0; k < NF; ++k) {
-          L[k] = X[k * m.fs + o];
-          R[k] = X[k * m.fs + nb];
-        }
-      } else if (os) {
-#pragma unroll
-        for (int k = 0; k < NF; ++k) L[k] = X[k * m.fs + o];
-        mesh_bc_state(m, kind, n, L, R);
-      } else {
-        // the fluid side is the neighbour: the boundary state sees the
-        // flipped normal (euler.cpp:219-222); the flux keeps the owner's
-        const double loc[3] = {-1. * n[0], -1. * n[1], -1. * n[2]};
-#pragma unroll
-        for (int k = 0; k < NF; ++k) R[k] = X[k * m.fs + nb];
-        mesh_bc_state(m, kind, loc, R, L);
-      }
-      double Fx[NF];
-      eval_splitting(L, R, n, Fx, &lam, &np, &nr);
-      const int32_t as = (kind >> MESH_KIND_AREA_SHIFT) & 255;
-      const double a = (as == MESH_AREA_GENERAL) ? m.area[f] : m.area_tab[as];
-#pragma unroll
-      for (int k = 0; k < NF; ++k) AF[k * m.F + f] = a * Fx[k];  // euler.cpp:239,245: interfaceArea * fluxes[k]
-    }
+// Owner-outward normal of incidence e.
+__device__ __forceinline__ void mesh_normal(const MeshDev &m, int64_t e, uint32_t kind, double *n) {
+  const uint32_t nc = (kind >> MESH_KIND_NRM_SHIFT) & 7;
+  if (nc == MESH_NRM_GENERAL) {
+    const int64_t f = m.inc[e] >> 1;
+    n[0] = m.normal[f];
+    n[1] = m.normal[m.F + f];
+    n[2] = m.normal[2 * m.F + f];
+  } else {  // +-e_a: the same doubles as the caller's (1 or -1, and +0)
+    const double s = (nc & 1) ? -1.0 : 1.0;
+    n[0] = (nc >> 1) == 0 ? s : 0.0;
+    n[1] = (nc >> 1) == 1 ? s : 0.0;
+    n[2] = (nc >> 1) == 2 ? s : 0.0;
   }
-  // positivity counts: one atomic per wave
-  unsigned int sp = np, sr = nr;
+}
+
+__device__ __forceinline__ double mesh_area(const MeshDev &m, int64_t e, uint32_t kind) {
+  const uint32_t as = (kind >> MESH_KIND_AREA_SHIFT) & 255;
+  return (as == MESH_AREA_GENERAL) ? m.area[m.inc[e] >> 1] : m.area_tab[as];
+}
+
+__device__ __forceinline__ double normal_velocity(const Tup &t, const double *n) {
+  return (t.vel[0] * n[0] + t.vel[1] * n[1] + t.vel[2] * n[2]);  // utils.cpp:37-40
+}
+
+// One incidence's contribution to the cell's residual (euler.cpp:237-247 with
+// eval_splitting, euler.cpp:42-73): own and other tuple, owner-outward normal
+// n, area a; as_neigh: the cell is the face's neighbour (R) side.  The two
+// physical fluxes are added whichever side is whose, and R - L is other - own
+// up to its sign, so own and other need not be swapped into L and R.
+__device__ __forceinline__ double mesh_face(const Tup &own, const Tup &oth, const double *n, double a, bool as_neigh,
+                                            double *rhs) {
+  const double un = normal_velocity(own, n), uo = normal_velocity(oth, n);
+  const double ln = fabs(un) + own.a, lo = fabs(uo) + oth.a;
+  const double lambdaL = as_neigh ? lo : ln, lambdaR = as_neigh ? ln : lo;
+  const double lam = (lambdaR < lambdaL) ? lambdaL : lambdaR;
+  const double s = as_neigh ? 1.0 : -1.0, sl = s * lam, sa = s * a;
+  const double mn = own.c[FID_RHO] * un, mo = oth.c[FID_RHO] * uo;
+  rhs[0] += sa * (0.5 * ((mn + mo) + sl * (oth.c[0] - own.c[0])));
+#pragma unroll
+  for (int b = 0; b < 3; ++b) {
+    const double fn = mn * own.vel[b] + own.p * n[b], fo = mo * oth.vel[b] + oth.p * n[b];
+    rhs[1 + b] += sa * (0.5 * ((fn + fo) + sl * (oth.c[1 + b] - own.c[1 + b])));
+  }
+  rhs[4] += sa * (0.5 * ((un * own.H + uo * oth.H) + sl * (oth.c[4] - own.c[4])));
+  return lam;
+}
+
+// What the faces of solved cell c, in state u, bring to the stage-1 maximum of
+// a step that starts from it (euler.cpp:232-234): the cell's own side of every
+// face, the virtual states, and the side of unsolved neighbours (whose state
+// does not change); a solved neighbour brings its own side.
+__device__ __forceinline__ double mesh_cell_lam(const MeshDev &m, int64_t c, const double *u, const double *U) {
+  // axis-aligned faces between solved cells (and free-flow borders, copies):
+  // |u_a| + c along the axes the cell has faces on
+  const uint32_t axes = m.lam_axes[c];
+  if (axes) return cell_max_eig_axes(u, axes);
+  Tup T;
+  make_tup_fast(u, T);
+  double l = 0.0;
+  const int64_t e1 = m.off[c + 1];
+  for (int64_t e = m.off[c]; e < e1; ++e) {
+    const uint32_t kind = m.adj_kind[e];
+    double n[3];
+    mesh_normal(m, e, kind, n);
+    l = lam_acc(l, fabs(normal_velocity(T, n)) + T.a);
+    double v[NF];
+    if (kind & MESH_KIND_BC_MASK) {
+      if ((kind & MESH_KIND_BC_MASK) - 1 == BC_FREE_FLOW) continue;  // a copy
+      const double s = (kind & MESH_KIND_NEIGH) ? -1. : 1.;
+      const double loc[3] = {s * n[0], s * n[1], s * n[2]};
+      mesh_bc_state(m, kind, loc, u, v);
+    } else {
+      const int64_t o = m.adj[e];
+      if (mesh_solved(m, o)) continue;
+#pragma unroll
+      for (int k = 0; k < NF; ++k) v[k] = U[k * m.fs + o];
+    }
+    Tup V;
+    make_tup(v, V);
+    l = lam_acc(l, fabs(normal_velocity(V, n)) + V.a);
+  }
+  return l;
+}
+
+// Ctrl::lam_now (zero beforehand) from state U.
+__global__ __launch_bounds__(MB) void k_mesh_lam(MeshDev m, const double *U, Ctrl *ctrl) {
+  const int64_t c = (int64_t)blockIdx.x * MB + threadIdx.x;
+  double l = 0.0;
+  if (c < m.N && mesh_solved(m, c)) {
+    double u[NF];
+#pragma unroll
+    for (int k = 0; k < NF; ++k) u[k] = U[k * m.fs + c];
+    l = mesh_cell_lam(m, c, u, U);
+  }
+  unsigned long long b = dbits(l);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
-    sp += __shfl_xor(sp, off, 64);
-    sr += __shfl_xor(sr, off, 64);
+    const unsigned long long o = __shfl_xor(b, off, 64);
+    b = (o > b) ? o : b;
   }
-  if ((threadIdx.x & 63) == 0) {
-    if (sp) atomicAdd(&ctrl->neg_p, (unsigned long long)sp);
-    if (sr) atomicAdd(&ctrl->neg_rho, (unsigned long long)sr);
-  }
-  block_max_to<MB>(ctrl, slot, lam, threadIdx.x);
+  if ((threadIdx.x & 63) == 0 && b) atomicMax(&ctrl->lam_now, b);
 }
 
-// One cell's residual: its incident faces in increasing face index.
-__device__ __forceinline__ void mesh_gather(const MeshDev &m, int64_t c, const double *__restrict__ AF, double *rhs) {
-#pragma unroll
-  for (int k = 0; k < NF; ++k) rhs[k] = 0.;  // euler.cpp:142-148
-  const int64_t e0 = m.off[c], e1 = m.off[c + 1];
-  for (int64_t e = e0; e < e1; ++e) {
-    const int64_t v = m.inc[e];
-    const int64_t f = v >> 1;
-    if (v & 1) {
-#pragma unroll
-      for (int k = 0; k < NF; ++k) rhs[k] += AF[k * m.F + f];
-    } else {
-#pragma unroll
-      for (int k = 0; k < NF; ++k) rhs[k] -= AF[k * m.F + f];
-    }
-  }
+// The other cell and the kind of every incidence, from the face arrays.
+__global__ __launch_bounds__(MB) void k_mesh_adjacency(MeshDev m, int64_t n, int32_t *adj, uint32_t *adj_kind) {
+  const int64_t e = (int64_t)blockIdx.x * MB + threadIdx.x;
+  if (e >= n) return;
+  const int32_t v = m.inc[e], f = v >> 1;
+  adj[e] = (v & 1) ? m.owner[f] : m.neigh[f];
+  adj_kind[e] = (uint32_t)m.kind[f] | ((v & 1) ? MESH_KIND_NEIGH : 0u);
 }
 
-template <int STAGE>
-__global__ __launch_bounds__(MB) void k_mesh_cells(MeshDev m, const double *__restrict__ U, const double *W,
-                                                   double *out, const double *__restrict__ AF, Ctrl *ctrl, int mode) {
-  if (mode == MODE_STEP && !(ctrl->t < ctrl->tmax)) return;
+// Per cell, the axes of its faces if its maximum is that of |u_a| + c along
+// them (mesh_cell_lam), else 0.
+__global__ __launch_bounds__(MB) void k_mesh_lam_axes(MeshDev m, uint8_t *lam_axes) {
   const int64_t c = (int64_t)blockIdx.x * MB + threadIdx.x;
   if (c >= m.N) return;
-  const bool sv = mesh_solved(m, c);
-  const int64_t fs = m.fs;
-  if (mode == MODE_RHS_ONLY) {
-    double rhs[NF] = {0., 0., 0., 0., 0.};
-    if (sv) mesh_gather(m, c, AF, rhs);
-#pragma unroll
-    for (int k = 0; k < NF; ++k) out[k * fs + c] = rhs[k];
-    return;
+  uint32_t axes = 0;
+  bool plain = true;
+  for (int64_t e = m.off[c]; e < m.off[c + 1]; ++e) {
+    const uint32_t kind = m.adj_kind[e], nc = (kind >> MESH_KIND_NRM_SHIFT) & 7, bc = kind & MESH_KIND_BC_MASK;
+    plain = plain && nc != MESH_NRM_GENERAL && (bc ? bc - 1 == BC_FREE_FLOW : mesh_solved(m, m.adj[e]));
+    axes |= 1u << (nc >> 1);
   }
-  if (!sv) return;  // main.cpp:411-414: unsolved cells keep their state
-  const double dt = step_dt(ctrl);
-  double rhs[NF];
-  mesh_gather(m, c, AF, rhs);
-  const double V = m.vol[c];  // rawGetCellVolume
+  lam_axes[c] = plain ? (uint8_t)axes : 0;
+}
+
+// Stage 1 reads X = U and writes W1, stage 2 reads X = W1, stage 3 X = W2 and
+// writes U (out); RHS only: the residual of X = U.
+template <int STAGE>
+__global__ __launch_bounds__(MB, 4) void k_mesh_stage(MeshDev m, const double *__restrict__ X, const double *U,
+                                                   double *out, Ctrl *ctrl, int mode) {
+  const bool step = mode == MODE_STEP;
+  const int64_t c = (int64_t)blockIdx.x * MB + threadIdx.x;
+  const int64_t fs = m.fs;
+  const bool live = c < m.N, sv = live && mesh_solved(m, c);
+  const bool run = !step || ctrl->t < ctrl->tmax;  // main.cpp:377 loop guard
+  const double dt = step ? step_dt_early(ctrl) : 0.0;
+  double lam = 0.0, lam_nx = 0.0;
+  NegCount neg;
+  if (sv && run) {
+    double Xc[NF], Xo[NF];
+    const int64_t e0 = m.off[c], e1 = m.off[c + 1];
+    // other cell and kind of this incidence and the next one
+    int32_t o = 0, o_nx = 0;
+    uint32_t kind = 0, kind_nx = 0;
+    if (e0 < e1) {
+      o = m.adj[e0];
+      kind = m.adj_kind[e0];
+    }
+    if (e0 + 1 < e1) {
+      o_nx = m.adj[e0 + 1];
+      kind_nx = m.adj_kind[e0 + 1];
+    }
 #pragma unroll
-  for (int k = 0; k < NF; ++k) {
-    const double u = U[k * fs + c];
-    double r;
-    if (STAGE == 1) r = u + dt * rhs[k] / V;                                     // main.cpp:421
-    else if (STAGE == 2) r = 0.75 * u + 0.25 * (W[k * fs + c] + dt * rhs[k] / V);  // main.cpp:457
-    else r = (1. / 3) * u + (2. / 3) * (W[k * fs + c] + dt * rhs[k] / V);          // main.cpp:493
-    out[k * fs + c] = r;
+    for (int k = 0; k < NF; ++k) Xc[k] = X[k * fs + c];
+#pragma unroll
+    for (int k = 0; k < NF; ++k) Xo[k] = X[k * fs + (o < 0 ? (int32_t)c : o)];
+    double a = (e0 < e1) ? mesh_area(m, e0, kind) : 0.0;
+    Tup Tc;
+    make_tup_fast(Xc, Tc);
+    double rhs[NF] = {0., 0., 0., 0., 0.};  // euler.cpp:142-148
+    for (int64_t e = e0; e < e1; ++e) {
+      // the next incidence's state and the one after it
+      double Xn[NF];
+      int32_t o2 = 0;
+      uint32_t kind2 = 0;
+#pragma unroll
+      for (int k = 0; k < NF; ++k) Xn[k] = X[k * fs + (o_nx < 0 ? (int32_t)c : o_nx)];
+      const double a_nx = (e + 1 < e1) ? mesh_area(m, e + 1, kind_nx) : 0.0;
+      if (e + 2 < e1) {
+        o2 = m.adj[e + 2];
+        kind2 = m.adj_kind[e + 2];
+      }
+      const bool as_neigh = kind & MESH_KIND_NEIGH;
+      double n[3];
+      mesh_normal(m, e, kind, n);
+      bool count = !as_neigh;
+      if (kind & MESH_KIND_BC_MASK) {
+        // the fluid side is this cell: the boundary state sees its outward
+        // normal (euler.cpp:219-222); the flux keeps the owner's
+        const double s = as_neigh ? -1. : 1.;
+        const double loc[3] = {s * n[0], s * n[1], s * n[2]};
+        double v[NF];
+        mesh_bc_state(m, kind, loc, Xc, v);
+#pragma unroll
+        for (int k = 0; k < NF; ++k) Xo[k] = v[k];
+        count = true;
+      } else if (as_neigh && m.flags) {
+        count = !(m.flags[o] & CELL_SOLVED);
+      }
+      Tup To;
+      make_tup_fast(Xo, To);
+      lam = lam_acc(lam, mesh_face(Tc, To, n, a, as_neigh, rhs));
+      if (count && (tup_negative(Tc) | tup_negative(To))) neg.add(Tc, To);
+#pragma unroll
+      for (int k = 0; k < NF; ++k) Xo[k] = Xn[k];
+      a = a_nx;
+      o = o_nx;
+      kind = kind_nx;
+      o_nx = o2;
+      kind_nx = kind2;
+    }
+    if (!step) {
+#pragma unroll
+      for (int k = 0; k < NF; ++k) out[k * fs + c] = rhs[k];
+    } else {
+      double x[NF], q[NF], nu[NF];
+#pragma unroll
+      for (int k = 0; k < NF; ++k) x[k] = dt * rhs[k];
+      const double V = m.vol[c];  // rawGetCellVolume
+      div5(x, V, quot_rcp(V), quot_divisor(V), q);
+#pragma unroll
+      for (int k = 0; k < NF; ++k) {
+        // stage 1: u + q (main.cpp:421), 2: main.cpp:457, 3: main.cpp:493
+        nu[k] = rk_update_q<STAGE>(STAGE == 1 ? 0.0 : U[k * fs + c], Xc[k], q[k]);
+        out[k * fs + c] = nu[k];
+      }
+      if (STAGE == 3) lam_nx = mesh_cell_lam(m, c, nu, U);
+    }
+  } else if (live && run) {
+    // unsolved cells keep their state (main.cpp:411-414); W2 has its own buffer
+    if (!step) {
+#pragma unroll
+      for (int k = 0; k < NF; ++k) out[k * fs + c] = 0.0;
+    } else if (STAGE == 2) {
+#pragma unroll
+      for (int k = 0; k < NF; ++k) out[k * fs + c] = X[k * fs + c];
+    }
+  }
+  if (!run) return;  // uniform over the grid
+  if (__any(neg.p | neg.r)) neg.flush(ctrl, threadIdx.x);
+  block_max_to<MB>(ctrl, step ? STAGE - 1 : 3, lam, threadIdx.x);
+  if (STAGE == 3 && step) {
+    block_lam_to<MB>(ctrl, lam_nx, threadIdx.x);
+    close_step<true>(ctrl, threadIdx.x);
   }
 }
 
-hipError_t launch_mesh_faces(const MeshDev &m, const double *X, double *AF, Ctrl *ctrl, int slot, int mode,
-                             hipStream_t s) {
-  const int64_t nb = (m.F + MB - 1) / MB;
-  if (nb < 1) return hipSuccess;
-  hipLaunchKernelGGL(k_mesh_faces, dim3((unsigned)nb), dim3(MB), 0, s, m, X, AF, ctrl, slot, mode);
+hipError_t launch_mesh_stage(const MeshDev &m, int stage, const double *X, const double *U, double *out, Ctrl *ctrl,
+                             int mode, hipStream_t s) {
+  const dim3 grid((unsigned)((m.N + MB - 1) / MB)), block(MB);
+  switch (stage) {
+    case 1: hipLaunchKernelGGL(k_mesh_stage<1>, grid, block, 0, s, m, X, U, out, ctrl, mode); break;
+    case 2: hipLaunchKernelGGL(k_mesh_stage<2>, grid, block, 0, s, m, X, U, out, ctrl, mode); break;
+    default: hipLaunchKernelGGL(k_mesh_stage<3>, grid, block, 0, s, m, X, U, out, ctrl, mode);
+  }
   return hipGetLastError();
 }
 
-hipError_t launch_mesh_cells(const MeshDev &m, int stage, const double *U, const double *W, double *out,
-                             const double *AF, Ctrl *ctrl, int mode, hipStream_t s) {
-  const int64_t nb = (m.N + MB - 1) / MB;
-  if (nb < 1) return hipSuccess;
-  switch (stage) {
-    case 1:
-      hipLaunchKernelGGL(k_mesh_cells<1>, dim3((unsigned)nb), dim3(MB), 0, s, m, U, W, out, AF, ctrl, mode);
-      break;
-    case 2:
-      hipLaunchKernelGGL(k_mesh_cells<2>, dim3((unsigned)nb), dim3(MB), 0, s, m, U, W, out, AF, ctrl, mode);
-      break;
-    default:
-      hipLaunchKernelGGL(k_mesh_cells<3>, dim3((unsigned)nb), dim3(MB), 0, s, m, U, W, out, AF, ctrl, mode);
-      break;
-  }
+hipError_t launch_mesh_lam(const MeshDev &m, const double *U, Ctrl *ctrl, hipStream_t s) {
+  hipLaunchKernelGGL(k_mesh_lam, dim3((unsigned)((m.N + MB - 1) / MB)), dim3(MB), 0, s, m, U, ctrl);
+  return hipGetLastError();
+}
+
+hipError_t launch_mesh_adjacency(const MeshDev &m, int64_t n, int32_t *adj, uint32_t *adj_kind, uint8_t *lam_axes,
+                                 hipStream_t s) {
+  if (n < 1) return hipSuccess;
+  hipLaunchKernelGGL(k_mesh_adjacency, dim3((unsigned)((n + MB - 1) / MB)), dim3(MB), 0, s, m, n, adj, adj_kind);
+  hipLaunchKernelGGL(k_mesh_lam_axes, dim3((unsigned)((m.N + MB - 1) / MB)), dim3(MB), 0, s, m, lam_axes);
   return hipGetLastError();
 }
 

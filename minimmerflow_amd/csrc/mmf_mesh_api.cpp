@@ -26,10 +26,12 @@ struct mmf_mesh {
   int32_t dim = 3;
   double hmin = 0.0;
   hipStream_t stream = nullptr;
-  double *dU = nullptr, *dW = nullptr, *dR = nullptr, *dAF = nullptr;
-  int32_t *downer = nullptr, *dneigh = nullptr, *dkind = nullptr, *doff = nullptr, *dinc = nullptr;
+  double *dU = nullptr, *dW = nullptr, *dR = nullptr;
+  int32_t *downer = nullptr, *dneigh = nullptr, *dkind = nullptr, *doff = nullptr, *dinc = nullptr, *dadj = nullptr;
+  uint32_t *dadj_kind = nullptr;
+  int64_t ninc = 0;
   double *darea = nullptr, *dnormal = nullptr, *dinfo = nullptr, *dvol = nullptr, *darea_tab = nullptr;
-  uint8_t *dflags = nullptr;
+  uint8_t *dflags = nullptr, *dlam_axes = nullptr;
   Ctrl *dctrl = nullptr;
   Ctrl *hctrl = nullptr;
   // host copies needed to rebuild the face kinds when the cell flags change:
@@ -37,12 +39,13 @@ struct mmf_mesh {
   std::vector<int32_t> owner, neigh, border_kind, geo;
   std::string err;
   bool timing = false;
-  std::vector<std::pair<hipEvent_t, hipEvent_t>> fev, cev;
-  double face_ms = 0.0, cell_ms = 0.0;
+  std::vector<std::pair<hipEvent_t, hipEvent_t>> events;
+  double stage_ms = 0.0;
   int64_t stages = 0;
   hipGraph_t graph[2] = {nullptr, nullptr};
   hipGraphExec_t exec[2] = {nullptr, nullptr};
   bool use_graphs = true;
+  bool lam_valid = false;  // Ctrl::lam_now holds the current state's maximum
 };
 
 namespace {
@@ -99,39 +102,51 @@ int upload_kinds(mmf_mesh *m, const std::vector<uint8_t> &fluid) {
   return MMF_OK;
 }
 
+// The per-incidence arrays, after the face kinds or the cell flags changed.
+int refresh_adjacency(mmf_mesh *m) {
+  MCHK(m, mmf::launch_mesh_adjacency(m->m, m->ninc, m->dadj, m->dadj_kind, m->dlam_axes, m->stream));
+  MCHK(m, hipStreamSynchronize(m->stream));
+  m->lam_valid = false;
+  return MMF_OK;
+}
+
+// W1 in dW, W2 in dR (the residual's buffer, free between the stages of a
+// step): a stage's cells read their neighbours' input while others are written.
 int launch_stage(mmf_mesh *m, int stage, int mode) {
-  const int slot = (mode == mmf::MODE_RHS_ONLY) ? 3 : stage - 1;
-  const double *X = (stage == 1) ? m->dU : m->dW;
-  hipEvent_t e[4] = {nullptr, nullptr, nullptr, nullptr};
-  if (m->timing)
+  const double *X = (stage == 1) ? m->dU : (stage == 2) ? m->dW : m->dR;
+  double *out = (mode == mmf::MODE_RHS_ONLY) ? m->dR : (stage == 1) ? m->dW : (stage == 2) ? m->dR : m->dU;
+  hipEvent_t e[2] = {nullptr, nullptr};
+  if (m->timing) {
     for (auto &x : e) MCHK(m, hipEventCreate(&x));
-  if (m->timing) MCHK(m, hipEventRecord(e[0], m->stream));
-  hipError_t r = mmf::launch_mesh_faces(m->m, X, m->dAF, m->dctrl, slot, mode, m->stream);
-  if (r != hipSuccess) return mfail(m, MMF_ERR_HIP, std::string("face kernel: ") + hipGetErrorString(r));
+    MCHK(m, hipEventRecord(e[0], m->stream));
+  }
+  const hipError_t r = mmf::launch_mesh_stage(m->m, stage, X, m->dU, out, m->dctrl, mode, m->stream);
+  if (r != hipSuccess) return mfail(m, MMF_ERR_HIP, std::string("stage kernel: ") + hipGetErrorString(r));
   if (m->timing) {
     MCHK(m, hipEventRecord(e[1], m->stream));
-    MCHK(m, hipEventRecord(e[2], m->stream));
-  }
-  double *out = (mode == mmf::MODE_RHS_ONLY) ? m->dR : (stage == 3 ? m->dU : m->dW);
-  r = mmf::launch_mesh_cells(m->m, stage, m->dU, m->dW, out, m->dAF, m->dctrl, mode, m->stream);
-  if (r != hipSuccess) return mfail(m, MMF_ERR_HIP, std::string("cell kernel: ") + hipGetErrorString(r));
-  if (m->timing) {
-    MCHK(m, hipEventRecord(e[3], m->stream));
-    m->fev.emplace_back(e[0], e[1]);
-    m->cev.emplace_back(e[2], e[3]);
+    m->events.emplace_back(e[0], e[1]);
   }
   return MMF_OK;
 }
 
+// The stage-3 launch advances the time.
 int enqueue_steps(mmf_mesh *m, int64_t n) {
-  for (int64_t s = 0; s < n; ++s) {
+  for (int64_t s = 0; s < n; ++s)
     for (int stage = 1; stage <= 3; ++stage) {
       int rc = launch_stage(m, stage, mmf::MODE_STEP);
       if (rc != MMF_OK) return rc;
     }
-    hipError_t e = mmf::launch_advance(m->dctrl, m->stream);
-    if (e != hipSuccess) return mfail(m, MMF_ERR_HIP, std::string("advance: ") + hipGetErrorString(e));
-  }
+  return MMF_OK;
+}
+
+// Before steps: the maximum of the current state, unless the steps before left
+// it (outside any capture).
+int ensure_lam(mmf_mesh *m) {
+  if (m->lam_valid) return MMF_OK;
+  MCHK(m, hipMemsetAsync(&m->dctrl->lam_now, 0, sizeof(unsigned long long), m->stream));
+  const hipError_t e = mmf::launch_mesh_lam(m->m, m->dU, m->dctrl, m->stream);
+  if (e != hipSuccess) return mfail(m, MMF_ERR_HIP, "early dt");
+  m->lam_valid = true;
   return MMF_OK;
 }
 
@@ -153,19 +168,16 @@ int capture(mmf_mesh *m, int slot, int64_t n) {
 }
 
 int collect_timing(mmf_mesh *m) {
-  for (int which = 0; which < 2; ++which) {
-    auto &v = which ? m->cev : m->fev;
-    for (auto &p : v) {
-      MCHK(m, hipEventSynchronize(p.second));
-      float ms = 0.f;
-      MCHK(m, hipEventElapsedTime(&ms, p.first, p.second));
-      (which ? m->cell_ms : m->face_ms) += ms;
-      if (which) m->stages += 1;
-      (void)hipEventDestroy(p.first);
-      (void)hipEventDestroy(p.second);
-    }
-    v.clear();
+  for (auto &p : m->events) {
+    MCHK(m, hipEventSynchronize(p.second));
+    float ms = 0.f;
+    MCHK(m, hipEventElapsedTime(&ms, p.first, p.second));
+    m->stage_ms += ms;
+    m->stages += 1;
+    (void)hipEventDestroy(p.first);
+    (void)hipEventDestroy(p.second);
   }
+  m->events.clear();
   return MMF_OK;
 }
 
@@ -185,13 +197,12 @@ const char *mmf_mesh_last_error(const mmf_mesh *m) { return m ? m->err.c_str() :
 int mmf_mesh_destroy(mmf_mesh *m) {
   if (!m) return MMF_OK;
   if (m->stream) (void)hipStreamSynchronize(m->stream);
-  for (auto *v : {&m->fev, &m->cev})
-    for (auto &p : *v) {
-      (void)hipEventDestroy(p.first);
-      (void)hipEventDestroy(p.second);
-    }
+  for (auto &p : m->events) {
+    (void)hipEventDestroy(p.first);
+    (void)hipEventDestroy(p.second);
+  }
   drop_graphs(m);  // before the buffers their kernel nodes point at
-  for (void *p : {(void *)m->dU, (void *)m->dW, (void *)m->dR, (void *)m->dAF, (void *)m->downer, (void *)m->dneigh,
+  for (void *p : {(void *)m->dU, (void *)m->dW, (void *)m->dR, (void *)m->dadj, (void *)m->dadj_kind, (void *)m->dlam_axes, (void *)m->downer, (void *)m->dneigh,
                   (void *)m->dkind, (void *)m->doff, (void *)m->dinc, (void *)m->darea, (void *)m->dnormal,
                   (void *)m->dinfo, (void *)m->dvol, (void *)m->dflags, (void *)m->dctrl, (void *)m->darea_tab})
     if (p) (void)hipFree(p);
@@ -314,7 +325,7 @@ int mmf_mesh_create(const mmf_mesh_desc *d, mmf_mesh **out) {
   if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess) return cleanup(MMF_ERR_HIP);
   const size_t sb = sizeof(double) * 5 * (size_t)m->m.fs;
   if (hipMalloc(&m->dU, sb) != hipSuccess || hipMalloc(&m->dW, sb) != hipSuccess ||
-      hipMalloc(&m->dR, sb) != hipSuccess || hipMalloc(&m->dAF, sizeof(double) * 5 * (size_t)F) != hipSuccess ||
+      hipMalloc(&m->dR, sb) != hipSuccess ||
       hipMalloc(&m->dkind, sizeof(int32_t) * (size_t)F) != hipSuccess || hipMalloc(&m->dctrl, sizeof(Ctrl)) != hipSuccess ||
       hipHostMalloc(&m->hctrl, sizeof(Ctrl), hipHostMallocDefault) != hipSuccess)
     return cleanup(MMF_ERR_OUT_OF_MEMORY);
@@ -325,27 +336,35 @@ int mmf_mesh_create(const mmf_mesh_desc *d, mmf_mesh **out) {
       upload(m, &m->dinfo, info.data(), info.size()) || upload(m, &m->dvol, d->cell_volume, (size_t)N) ||
       upload(m, &m->doff, count.data(), (size_t)N + 1) || upload(m, &m->dinc, inc.data(), inc.size()))
     return cleanup(MMF_ERR_OUT_OF_MEMORY);
+  m->ninc = (int64_t)inc.size();
+  if (hipMalloc(&m->dadj, sizeof(int32_t) * inc.size()) != hipSuccess ||
+      hipMalloc(&m->dadj_kind, sizeof(uint32_t) * inc.size()) != hipSuccess ||
+      hipMalloc(&m->dlam_axes, (size_t)N) != hipSuccess)
+    return cleanup(MMF_ERR_OUT_OF_MEMORY);
+  m->m.owner = m->downer;
+  m->m.neigh = m->dneigh;
+  m->m.kind = m->dkind;
+  m->m.inc = m->dinc;
+  m->m.adj = m->dadj;
+  m->m.adj_kind = m->dadj_kind;
+  m->m.lam_axes = m->dlam_axes;
+  m->m.off = m->doff;
   m->owner.swap(owner);
   m->neigh.swap(neigh);
   m->border_kind.swap(bkind);
   m->geo.swap(geo);
-  if (upload_kinds(m, {}) != MMF_OK) return cleanup(MMF_ERR_HIP);
+  if (upload_kinds(m, {}) != MMF_OK || refresh_adjacency(m) != MMF_OK) return cleanup(MMF_ERR_HIP);
   if (hipMemset(m->dU, 0, sb) != hipSuccess || hipMemset(m->dW, 0, sb) != hipSuccess ||
       hipMemset(m->dR, 0, sb) != hipSuccess || hipMemset(m->dctrl, 0, sizeof(Ctrl)) != hipSuccess ||
       hipDeviceSynchronize() != hipSuccess)
     return cleanup(MMF_ERR_HIP);
   std::memset(m->hctrl, 0, sizeof(Ctrl));
-  m->m.owner = m->downer;
-  m->m.neigh = m->dneigh;
   m->m.area = m->darea;
   m->m.normal = m->dnormal;
   m->m.area_tab = m->darea_tab;
-  m->m.kind = m->dkind;
   m->m.info = m->dinfo;
   m->m.vol = m->dvol;
   m->m.flags = nullptr;
-  m->m.off = m->doff;
-  m->m.inc = m->dinc;
   *out = m;
   return MMF_OK;
 }
@@ -378,12 +397,12 @@ int mmf_mesh_set_cell_flags(mmf_mesh *m, const uint8_t *fluid, const uint8_t *so
     if (m->dflags) (void)hipFree(m->dflags);
     m->dflags = nullptr;
     m->m.flags = nullptr;
-    return MMF_OK;
+    return refresh_adjacency(m);
   }
   if (!m->dflags) MCHK(m, hipMalloc(&m->dflags, (size_t)N));
   MCHK(m, hipMemcpy(m->dflags, bits.data(), (size_t)N, hipMemcpyHostToDevice));
   m->m.flags = m->dflags;
-  return MMF_OK;
+  return refresh_adjacency(m);
 }
 
 int mmf_mesh_set_state(mmf_mesh *m, const double *U) {
@@ -394,7 +413,8 @@ int mmf_mesh_set_state(mmf_mesh *m, const double *U) {
     for (int k = 0; k < 5; ++k) soa[(size_t)(k * fs + c)] = U[5 * c + k];
   MCHK(m, hipStreamSynchronize(m->stream));
   MCHK(m, hipMemcpy(m->dU, soa.data(), sizeof(double) * soa.size(), hipMemcpyHostToDevice));
-  // the stage buffer starts as a copy, so cells never solved hold finite values
+  m->lam_valid = false;
+  // the stage buffer starts as a copy: cells never solved keep their state in it
   MCHK(m, hipMemcpy(m->dW, soa.data(), sizeof(double) * soa.size(), hipMemcpyHostToDevice));
   return MMF_OK;
 }
@@ -439,6 +459,7 @@ int mmf_mesh_set_time(mmf_mesh *m, double t, double tmax, double cfl) {
   c.t = t;
   c.tmax = tmax;
   c.cfl = cfl;
+  m->lam_valid = false;
   c.hmin = m->hmin;  // main.cpp:351-356
   c.neg_p = m->hctrl->neg_p;
   c.neg_rho = m->hctrl->neg_rho;
@@ -450,6 +471,8 @@ int mmf_mesh_set_time(mmf_mesh *m, double t, double tmax, double cfl) {
 
 int mmf_mesh_advance(mmf_mesh *m, int64_t nsteps) {
   if (!m || nsteps < 0) return MMF_ERR_INVALID;
+  const int rc0 = ensure_lam(m);
+  if (rc0 != MMF_OK) return rc0;
   if (m->timing || !m->use_graphs || nsteps == 0) return enqueue_steps(m, nsteps);
   while (nsteps > 0) {
     const int slot = (nsteps >= GRAPH_STEPS) ? 1 : 0;
@@ -525,7 +548,7 @@ int mmf_mesh_enable_timing(mmf_mesh *m, int32_t on) {
   int rc = collect_timing(m);
   if (rc != MMF_OK) return rc;
   m->timing = on != 0;
-  m->face_ms = m->cell_ms = 0.0;
+  m->stage_ms = 0.0;
   m->stages = 0;
   return MMF_OK;
 }
@@ -534,8 +557,8 @@ int mmf_mesh_read_timing(mmf_mesh *m, double *face_ms, double *cell_ms, int64_t 
   if (!m) return MMF_ERR_INVALID;
   int rc = collect_timing(m);
   if (rc != MMF_OK) return rc;
-  if (face_ms) *face_ms = m->face_ms;
-  if (cell_ms) *cell_ms = m->cell_ms;
+  if (face_ms) *face_ms = 0.0;  // no face kernel: the cells evaluate their faces
+  if (cell_ms) *cell_ms = m->stage_ms;
   if (stages) *stages = m->stages;
   return MMF_OK;
 }

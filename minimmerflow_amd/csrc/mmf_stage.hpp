@@ -13,6 +13,22 @@ namespace mmf {
 // division sequence.
 __device__ __forceinline__ double div_vol(const GridDev &g, double x) { return g.pow2V ? x * g.invV : x / g.V; }
 
+// x_k / V from y, the reciprocal of V, where in_range says V allows it.
+__device__ __forceinline__ void div5(const double *x, double V, double y, bool in_range, double *q) {
+  int e = __builtin_amdgcn_frexp_exp(x[0]);
+#pragma unroll
+  for (int k = 1; k < NF; ++k) {
+    const int ek = __builtin_amdgcn_frexp_exp(x[k]);
+    e = (ek < e) ? ek : e;
+  }
+#pragma unroll
+  for (int k = 0; k < NF; ++k) q[k] = __builtin_amdgcn_div_fixup(quot(x[k], V, y), V, x[k]);
+  if (__builtin_expect(e < QUOT_MIN_EXP || !in_range, 0)) {
+#pragma unroll
+    for (int k = 0; k < NF; ++k) q[k] = x[k] / V;
+  }
+}
+
 // The five x_k / V of a cell's update.  Where V is not a power of two they
 // share its reciprocal (quot(): five instead of fourteen issue slots each), the
 // division sequences only where an operand is outside its range.
@@ -23,18 +39,7 @@ __device__ __forceinline__ void div_vol5(const GridDev &g, const double *x, doub
     for (int k = 0; k < NF; ++k) q[k] = x[k] * g.invV;
     return;
   }
-  int e = __builtin_amdgcn_frexp_exp(x[0]);
-#pragma unroll
-  for (int k = 1; k < NF; ++k) {
-    const int ek = __builtin_amdgcn_frexp_exp(x[k]);
-    e = (ek < e) ? ek : e;
-  }
-#pragma unroll
-  for (int k = 0; k < NF; ++k) q[k] = __builtin_amdgcn_div_fixup(quot(x[k], g.V, g.invV), g.V, x[k]);
-  if (__builtin_expect(e < QUOT_MIN_EXP || !g.quotV, 0)) {
-#pragma unroll
-    for (int k = 0; k < NF; ++k) q[k] = x[k] / g.V;
-  }
+  div5(x, g.V, g.invV, g.quotV, q);
 }
 
 // Tile of block b of n: consecutive blocks go to the 8 XCDs in turn; each XCD
@@ -231,31 +236,28 @@ __device__ __forceinline__ void block_lam_to(Ctrl *ctrl, double v, int tid) {
 // fl(max_a |m_a| / |rho|), and fl(x + a) is non-decreasing in x; T is
 // cons2prim's (utils.cpp:48-63) to the bit.  A NaN momentum wins the u64
 // maximum and stays NaN.
-template <int DIM>
-__device__ __forceinline__ double cell_max_eig(const double *c) {
-  double m = fabs(c[FID_RHO_U]);
+// Over the axes in the mask, with the shared reciprocal of rho (the division
+// sequences outside its range).
+__device__ __forceinline__ double cell_max_eig_axes(const double *c, uint32_t axes) {
+  double m = 0.0;
 #pragma unroll
-  for (int a = 1; a < DIM; ++a) m = lam_acc(m, fabs(c[FID_RHO_U + a]));
-  const double umax = m / fabs(c[FID_RHO]);
-  const double K = (c[FID_RHO_U] * c[FID_RHO_U] + c[FID_RHO_V] * c[FID_RHO_V] + c[FID_RHO_W] * c[FID_RHO_W]) /
-                   (c[FID_RHO] * c[FID_RHO]);
-  const double T = (2.0 * c[FID_RHO_E] / c[FID_RHO] - K) / (2.0 / (GAMMA - 1.0));
-  return umax + sqrt(GAMMA * T);
-}
-
-// cell_max_eig with the shared reciprocal of rho.
-template <int DIM>
-__device__ __forceinline__ double cell_max_eig_fast(const double *c) {
-  double m = fabs(c[FID_RHO_U]);
-#pragma unroll
-  for (int a = 1; a < DIM; ++a) m = lam_acc(m, fabs(c[FID_RHO_U + a]));
+  for (int a = 0; a < 3; ++a)
+    if (axes & (1u << a)) m = lam_acc(m, fabs(c[FID_RHO_U + a]));
   const double rho = fabs(c[FID_RHO]), y = quot_rcp(c[FID_RHO]);
   double T, s;
   const bool ok = temperature_quot(c, y, T, s);
   const double l = quot(m, rho, fabs(y)) + s;
-  if (__builtin_expect(!(ok & (__builtin_amdgcn_frexp_exp(m) >= QUOT_MIN_EXP) & quot_divisor(rho) & finite_bits(l)), 0))
-    return cell_max_eig<DIM>(c);
-  return l;
+  if (__builtin_expect(ok & (__builtin_amdgcn_frexp_exp(m) >= QUOT_MIN_EXP) & quot_divisor(rho) & finite_bits(l), 1))
+    return l;
+  const double K = (c[FID_RHO_U] * c[FID_RHO_U] + c[FID_RHO_V] * c[FID_RHO_V] + c[FID_RHO_W] * c[FID_RHO_W]) /
+                   (c[FID_RHO] * c[FID_RHO]);
+  T = (2.0 * c[FID_RHO_E] / c[FID_RHO] - K) / (2.0 / (GAMMA - 1.0));
+  return m / rho + sqrt(GAMMA * T);
+}
+
+template <int DIM>
+__device__ __forceinline__ double cell_max_eig(const double *c) {
+  return cell_max_eig_axes(c, DIM == 3 ? 7u : 3u);
 }
 
 // Neighbour of cell q along axis a (dir +-1); false outside a non-periodic border.
