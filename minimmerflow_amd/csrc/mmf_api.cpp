@@ -20,6 +20,7 @@
 #include "mmf_ctx.hpp"
 #include "mmf_internal.hpp"
 #include "mmf_learn.hpp"
+#include "mmf_transfer.hpp"
 
 
 namespace {
@@ -275,6 +276,7 @@ int mmf_create(const mmf_grid_desc *d, mmf_ctx **out) {
 
   mmf_ctx *ctx = new (std::nothrow) mmf_ctx();
   if (!ctx) return MMF_ERR_OUT_OF_MEMORY;
+  mmf::transfer_attach();
   ctx->desc = *d;
   GridDev &g = ctx->g;
   g = gd;
@@ -311,6 +313,7 @@ int mmf_create(const mmf_grid_desc *d, mmf_ctx **out) {
 
 int mmf_destroy(mmf_ctx *ctx) {
   if (!ctx) return MMF_OK;
+  mmf::transfer_detach();
   mmf_output_release(ctx);
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   for (auto &p : ctx->events) {
@@ -668,8 +671,7 @@ int mmf_get_state(mmf_ctx *ctx, double *U) {
   if (!ctx || !U) return MMF_ERR_INVALID;
   const int64_t N = ctx->g.N, fs = ctx->g.fs;
   HIPCHK(ctx, mmf::launch_soa_to_aos(ctx->dU, ctx->draw, N, fs, ctx->dR, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  HIPCHK(ctx, hipMemcpy(U, ctx->dR, sizeof(double) * 5 * (size_t)N, hipMemcpyDeviceToHost));
+  HIPCHK(ctx, mmf::copy_to_host(U, ctx->dR, sizeof(double) * 5 * (size_t)N, ctx->stream));
   return MMF_OK;
 }
 
@@ -683,8 +685,7 @@ int mmf_compute_rhs(mmf_ctx *ctx, double *rhs, double *max_eig) {
     // the copy of U it holds after mmf_set_state
     const int64_t N = ctx->g.N, fs = ctx->g.fs;
     HIPCHK(ctx, mmf::launch_soa_to_aos(ctx->dR, ctx->draw, N, fs, ctx->dW, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    HIPCHK(ctx, hipMemcpy(rhs, ctx->dW, sizeof(double) * 5 * (size_t)N, hipMemcpyDeviceToHost));
+    HIPCHK(ctx, mmf::copy_to_host(rhs, ctx->dW, sizeof(double) * 5 * (size_t)N, ctx->stream));
     HIPCHK(ctx, hipMemcpyAsync(ctx->dW, ctx->dU, sizeof(double) * 5 * (size_t)fs, hipMemcpyDeviceToDevice, ctx->stream));
   }
   int r2 = read_ctrl(ctx);

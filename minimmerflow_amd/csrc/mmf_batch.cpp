@@ -18,6 +18,7 @@
 
 #include "mmf.h"
 #include "mmf_batch.hpp"
+#include "mmf_transfer.hpp"
 #include "mmf_internal.hpp"
 
 using mmf::BatchCase;
@@ -218,6 +219,7 @@ int mmf_batch_create(const mmf_grid_desc *cases, int32_t ncases, mmf_batch **out
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) return MMF_ERR_NO_DEVICE;
   mmf_batch *b = new (std::nothrow) mmf_batch();
   if (!b) return MMF_ERR_OUT_OF_MEMORY;
+  mmf::transfer_attach();
   auto cleanup = [&](int code) {
     mmf_batch_destroy(b);
     return code;
@@ -258,6 +260,7 @@ int mmf_batch_create(const mmf_grid_desc *cases, int32_t ncases, mmf_batch **out
     int e2 = 0;
     g.pow2V = std::frexp(g.V, &e2) == 0.5 ? 1 : 0;
     g.invV = 1.0 / g.V;
+    g.quotV = g.V > 0x1p-100 && g.V < 0x1p100 ? 1 : 0;
     g.pow2A = std::frexp(g.A, &e2) == 0.5 ? 1 : 0;
     g.halfA = 0.5 * g.A;
     c.offset = off;
@@ -290,6 +293,7 @@ int mmf_batch_create(const mmf_grid_desc *cases, int32_t ncases, mmf_batch **out
 
 int mmf_batch_destroy(mmf_batch *b) {
   if (!b) return MMF_OK;
+  mmf::transfer_detach();
   if (b->stream) (void)hipStreamSynchronize(b->stream);
   for (auto &p : b->events) {
     (void)hipEventDestroy(p.first);
@@ -318,12 +322,14 @@ int mmf_batch_set_state(mmf_batch *b, int32_t ci, const double *U) {
   if (!b || !U || ci < 0 || ci >= b->ncases) return MMF_ERR_INVALID;
   const BatchCase &c = b->hcases[(size_t)ci];
   const int64_t N = c.g.N, fs = c.g.fs;
-  std::vector<double> soa((size_t)(5 * fs), 0.0);
-  for (int64_t i = 0; i < N; ++i)
-    for (int k = 0; k < 5; ++k) soa[(size_t)(k * fs + i)] = U[5 * i + k];
+  // the rows cross as they are; the planes are formed on the device, through
+  // the residual's buffer (dead between steps)
   BCHK(b, hipStreamSynchronize(b->stream));
-  BCHK(b, hipMemcpy(b->dU + c.offset, soa.data(), sizeof(double) * soa.size(), hipMemcpyHostToDevice));
-  BCHK(b, hipMemcpy(b->dW + c.offset, b->dU + c.offset, sizeof(double) * soa.size(), hipMemcpyDeviceToDevice));
+  BCHK(b, hipMemcpy(b->dR + c.offset, U, sizeof(double) * 5 * (size_t)N, hipMemcpyHostToDevice));
+  BCHK(b, mmf::launch_aos_to_soa(b->dR + c.offset, nullptr, N, fs, b->dU + c.offset, b->stream));
+  BCHK(b, hipMemcpyAsync(b->dW + c.offset, b->dU + c.offset, sizeof(double) * 5 * (size_t)fs, hipMemcpyDeviceToDevice,
+                         b->stream));
+  BCHK(b, hipStreamSynchronize(b->stream));
   return MMF_OK;
 }
 
@@ -331,11 +337,8 @@ int mmf_batch_get_state(mmf_batch *b, int32_t ci, double *U) {
   if (!b || !U || ci < 0 || ci >= b->ncases) return MMF_ERR_INVALID;
   const BatchCase &c = b->hcases[(size_t)ci];
   const int64_t N = c.g.N, fs = c.g.fs;
-  std::vector<double> soa((size_t)(5 * fs));
-  BCHK(b, hipStreamSynchronize(b->stream));
-  BCHK(b, hipMemcpy(soa.data(), b->dU + c.offset, sizeof(double) * soa.size(), hipMemcpyDeviceToHost));
-  for (int64_t i = 0; i < N; ++i)
-    for (int k = 0; k < 5; ++k) U[5 * i + k] = soa[(size_t)(k * fs + i)];
+  BCHK(b, mmf::launch_soa_to_aos(b->dU + c.offset, nullptr, N, fs, b->dR + c.offset, b->stream));
+  BCHK(b, mmf::copy_to_host(U, b->dR + c.offset, sizeof(double) * 5 * (size_t)N, b->stream));
   return MMF_OK;
 }
 

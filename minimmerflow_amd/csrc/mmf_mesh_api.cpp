@@ -17,6 +17,7 @@
 #include "mmf.h"
 #include "mmf_internal.hpp"
 #include "mmf_mesh.hpp"
+#include "mmf_transfer.hpp"
 
 using mmf::Ctrl;
 using mmf::MeshDev;
@@ -196,6 +197,7 @@ const char *mmf_mesh_last_error(const mmf_mesh *m) { return m ? m->err.c_str() :
 
 int mmf_mesh_destroy(mmf_mesh *m) {
   if (!m) return MMF_OK;
+  mmf::transfer_detach();
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   for (auto &p : m->events) {
     (void)hipEventDestroy(p.first);
@@ -313,6 +315,7 @@ int mmf_mesh_create(const mmf_mesh_desc *d, mmf_mesh **out) {
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) return MMF_ERR_NO_DEVICE;
   mmf_mesh *m = new (std::nothrow) mmf_mesh();
   if (!m) return MMF_ERR_OUT_OF_MEMORY;
+  mmf::transfer_attach();
   auto cleanup = [&](int code) {
     mmf_mesh_destroy(m);
     return code;
@@ -408,30 +411,28 @@ int mmf_mesh_set_cell_flags(mmf_mesh *m, const uint8_t *fluid, const uint8_t *so
 int mmf_mesh_set_state(mmf_mesh *m, const double *U) {
   if (!m || !U) return MMF_ERR_INVALID;
   const int64_t N = m->m.N, fs = m->m.fs;
-  std::vector<double> soa((size_t)(5 * fs), 0.0);
-  for (int64_t c = 0; c < N; ++c)
-    for (int k = 0; k < 5; ++k) soa[(size_t)(k * fs + c)] = U[5 * c + k];
+  // the rows cross as they are; the planes are formed on the device, through
+  // dR (dead between steps)
   MCHK(m, hipStreamSynchronize(m->stream));
-  MCHK(m, hipMemcpy(m->dU, soa.data(), sizeof(double) * soa.size(), hipMemcpyHostToDevice));
+  MCHK(m, hipMemcpy(m->dR, U, sizeof(double) * 5 * (size_t)N, hipMemcpyHostToDevice));
+  MCHK(m, mmf::launch_aos_to_soa(m->dR, nullptr, N, fs, m->dU, m->stream));
   m->lam_valid = false;
   // the stage buffer starts as a copy: cells never solved keep their state in it
-  MCHK(m, hipMemcpy(m->dW, soa.data(), sizeof(double) * soa.size(), hipMemcpyHostToDevice));
+  MCHK(m, hipMemcpyAsync(m->dW, m->dU, sizeof(double) * 5 * (size_t)fs, hipMemcpyDeviceToDevice, m->stream));
   return MMF_OK;
 }
 
-static int get_soa(mmf_mesh *m, const double *dsrc, double *U) {
+// Rows of the planes src through rows, a device buffer of their size.
+static int get_rows(mmf_mesh *m, const double *src, double *rows, double *U) {
   const int64_t N = m->m.N, fs = m->m.fs;
-  std::vector<double> soa((size_t)(5 * fs));
-  MCHK(m, hipStreamSynchronize(m->stream));
-  MCHK(m, hipMemcpy(soa.data(), dsrc, sizeof(double) * soa.size(), hipMemcpyDeviceToHost));
-  for (int64_t c = 0; c < N; ++c)
-    for (int k = 0; k < 5; ++k) U[5 * c + k] = soa[(size_t)(k * fs + c)];
+  MCHK(m, mmf::launch_soa_to_aos(src, nullptr, N, fs, rows, m->stream));
+  MCHK(m, mmf::copy_to_host(U, rows, sizeof(double) * 5 * (size_t)N, m->stream));
   return MMF_OK;
 }
 
 int mmf_mesh_get_state(mmf_mesh *m, double *U) {
   if (!m || !U) return MMF_ERR_INVALID;
-  return get_soa(m, m->dU, U);
+  return get_rows(m, m->dU, m->dR, U);
 }
 
 int mmf_mesh_compute_rhs(mmf_mesh *m, double *rhs, double *max_eig) {
@@ -441,8 +442,10 @@ int mmf_mesh_compute_rhs(mmf_mesh *m, double *rhs, double *max_eig) {
   int rc = launch_stage(m, 1, mmf::MODE_RHS_ONLY);
   if (rc != MMF_OK) return rc;
   if (rhs) {
-    rc = get_soa(m, m->dR, rhs);
+    // through W, dead between steps but for the copy of U it then holds again
+    rc = get_rows(m, m->dR, m->dW, rhs);
     if (rc != MMF_OK) return rc;
+    MCHK(m, hipMemcpyAsync(m->dW, m->dU, sizeof(double) * 5 * (size_t)m->m.fs, hipMemcpyDeviceToDevice, m->stream));
   }
   rc = read_ctrl(m);
   if (rc != MMF_OK) return rc;
