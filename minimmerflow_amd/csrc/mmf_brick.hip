@@ -54,15 +54,6 @@ __device__ __forceinline__ void get_tup(const double *lds, int slot, Tup &t) {
   t.H = lds[10 * NS + slot];
 }
 
-__device__ __forceinline__ unsigned long long wave_max(unsigned long long b) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const unsigned long long o = __shfl_xor(b, off, 64);
-    b = (o > b) ? o : b;
-  }
-  return b;
-}
-
 }  // namespace
 
 // MASK: the grid has cell flags (every fluid cell solved).  P2: A and V are
@@ -326,22 +317,23 @@ __global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X
 
   if (!run) return;  // uniform over the grid: t does not change before the step closes
   if (anyneg || MASK) neg.flush(ctrl, tid);
-  const unsigned long long ml = wave_max(dbits(lam));
-  const unsigned long long mn = (STAGE == 3 && step) ? wave_max(dbits(lam_nx)) : 0ull;
+  if (STAGE == 1 && step) return;  // its maximum was known before the step
+  const unsigned long long ml = wave_max_u64(dbits(lam));
+  const unsigned long long mn = (STAGE == 3) ? wave_max_u64(dbits(lam_nx)) : 0ull;
   if ((tid & 63) == 0) {
     red[tid >> 6] = ml;
     red[NW + (tid >> 6)] = mn;
   }
-  __syncthreads();
+  if (NW > 1) __syncthreads();
   if (tid == 0) {
-    unsigned long long m = red[0], n = red[NW];
+    unsigned long long m = ml, n = mn;
 #pragma unroll
     for (int i = 1; i < NW; ++i) {
       m = (red[i] > m) ? red[i] : m;
       n = (red[NW + i] > n) ? red[NW + i] : n;
     }
     stage_max_put(ctrl, step ? STAGE - 1 : 3, m);
-    if (STAGE == 3 && step) lam_put(ctrl, n);
+    if (STAGE == 3) lam_put(ctrl, n);
   }
   if (STAGE == 3 && step) close_step<true>(ctrl, tid);
 }

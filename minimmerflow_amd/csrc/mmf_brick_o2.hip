@@ -83,15 +83,6 @@ __device__ __forceinline__ void face_tup(const double *mean, const double *half,
   if (__builtin_expect(!(T.c[FID_RHO] > 0.0) || !(T.p > 0.0), 0)) make_tup(mean, T);
 }
 
-__device__ __forceinline__ unsigned long long wave_max(unsigned long long b) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const unsigned long long o = __shfl_xor(b, off, 64);
-    b = (o > b) ? o : b;
-  }
-  return b;
-}
-
 }  // namespace
 
 template <int DIM, int STAGE, bool P2>
@@ -325,7 +316,7 @@ __global__ __launch_bounds__(DIM == 3 ? 256 : 64, 3) void k_brick_o2(GridDev g, 
     }
   }
   if (__any(neg.p | neg.r)) neg.flush(ctrl, tid);
-  const unsigned long long m = wave_max(dbits(lam));
+  const unsigned long long m = wave_max_u64(dbits(lam));
   const int slot = step ? STAGE - 1 : 3;
   if (NW == 1) {
     if (tid == 0) stage_max_put(ctrl, slot, m);

@@ -248,12 +248,7 @@ __global__ __launch_bounds__(256) void k_lam_init(GridDev g, const double *U, Ct
     }
   }
   __shared__ unsigned long long red[4];
-  unsigned long long b = dbits(m);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const unsigned long long o = __shfl_xor(b, off, 64);
-    b = (o > b) ? o : b;
-  }
+  const unsigned long long b = wave_max_u64(dbits(m));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = b;
   __syncthreads();
   if (threadIdx.x == 0) {

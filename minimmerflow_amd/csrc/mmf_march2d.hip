@@ -634,15 +634,9 @@ __device__ __forceinline__ bool flat_item(const GridDev &g, int tile) {
   return lo && hi;
 }
 
-// wave-wide max of non-negative doubles as u64 bits; lane 0 holds the result
+// wave-wide max of non-negative doubles as u64 bits
 __device__ __forceinline__ unsigned long long wave_max_bits(double v) {
-  unsigned long long b = dbits(v);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    unsigned long long o = __shfl_xor(b, off, 64);
-    b = (o > b) ? o : b;
-  }
-  return b;
+  return wave_max_u64(dbits(v));
 }
 
 }  // namespace

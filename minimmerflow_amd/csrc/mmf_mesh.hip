@@ -146,12 +146,7 @@ __global__ __launch_bounds__(MB) void k_mesh_lam(MeshDev m, const double *U, Ctr
     for (int k = 0; k < NF; ++k) u[k] = U[k * m.fs + c];
     l = mesh_cell_lam(m, c, u, U);
   }
-  unsigned long long b = dbits(l);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const unsigned long long o = __shfl_xor(b, off, 64);
-    b = (o > b) ? o : b;
-  }
+  const unsigned long long b = wave_max_u64(dbits(l));
   if ((threadIdx.x & 63) == 0 && b) atomicMax(&ctrl->lam_now, b);
 }
 
@@ -284,6 +279,7 @@ __global__ __launch_bounds__(MB, 4) void k_mesh_stage(MeshDev m, const double *_
   }
   if (!run) return;  // uniform over the grid
   if (__any(neg.p | neg.r)) neg.flush(ctrl, threadIdx.x);
+  if (STAGE == 1 && step) return;  // its maximum was known before the step
   block_max_to<MB>(ctrl, step ? STAGE - 1 : 3, lam, threadIdx.x);
   if (STAGE == 3 && step) {
     block_lam_to<MB>(ctrl, lam_nx, threadIdx.x);

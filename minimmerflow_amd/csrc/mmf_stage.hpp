@@ -49,6 +49,27 @@ __device__ __forceinline__ int xcd_range(int b, int n) {
   return x * q + (x < r ? x : r) + b / 8;
 }
 
+// Largest of a wave's 32-bit values (every lane active), in a scalar.
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  auto step = [](uint32_t a, uint32_t b) { return a > b ? a : b; };
+  v = step(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));  // row_shr:1
+  v = step(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));
+  v = step(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));
+  v = step(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));
+  v = step(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+  v = step(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// The same of 64-bit values: the high words, then the low words of the lanes
+// that hold the largest (16 VALU instructions; the shuffles it replaces took
+// 30 and 12 LDS operations, an eighth of a 2D brick's stage).
+__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long b) {
+  const uint32_t hi = (uint32_t)(b >> 32), h = wave_max_u32(hi);
+  const uint32_t l = wave_max_u32(hi == h ? (uint32_t)b : 0u);
+  return ((unsigned long long)h << 32) | l;
+}
+
 // Linear index of this block in its grid.
 __device__ __forceinline__ unsigned int block_linear() {
   return blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
@@ -117,12 +138,13 @@ __device__ __forceinline__ void advance_ctrl_wave(Ctrl *c, int lane) {
   const unsigned long long e0 = __shfl(v, 0, 64), e1 = __shfl(v, EIG_SPLIT, 64), e2 = __shfl(v, 2 * EIG_SPLIT, 64);
   const unsigned long long e3 = __shfl(v, 3 * EIG_SPLIT, 64);
   if (lane == 0 && c->t < c->tmax) {
+    // with early dt the stage-1 maximum is the one known before the step
     const unsigned long long me = EARLY ? c->lam_now : e0;
-    c->last_eig[0] = __longlong_as_double((long long)e0);
+    c->last_eig[0] = __longlong_as_double((long long)me);
     c->last_eig[1] = __longlong_as_double((long long)e1);
     c->last_eig[2] = __longlong_as_double((long long)e2);
     if (EARLY) c->lam_now = e3;
-    if (e0 >= NONFINITE_BITS || e1 >= NONFINITE_BITS || e2 >= NONFINITE_BITS || me >= NONFINITE_BITS) {
+    if (e1 >= NONFINITE_BITS || e2 >= NONFINITE_BITS || me >= NONFINITE_BITS) {
       c->nonfinite += 1;  // a NaN or infinite state: the time does not advance
     } else {
       double dt = 0.9 * c->cfl * c->hmin / __longlong_as_double((long long)me);
@@ -190,12 +212,7 @@ struct StageIn {
 template <int NT>
 __device__ __forceinline__ void block_max_to(Ctrl *ctrl, int s, double v, int tid) {
   __shared__ unsigned long long red[(NT + 63) / 64];
-  unsigned long long b = dbits(v);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    unsigned long long o = __shfl_xor(b, off, 64);
-    b = (o > b) ? o : b;
-  }
+  const unsigned long long b = wave_max_u64(dbits(v));
   const int lane = tid & 63, wid = tid >> 6;
   if (lane == 0) red[wid] = b;
   __syncthreads();
@@ -212,12 +229,7 @@ __device__ __forceinline__ void block_max_to(Ctrl *ctrl, int s, double v, int ti
 template <int NT>
 __device__ __forceinline__ void block_lam_to(Ctrl *ctrl, double v, int tid) {
   __shared__ unsigned long long red[(NT + 63) / 64];
-  unsigned long long b = dbits(v);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    unsigned long long o = __shfl_xor(b, off, 64);
-    b = (o > b) ? o : b;
-  }
+  const unsigned long long b = wave_max_u64(dbits(v));
   const int lane = tid & 63, wid = tid >> 6;
   if (lane == 0) red[wid] = b;
   __syncthreads();
