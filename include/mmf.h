@@ -358,8 +358,10 @@ int mmf_get_centroids(const mmf_ctx *ctx, double *xyz);
 /* The reference runs one grid per process; a batch advances ncases uneven 2D
  * grids together, each with the reference's own time loop (main.cpp:386-512:
  * its own dt from its own stage-1 maximum eigenvalue, its own end time).
- * One step is three persistent stage launches plus the per-case time update,
- * captured once into a HIP graph and replayed.  Cases are order 1, with no
+ * One step is three stage launches, captured once into a HIP graph and
+ * replayed: below 2^23 cells in all, a block per brick of 16 x 16 cells (the
+ * last stage also advances every case's time); from there, persistent blocks
+ * taking strip items, and a launch for the time update.  Cases are order 1, with no
  * immersed bodies; border BCs as in the grid descriptor, periodic allowed.  Per
  * case the results are bitwise those of a single-grid mmf_ctx. */
 typedef struct mmf_batch mmf_batch;
@@ -376,7 +378,7 @@ int mmf_batch_get_state(mmf_batch *b, int32_t ci, double *cons);
 int mmf_batch_set_initial_states(mmf_batch *b, const mmf_problem *problems);
 /* per-case start time, end time and CFL (arrays of ncases) */
 int mmf_batch_set_time(mmf_batch *b, const double *t0, const double *tmax, const double *cfl);
-/* rows per work item and persistent grid size of stages 2 and 3 (<= 0 keeps
+/* Strips: rows per work item and persistent grid size of stages 2 and 3 (<= 0 keeps
  * the current value; stage 1, resident at three waves per SIMD where they
  * are at two, runs proportionally more blocks).  The items are cut into one
  * queue per XCD, runs of neighbouring strips and row bands of equal cost; a

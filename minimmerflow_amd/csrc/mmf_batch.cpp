@@ -40,6 +40,10 @@ struct mmf_batch {
   BatchCase *dcases = nullptr;
   int *ditems = nullptr;
   int nitems = 0;
+  int *dbricks = nullptr;  // (case, brick) of every block of the brick stages
+  int nbricks = 0;
+  bool bricks = false;     // the stages run as bricks
+  bool lam_valid = false;  // every case's Ctrl::lam_now is its state's
   mmf::BatchQueues queues{};
   unsigned int *dcounters = nullptr;
   int chunk = 16;
@@ -129,6 +133,39 @@ int build_items(mmf_batch *b) {
   return MMF_OK;
 }
 
+// Batches below this many cells run as bricks, one block each, larger ones as
+// the persistent strips, which issue a little less per cell but march their
+// rows one after another (us per step, strips / bricks, MI355X: 8 cases of
+// 316,416 cells 164 / 41, 60 of 1,728,000 217 / 129, 512 of 13,116,160 1012 /
+// 1064).
+constexpr int64_t BATCH_BRICKS_MAX_CELLS = (int64_t)1 << 23;
+
+// The blocks of the brick stages, in case order.
+int build_bricks(mmf_batch *b) {
+  b->bricks = b->total_cells < BATCH_BRICKS_MAX_CELLS;
+  if (!b->bricks) return MMF_OK;
+  std::vector<int> v;
+  for (int i = 0; i < b->ncases; ++i) {
+    const int64_t n = mmf::batch_bricks(b->hcases[(size_t)i].g);
+    for (int64_t k = 0; k < n; ++k) {
+      v.push_back(i);
+      v.push_back((int)k);
+    }
+  }
+  b->nbricks = (int)(v.size() / 2);
+  BCHK(b, hipMalloc(&b->dbricks, sizeof(int) * v.size()));
+  BCHK(b, hipMemcpy(b->dbricks, v.data(), sizeof(int) * v.size(), hipMemcpyHostToDevice));
+  return MMF_OK;
+}
+
+// Before brick steps: every case's maximum, unless the steps before left it.
+int ensure_lam(mmf_batch *b) {
+  if (!b->bricks || b->lam_valid) return MMF_OK;
+  BCHK(b, mmf::launch_batch_lam(b->dcases, b->ncases, b->dbricks, b->nbricks, b->dU, b->stream));
+  b->lam_valid = true;
+  return MMF_OK;
+}
+
 // Persistent blocks of stage s: 'blocks' for stages 2 and 3; stage 1, which
 // holds three waves per SIMD where they hold two, proportionally more.
 int stage_blocks(const mmf_batch *b, int s) {
@@ -137,6 +174,14 @@ int stage_blocks(const mmf_batch *b, int s) {
 }
 
 int enqueue_step(mmf_batch *b) {
+  if (b->bricks) {  // stage 3 advances every case's time
+    for (int s = 1; s <= 3; ++s) {
+      const hipError_t e =
+          mmf::launch_batch_bricks(s, b->dcases, b->dbricks, b->nbricks, b->dU, b->dR, b->dW, b->stream);
+      if (e != hipSuccess) return bfail(b, MMF_ERR_HIP, std::string("batch stage: ") + hipGetErrorString(e));
+    }
+    return MMF_OK;
+  }
   for (int s = 1; s <= 3; ++s) {
     hipError_t e = mmf::launch_batch_stage(s, b->dcases, b->ditems, b->queues, b->dcounters, b->dU, b->dR, b->dW,
                                            stage_blocks(b, s), b->stream);
@@ -286,7 +331,7 @@ int mmf_batch_create(const mmf_grid_desc *cases, int32_t ncases, mmf_batch **out
     return cleanup(MMF_ERR_HIP);
   std::memset(b->hctrl, 0, sizeof(Ctrl) * (size_t)ncases);
   for (int i = 0; i < ncases; ++i) b->hcases[(size_t)i].ctrl = b->dctrl + i;
-  if (build_items(b) != MMF_OK) return cleanup(MMF_ERR_HIP);
+  if (build_items(b) != MMF_OK || build_bricks(b) != MMF_OK) return cleanup(MMF_ERR_HIP);
   *out = b;
   return MMF_OK;
 }
@@ -301,7 +346,7 @@ int mmf_batch_destroy(mmf_batch *b) {
   }
   drop_graph(b);
   for (void *p : {(void *)b->dU, (void *)b->dR, (void *)b->dW, (void *)b->dctrl, (void *)b->dcases,
-                  (void *)b->ditems, (void *)b->dcounters, (void *)b->dpartials, (void *)b->derr})
+                  (void *)b->ditems, (void *)b->dbricks, (void *)b->dcounters, (void *)b->dpartials, (void *)b->derr})
     if (p) (void)hipFree(p);
   if (b->hctrl) (void)hipHostFree(b->hctrl);
   if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -322,6 +367,7 @@ int mmf_batch_set_state(mmf_batch *b, int32_t ci, const double *U) {
   if (!b || !U || ci < 0 || ci >= b->ncases) return MMF_ERR_INVALID;
   const BatchCase &c = b->hcases[(size_t)ci];
   const int64_t N = c.g.N, fs = c.g.fs;
+  b->lam_valid = false;
   // the rows cross as they are; the planes are formed on the device, through
   // the residual's buffer (dead between steps)
   BCHK(b, hipStreamSynchronize(b->stream));
@@ -363,6 +409,7 @@ int mmf_batch_set_initial_states(mmf_batch *b, const mmf_problem *problems) {
 
 int mmf_batch_set_time(mmf_batch *b, const double *t0, const double *tmax, const double *cfl) {
   if (!b || !t0 || !tmax || !cfl) return MMF_ERR_INVALID;
+  b->lam_valid = false;
   for (int i = 0; i < b->ncases; ++i) {
     if (!(cfl[i] > 0.0)) return bfail(b, MMF_ERR_INVALID, "cfl must be positive");
     Ctrl &c = b->hctrl[i];
@@ -415,7 +462,8 @@ int mmf_batch_get_shape(const mmf_batch *b, int32_t *chunk, int32_t *blocks) {
 
 int mmf_batch_advance(mmf_batch *b, int64_t nsteps) {
   if (!b || nsteps < 0) return MMF_ERR_INVALID;
-  int rc = ensure_graph(b);
+  int rc = ensure_lam(b);
+  if (rc == MMF_OK) rc = ensure_graph(b);
   if (rc != MMF_OK) return rc;
   for (int64_t s = 0; s < nsteps; ++s) {
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -548,13 +596,15 @@ int mmf_batch_autotune(mmf_batch *b, int32_t steps_per_trial, int32_t *best_chun
   int bc = keep_chunk, bb = keep_blocks, bt = keep_tail;
   double best = 1e300;
   int rc = MMF_OK;
-  for (int trial = 0; trial < 2 * 5 * 4 && rc == MMF_OK; ++trial) {
-    const int ch = chunks[trial / 8], pc = per_cu[trial % 4];
-    const int tl = ((trial / 4) % 2) ? std::max(4, ch / 4) : 0;  // no tail, or items of a quarter
-    if (tl >= ch) continue;
+  // bricks have one shape: only its time is taken
+  for (int trial = 0; trial < (b->bricks ? 1 : 2 * 5 * 4) && rc == MMF_OK; ++trial) {
+    const int ch = b->bricks ? keep_chunk : chunks[trial / 8];
+    const int nb = b->bricks ? keep_blocks : per_cu[trial % 4] * b->num_cus;
+    const int tl = b->bricks ? keep_tail : ((trial / 4) % 2) ? std::max(4, ch / 4) : 0;  // no tail, or items of a quarter
+    if (tl >= ch && !b->bricks) continue;
     {
       rc = mmf_batch_set_tail(b, tl);
-      if (rc == MMF_OK) rc = mmf_batch_set_shape(b, ch, pc * b->num_cus);
+      if (rc == MMF_OK) rc = mmf_batch_set_shape(b, ch, nb);
       if (rc == MMF_OK) rc = mmf_batch_enable_timing(b, 1);
       if (rc == MMF_OK) rc = mmf_batch_advance(b, 1);  // warm-up (and graph build)
       if (rc == MMF_OK) rc = mmf_batch_enable_timing(b, 1);
@@ -565,10 +615,11 @@ int mmf_batch_autotune(mmf_batch *b, int32_t steps_per_trial, int32_t *best_chun
       if (rc == MMF_OK && n > 0 && ms / n < best) {
         best = ms / n;
         bc = ch;
-        bb = pc * b->num_cus;
+        bb = nb;
         bt = tl;
       }
       // restore the state for the next trial
+      b->lam_valid = false;
       if (hipMemcpyAsync(b->dU, snapU, bytes, hipMemcpyDeviceToDevice, b->stream) != hipSuccess ||
           hipMemcpyAsync(b->dctrl, snapC.data(), sizeof(Ctrl) * snapC.size(), hipMemcpyHostToDevice, b->stream) !=
               hipSuccess ||

@@ -37,6 +37,13 @@ hipError_t launch_batch_stage(int stage, const BatchCase *cases, const int *item
                               unsigned int *counters, double *U, double *R, double *W, int nblocks, hipStream_t s);
 // Resident blocks per CU of the stage's batch kernel (0 if unknown).
 int batch_stage_occupancy(int stage);
+// Bricks of 16 x 16 cells, a block each (mmf_brick.hip): bricks of grid g, a
+// stage of every case, every case's early maximum.
+int64_t batch_bricks(const GridDev &g);
+hipError_t launch_batch_bricks(int stage, const BatchCase *cases, const int *bricks, int nbricks, double *U, double *R,
+                               double *W, hipStream_t s);
+hipError_t launch_batch_lam(const BatchCase *cases, int ncases, const int *bricks, int nbricks, const double *U,
+                            hipStream_t s);
 hipError_t launch_batch_advance(const BatchCase *cases, int ncases, unsigned int *counters, hipStream_t s);
 
 }  // namespace mmf

@@ -23,6 +23,7 @@
 #include <hip/hip_runtime.h>
 
 #include "mmf_device.hpp"
+#include "mmf_batch.hpp"
 #include "mmf_internal.hpp"
 #include "mmf_stage.hpp"
 
@@ -56,12 +57,13 @@ __device__ __forceinline__ void get_tup(const double *lds, int slot, Tup &t) {
 
 }  // namespace
 
-// MASK: the grid has cell flags (every fluid cell solved).  P2: A and V are
+// One brick's stage: brick (bx, by, bz) of grid g, block blk of the nblk that
+// advance the grid.  MASK: the grid has cell flags (every fluid cell solved).  P2: A and V are
 // powers of two (the faces hand over unscaled sums, scaled once at the update;
 // the same doubles).
 template <int DIM, int BX, int BY, int BZ, int STAGE, bool MASK, bool P2>
-__global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X, const double *U, double *out,
-                                                      Ctrl *ctrl, int mode, int nbx, int nby) {
+__device__ __forceinline__ void brick_stage(const GridDev &g, const double *X, const double *U, double *out, Ctrl *ctrl,
+                                            int mode, int bx, int by, int bz, unsigned int blk, unsigned int nblk) {
   constexpr int NT = BX * BY * BZ;
   constexpr int HX = BY * BZ, HY = BX * BZ, HZ = (DIM == 3) ? BX * BY : 0;
   constexpr int XM = NT, XP = XM + HX, YM = XP + HX, YP = YM + HY, ZM = YP + HY, ZP = ZM + HZ;
@@ -76,9 +78,6 @@ __global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X
 
   const int tid = threadIdx.x;
   const bool step = mode == MODE_STEP;
-  const int tile = xcd_range((int)blockIdx.x, (int)gridDim.x);
-  const int bz = (DIM == 3) ? tile / (nbx * nby) : 0;
-  const int by = (tile / nbx) % nby, bx = tile % nbx;
   const int nx = (int)g.n[0], ny = (int)g.n[1], nz = (DIM == 3) ? (int)g.n[2] : 1;
   const int x0 = bx * BX, y0 = by * BY, z0 = bz * BZ;
   const int w = (nx - x0 < BX) ? nx - x0 : BX;
@@ -332,10 +331,81 @@ __global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X
       m = (red[i] > m) ? red[i] : m;
       n = (red[NW + i] > n) ? red[NW + i] : n;
     }
-    stage_max_put(ctrl, step ? STAGE - 1 : 3, m);
-    if (STAGE == 3) lam_put(ctrl, n);
+    stage_max_put(ctrl, step ? STAGE - 1 : 3, m, blk);
+    if (STAGE == 3) lam_put(ctrl, n, blk);
   }
-  if (STAGE == 3 && step) close_step<true>(ctrl, tid);
+  if (STAGE == 3 && step) close_step<true>(ctrl, tid, blk, nblk);
+}
+
+template <int DIM, int BX, int BY, int BZ, int STAGE, bool MASK, bool P2>
+__global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X, const double *U, double *out,
+                                                      Ctrl *ctrl, int mode, int nbx, int nby) {
+  const int tile = xcd_range((int)blockIdx.x, (int)gridDim.x);
+  const int bz = (DIM == 3) ? tile / (nbx * nby) : 0;
+  brick_stage<DIM, BX, BY, BZ, STAGE, MASK, P2>(g, X, U, out, ctrl, mode, tile % nbx, (tile / nbx) % nby, bz, blockIdx.x,
+                                                gridDim.x);
+}
+
+// ---- batches: one block per brick of every case --------------------------------
+// bricks[2 i], [2 i + 1]: case and brick number of block i, in case order, the
+// blocks of an XCD a contiguous run of them.
+constexpr int BATCH_BX = 16, BATCH_BY = 16;
+
+template <int STAGE>
+__global__ __launch_bounds__(BATCH_BX *BATCH_BY) void k_brick_batch(const BatchCase *cases, const int *bricks, double *U,
+                                                                    double *R, double *W) {
+  const int i = xcd_range((int)blockIdx.x, (int)gridDim.x);
+  const BatchCase &bc = cases[__builtin_amdgcn_readfirstlane(bricks[2 * i])];
+  const int b = __builtin_amdgcn_readfirstlane(bricks[2 * i + 1]);
+  const GridDev &g = bc.g;
+  const int nbx = ((int)g.n[0] + BATCH_BX - 1) / BATCH_BX, nby = ((int)g.n[1] + BATCH_BY - 1) / BATCH_BY;
+  double *Ub = U + bc.offset, *Rb = R + bc.offset, *Wb = W + bc.offset;
+  const double *X = (STAGE == 1) ? Ub : (STAGE == 2) ? Rb : Wb;
+  double *out = (STAGE == 1) ? Rb : (STAGE == 2) ? Wb : Ub;
+  brick_stage<2, BATCH_BX, BATCH_BY, 1, STAGE, false, false>(g, X, Ub, out, bc.ctrl, MODE_STEP, b % nbx, b / nbx, 0,
+                                                             (unsigned)b, (unsigned)(nbx * nby));
+}
+
+__global__ __launch_bounds__(256) void k_batch_lam_zero(const BatchCase *cases, int ncases) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < ncases) cases[i].ctrl->lam_now = 0ull;
+}
+
+// Every case's Ctrl::lam_now from its state.
+__global__ __launch_bounds__(BATCH_BX *BATCH_BY) void k_batch_lam(const BatchCase *cases, const int *bricks,
+                                                                  const double *U) {
+  const int i = xcd_range((int)blockIdx.x, (int)gridDim.x);
+  const BatchCase &bc = cases[__builtin_amdgcn_readfirstlane(bricks[2 * i])];
+  const int b = __builtin_amdgcn_readfirstlane(bricks[2 * i + 1]);
+  const int nbx = ((int)bc.g.n[0] + BATCH_BX - 1) / BATCH_BX;
+  const int64_t x = (int64_t)(b % nbx) * BATCH_BX + threadIdx.x % BATCH_BX;
+  const int64_t y = (int64_t)(b / nbx) * BATCH_BY + threadIdx.x / BATCH_BX;
+  double l = 0.0;
+  if (x < bc.g.n[0] && y < bc.g.n[1]) l = grid_cell_lam(bc.g, U + bc.offset, x + bc.g.n[0] * y);
+  const unsigned long long m = wave_max_u64(dbits(l));
+  if ((threadIdx.x & 63) == 0 && m) atomicMax(&bc.ctrl->lam_now, m);
+}
+
+int64_t batch_bricks(const GridDev &g) {
+  return ((g.n[0] + BATCH_BX - 1) / BATCH_BX) * ((g.n[1] + BATCH_BY - 1) / BATCH_BY);
+}
+
+hipError_t launch_batch_bricks(int stage, const BatchCase *cases, const int *bricks, int nbricks, double *U, double *R,
+                               double *W, hipStream_t s) {
+  const dim3 grid((unsigned)nbricks), block(BATCH_BX * BATCH_BY);
+  switch (stage) {
+    case 1: hipLaunchKernelGGL(k_brick_batch<1>, grid, block, 0, s, cases, bricks, U, R, W); break;
+    case 2: hipLaunchKernelGGL(k_brick_batch<2>, grid, block, 0, s, cases, bricks, U, R, W); break;
+    default: hipLaunchKernelGGL(k_brick_batch<3>, grid, block, 0, s, cases, bricks, U, R, W);
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_batch_lam(const BatchCase *cases, int ncases, const int *bricks, int nbricks, const double *U,
+                            hipStream_t s) {
+  hipLaunchKernelGGL(k_batch_lam_zero, dim3((unsigned)((ncases + 255) / 256)), dim3(256), 0, s, cases, ncases);
+  hipLaunchKernelGGL(k_batch_lam, dim3((unsigned)nbricks), dim3(BATCH_BX * BATCH_BY), 0, s, cases, bricks, U);
+  return hipGetLastError();
 }
 
 template <int DIM, int BX, int BY, int BZ, bool MASK, bool P2>

@@ -84,8 +84,11 @@ __device__ __forceinline__ double stage_max(const Ctrl *c, int s) {
 }
 
 // This block's contribution (bits of a non-negative double) to stage maximum s.
+__device__ __forceinline__ void stage_max_put(Ctrl *c, int s, unsigned long long bits, unsigned int blk) {
+  if (bits) atomicMax(&c->eig[s][blk % EIG_SPLIT][0], bits);
+}
 __device__ __forceinline__ void stage_max_put(Ctrl *c, int s, unsigned long long bits) {
-  if (bits) atomicMax(&c->eig[s][block_linear() % EIG_SPLIT][0], bits);
+  stage_max_put(c, s, bits, block_linear());
 }
 
 // dt rule of main.cpp:398-402, evaluated identically by every thread.
@@ -106,9 +109,10 @@ __device__ __forceinline__ double step_dt_early(const Ctrl *c) {
 
 // This block's contribution (bits of a non-negative double) to the next
 // step's early maximum.
-__device__ __forceinline__ void lam_put(Ctrl *c, unsigned long long bits) {
-  if (bits) atomicMax(&c->lam[block_linear() % EIG_SPLIT][0], bits);
+__device__ __forceinline__ void lam_put(Ctrl *c, unsigned long long bits, unsigned int blk) {
+  if (bits) atomicMax(&c->lam[blk % EIG_SPLIT][0], bits);
 }
+__device__ __forceinline__ void lam_put(Ctrl *c, unsigned long long bits) { lam_put(c, bits, block_linear()); }
 
 // Batched cases keep their stage maxima on line 0 of their control block
 // alone (a case's blocks are few, so one line does not serialise them).
@@ -166,11 +170,12 @@ __device__ __forceinline__ void advance_ctrl_wave(Ctrl *c, int lane) {
 // a line counts the line, and the block completing the last line reads every
 // block's maximum with its own atomics.  Only atomics carry the hand-over,
 // so no L2 write-back fence is needed.
-template <bool EARLY = false>
-__device__ __forceinline__ void close_step(Ctrl *ctrl, int tid) {
+// blk of nb: this block's number among those that advance the control block.
+template <bool EARLY>
+__device__ __forceinline__ void close_step(Ctrl *ctrl, int tid, unsigned int blk, unsigned int nb) {
   __shared__ int last;
   if (tid == 0) {
-    const unsigned int nb = gridDim.x * gridDim.y * gridDim.z, k = block_linear() % EIG_SPLIT;
+    const unsigned int k = blk % EIG_SPLIT;
     const unsigned long long nk = (nb - k + EIG_SPLIT - 1) / EIG_SPLIT;  // blocks on line k
     const unsigned long long nl = (nb < (unsigned)EIG_SPLIT) ? nb : EIG_SPLIT;  // lines in use
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -185,6 +190,11 @@ __device__ __forceinline__ void close_step(Ctrl *ctrl, int tid) {
     advance_ctrl_wave<EARLY>(ctrl, tid);
     if (tid <= EIG_SPLIT) atomicExch(&ctrl->done[tid][0], 0ull);
   }
+}
+
+template <bool EARLY = false>
+__device__ __forceinline__ void close_step(Ctrl *ctrl, int tid) {
+  close_step<EARLY>(ctrl, tid, block_linear(), gridDim.x * gridDim.y * gridDim.z);
 }
 
 // Stage input state of one cell: U (stage 1), W1 = U + dt R / V rebuilt on the
@@ -364,6 +374,51 @@ struct NegCount {
     }
   }
 };
+
+// Cell i's part of the early maximum of state U: what the stage-1 faces of a
+// step starting from U give on a grid whose unsolved cells are all solid
+// (every face with a solved side takes the larger of its two sides' |u_a| + c,
+// euler.cpp:232-234): for a solved cell, every axis (it has faces along each);
+// along an axis with a wall face (a non-fluid neighbour) or a reflecting /
+// wall border, the reflected virtual state's (euler.cpp:318-356); at a
+// Dirichlet border, the border state's (euler.cpp:366-376).
+__device__ __forceinline__ double grid_cell_lam(const GridDev &g, const double *U, int64_t i) {
+  double m = 0.0;
+  if (g.flags && !(g.flags[i] & CELL_SOLVED)) return m;
+  double c[NF];
+#pragma unroll
+  for (int k = 0; k < NF; ++k) c[k] = U[k * g.fs + i];
+  Tup T;
+  make_tup(c, T);
+  const int64_t q[3] = {i % g.n[0], (i / g.n[0]) % g.n[1], i / (g.n[0] * g.n[1])};
+  for (int a = 0; a < g.dim; ++a) {
+    m = lam_acc(m, fabs(T.vel[a]) + T.a);
+    bool refl = false;
+    for (int d = 0; d < 2; ++d) {
+      const int side = 2 * a + d;
+      int64_t nb;
+      if (neighbour(g, q, a, d ? 1 : -1, nb)) {
+        refl = refl || (g.flags && !(g.flags[nb] & CELL_FLUID));
+      } else if (g.bc[side] == BC_REFLECTING || g.bc[side] == BC_WALL) {
+        refl = true;
+      } else if (g.bc[side] == BC_DIRICHLET) {
+        double v[NF];
+        Tup V;
+        prim2cons(g.info[side], v);
+        make_tup(v, V);
+        m = lam_acc(m, fabs(V.vel[a]) + V.a);
+      }
+    }
+    if (refl) {
+      double v[NF];
+      Tup V;
+      reflect_axis(c, a, v);
+      make_tup(v, V);
+      m = lam_acc(m, fabs(V.vel[a]) + V.a);
+    }
+  }
+  return m;
+}
 
 // RK stage update of one field (main.cpp:421,457,493).
 template <int STAGE>

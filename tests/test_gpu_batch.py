@@ -116,6 +116,31 @@ def test_batch_shape_independent(mmf, chunk, blocks, tail):
         assert np.array_equal(b.get_state(i), ref.get_state(i)), (chunk, blocks, i)
 
 
+def test_strips_equal_bricks(mmf):
+    """The strips of large batches (2^23 cells and more: here by an idle case,
+    already at its end time) against the bricks of small ones, for several
+    strip shapes."""
+    cs, states = setup(mmf)
+    ref = make_batch(mmf, cs, states)
+    ref.advance(STEPS)
+    idle = mmf.grid_desc(2, [2900, 2897], [-1.0, -1.0, 0.0], 1e-3, [4] * 4 + [0, 0])
+    for chunk, blocks, tail in ((0, 0, 0), (1, 5, 0), (16, 500, 4), (64, 64, 5), (1000, 300, 0)):
+        b = mmf.Batch([c[0] for c in cs] + [idle])
+        assert b.total_cells >= 1 << 23
+        if chunk:
+            b.set_shape(chunk, blocks)
+        b.set_tail(tail)
+        for i, U in enumerate(states):
+            b.set_state(i, U)
+        b.set_time(0.0, [c[3] for c in cs] + [0.0], [c[2] for c in cs] + [0.5])
+        b.advance(STEPS)
+        t, steps = b.times()
+        assert np.array_equal(t[:-1], ref.times()[0]) and np.array_equal(steps[:-1], ref.times()[1])
+        for i in range(len(cs)):
+            assert np.array_equal(b.get_state(i), ref.get_state(i)), (chunk, blocks, tail, i)
+        b.close()
+
+
 def test_batch_graph_replays_with_eager_work_between(mmf):
     """Each replay of the captured step matches a fresh batch advanced the same
     number of steps, with host reads and state uploads between the replays."""
