@@ -227,6 +227,19 @@ __device__ __forceinline__ bool make_tup_quot(const double *c, Tup &t) {
   return ok & ((e < ew ? e : ew) >= QUOT_MIN_EXP) & quot_divisor(rho) & finite_bits(t.H);
 }
 
+// cons2prim's pressure (utils.cpp:48-63), the same way.
+__device__ __forceinline__ double pressure_fast(const double *c) {
+  double T, a;
+  const bool ok = temperature_quot(c, quot_rcp(c[FID_RHO]), T, a);
+  double p = c[FID_RHO] * T;
+  if (__builtin_expect(!(ok & quot_divisor(c[FID_RHO]) & finite_bits(p)), 0)) {
+    double prim[NF];
+    cons2prim(c, prim);
+    p = prim[FID_P];
+  }
+  return p;
+}
+
 // make_tup, the division sequences only where the quotients do not apply.
 __device__ __forceinline__ void make_tup_fast(const double *c, Tup &t) {
   if (__builtin_expect(!make_tup_quot(c, t), 0)) make_tup(c, t);

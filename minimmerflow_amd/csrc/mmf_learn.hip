@@ -641,9 +641,24 @@ __device__ __forceinline__ void load_region(const GridDev &g, int xo, int yo, co
     rex[ry][rx] = ex;
     const int64_t i = gx + (int64_t)nx * gy;
     double v[NF];
+    if (STAGE == 2) {
+      double x[NF], q[NF];
+#pragma unroll
+      for (int k = 0; k < NF; ++k) {
+        v[k] = U[k * fs + i];
+        x[k] = dt * R[k * fs + i];
+      }
+      if (g.pow2V) div_vol5<true>(g, x, q);
+      else div_vol5<false>(g, x, q);
+#pragma unroll
+      for (int k = 0; k < NF; ++k) v[k] = v[k] + q[k];
+    } else {
+#pragma unroll
+      for (int k = 0; k < NF; ++k) v[k] = Xin[k * fs + i];
+    }
 #pragma unroll
     for (int k = 0; k < NF; ++k) {
-      v[k] = !ex ? 0.0 : (STAGE == 2) ? U[k * fs + i] + div_vol(g, dt * R[k * fs + i]) : Xin[k * fs + i];
+      v[k] = ex ? v[k] : 0.0;
       reg[k][ry][rx] = v[k];
     }
     // p = (gamma - 1) (rho E - |rho u|^2 / (2 rho)) for the shock sensor
@@ -719,7 +734,7 @@ __device__ __forceinline__ bool cell_face(const GridDev &g, const LearnRun &run,
     const int a = grp >> 1, side = grp & 1;
     const int my = ry - a, mx = rx - (1 - a), py = ry + a, px = rx + (1 - a);
     const bool em = rex[my][mx], ep = rex[py][px];
-    double X0[NF], pr[NF];
+    double X0[NF];
 #pragma unroll
     for (int k = 0; k < NF; ++k) {
       X0[k] = reg[k][ry][rx];
@@ -728,8 +743,7 @@ __device__ __forceinline__ bool cell_face(const GridDev &g, const LearnRun &run,
       const double sl = minmod(dp, dm);
       P[k] = side ? X0[k] + 0.5 * sl : X0[k] - 0.5 * sl;
     }
-    cons2prim(P, pr);
-    if (!(P[FID_RHO] > 0.0) || !(pr[FID_P] > 0.0)) {
+    if (!(P[FID_RHO] > 0.0) || !(pressure_fast(P) > 0.0)) {
 #pragma unroll
       for (int k = 0; k < NF; ++k) P[k] = X0[k];
     }
@@ -887,8 +901,8 @@ __device__ __forceinline__ double fs_face(const GridDev &g, const double *FS, co
     cr[k] = upper ? oth[k] : own[k];
   }
   Tup TL, TR;
-  make_tup(cl, TL);
-  make_tup(cr, TR);
+  make_tup_fast(cl, TL);
+  make_tup_fast(cr, TR);
   double F[NF];
   const double lam = face_flux(TL, TR, A, F);
   // each face counted once: a cell's lower face only at a border
@@ -978,8 +992,8 @@ __device__ __forceinline__ double face_of_states(const GridDev &g, const double 
     }
   }
   Tup TL, TR;
-  make_tup(cl, TL);
-  make_tup(cr, TR);
+  make_tup_fast(cl, TL);
+  make_tup_fast(cr, TR);
   double F[NF];
   const double lam = face_flux(TL, TR, A, F);
   if (count) count_neg(TL, TR, ctrl);
