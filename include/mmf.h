@@ -89,10 +89,11 @@ enum { MMF_KERNEL_AUTO = 0, MMF_KERNEL_GATHER = 1, MMF_KERNEL_MARCH = 2, MMF_KER
  * 2D order-2 grids without bodies (each face once, the step's time advance
  * in its last stage; also the learned reconstruction's kernel).  AUTO: TILE
  * for 2D order-2 grids without bodies; MARCH where it applies from 2^18 cells
- * (2D order 1, strips that need no reflected state) or 2^20 cells (3D); else
- * GATHER, which AUTO runs as LDS bricks (a thread per cell, every flux tuple
- * once per brick) where they apply: 3D order 2 without bodies at any size,
- * order 1 where every fluid cell is solved, border conditions per side.  mmf_set_kernel refuses MARCH or TILE on a grid they do not
+ * (2D order 1) or 2^20 cells (3D); else GATHER, which AUTO runs as LDS bricks
+ * (a thread per cell, every flux tuple once per brick) where they apply: 3D
+ * order 2 without bodies at any size, order 1 where every fluid cell is solved
+ * and border conditions are per side, in 2D instead of MARCH below 2^24 cells,
+ * in 3D from 2^20 cells only where MARCH's 64 x 8 tiles would be partly empty.  mmf_set_kernel refuses MARCH or TILE on a grid they do not
  * apply to; bodies set afterwards make them fall back to GATHER.  tile_rows (3D: 4 or 8) and chunk (planes per block along the last axis)
  * shape the marching kernel; <= 0 keeps the default (3D order 1, 64 x 8
  * tiles: where the chunks would leave a partial round of blocks, the planes

@@ -56,8 +56,8 @@ bool valid_bc(int b) { return b >= MMF_BC_FREE_FLOW && b <= MMF_BC_PERIODIC; }
 // 2D order 1 from 2^18 cells (64^2 56 vs 28 us per step, 512^2 equal, 1024^2
 // 137 vs 188), 3D order 1 from 2^20 (32^3 273 vs 37 us, 96^3 319 vs 193,
 // 128^3 271 vs 379), 3D order 2 (with bodies) from 2^20.  Order-1 grids without
-// ghost cells or per-face conditions go to the brick kernel below
-// brick_auto_max, order-2 grids without bodies to the tile kind and the bricks.
+// ghost cells or per-face conditions go to the brick kernel where prefer_bricks
+// says so, order-2 grids without bodies to the tile kind and the bricks.
 bool use_march(const mmf_ctx *ctx) {
   if (ctx->kernel == mmf::KERNEL_GATHER || !mmf::march_shape_supported(ctx->g, ctx->shape)) return false;
   if (ctx->kernel == mmf::KERNEL_AUTO) {
@@ -85,19 +85,27 @@ bool o2_bricks(const GridDev &g) {
   return mmf::brick_o2_supported(g) && (g.dim == 3 || g.N > TILE_SIX_WAVES_MAX_N);
 }
 
-// AUTO takes the brick kernel for order-1 grids below this size (us per step,
-// gather / best marching shape / brick; MI355X).  3D: 32^3 37 / 36 / 23, 64^3
-// 65 / 57 / 48, 100 x 90 x 84 173 / 163 / 108, 168 x 133 x 32 156 / 104 / 98,
-// but 128^3 385 / 155 / 225: the marching kernel builds fewer halo tuples.
-// 2D: 64^2 29 / 76 / 19, 500 x 400 55 / 57 / 31.  Strips without a reflecting
-// x border or a body march without branches and issue fewer instructions per
-// cell: with several grids in flight 1000 x 600 takes 43 us per step against
-// 46 (alone 79 against 60), so they keep their sizes; the others (1448^2,
-// reflecting, 316 / 167; 1024^2 with a cylinder 168 / 107) go to the bricks.
-int64_t brick_auto_max(const GridDev &g) {
-  if (g.dim == 3) return (int64_t)1 << 20;
-  const bool flat_strips = !g.flags && (g.periodic[0] || (g.bc[0] == MMF_BC_FREE_FLOW && g.bc[1] == MMF_BC_FREE_FLOW));
-  return (int64_t)1 << (flat_strips ? 18 : 22);
+// AUTO's choice between the brick and the marching kernel for order 1 (us per
+// step alone / with three grids in flight, marching against brick; MI355X).
+// 2D: bricks; 400 x 300 50 / 25 and 21 / 17, 1000 x 600 70 / 42 and 53 / 39,
+// 1200 x 1000 periodic 115 / 86 and 84 / 91, 1500 x 1400 reflecting 333 / 167
+// and 141 / 179, 2048^2 443 / 319 and 353 / 322.
+// 3D below 2^20 cells: bricks; 64^3 57 (best shape) and 44, 96^3 115 / 97 and
+// 97 / 88, 100 x 90 x 84 163 (best shape) and 96.  From there three states no
+// longer fit the last-level cache and a brick's halo costs more than a
+// marching tile's: 128^3 138 / 152 and 190 / 256, reflecting 258 / 224 and 198 /
+// 259; but the marching tiles cover 64 x 8 columns, so grids that leave them
+// partly empty go to the bricks (40 x 40 x 900 202 / 188 and 144 / 164): where
+// the padded cells exceed 1.3 times the grid's, or 1.86 times without
+// reflected states, whose full tiles march the cheaper flat pass.
+bool prefer_bricks(const GridDev &g) {
+  if (g.dim == 2) return g.N < ((int64_t)1 << 24);
+  if (g.N < ((int64_t)1 << 20)) return true;
+  bool refl = g.flags != nullptr;
+  for (int s = 0; s < 6; ++s)
+    refl = refl || (!g.periodic[s / 2] && (g.bc[s] == MMF_BC_REFLECTING || g.bc[s] == MMF_BC_WALL));
+  const int64_t padded = (g.n[0] + 63) / 64 * 64 * ((g.n[1] + 7) / 8 * 8) * g.n[2];
+  return padded * (refl ? 10 : 7) > g.N * 13;
 }
 
 // The stage kernel of the next launches.  With the learned reconstruction on:
@@ -107,7 +115,7 @@ int kernel_used(const mmf_ctx *ctx) {
   if (ctx->kernel == mmf::KERNEL_TILE) return tile_applies(ctx) ? mmf::KERNEL_TILE : mmf::KERNEL_GATHER;
   if (ctx->kernel == mmf::KERNEL_AUTO && tile_applies(ctx)) return mmf::KERNEL_TILE;
   if (ctx->kernel == mmf::KERNEL_AUTO && ctx->g.dim == 3 && mmf::brick_o2_supported(ctx->g)) return mmf::KERNEL_BRICK;
-  if (ctx->kernel == mmf::KERNEL_AUTO && ctx->g.N < brick_auto_max(ctx->g) && mmf::brick_supported(ctx->g))
+  if (ctx->kernel == mmf::KERNEL_AUTO && mmf::brick_supported(ctx->g) && prefer_bricks(ctx->g))
     return mmf::KERNEL_BRICK;
   return use_march(ctx) ? mmf::KERNEL_MARCH : mmf::KERNEL_GATHER;
 }
