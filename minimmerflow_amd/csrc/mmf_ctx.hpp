@@ -48,10 +48,10 @@ struct mmf_ctx {
   bool learn_on = false;
   mmf::LearnRun learn{};
   bool learn_opts_set = false;
-  // captured step graphs (1 step, GRAPH_STEPS steps) and the launch
-  // configuration they were captured with
-  hipGraph_t step_graph[2] = {nullptr, nullptr};
-  hipGraphExec_t step_exec[2] = {nullptr, nullptr};
+  // the captured graph of GRAPH_STEPS steps and the launch configuration it
+  // was captured with
+  hipGraph_t step_graph = nullptr;
+  hipGraphExec_t step_exec = nullptr;
   std::vector<char> graph_key;
   bool use_graphs = true;
   // Ctrl::lam_now holds the early maximum of the current state (the 3D

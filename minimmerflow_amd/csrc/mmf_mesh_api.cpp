@@ -43,8 +43,8 @@ struct mmf_mesh {
   std::vector<std::pair<hipEvent_t, hipEvent_t>> events;
   double stage_ms = 0.0;
   int64_t stages = 0;
-  hipGraph_t graph[2] = {nullptr, nullptr};
-  hipGraphExec_t exec[2] = {nullptr, nullptr};
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec = nullptr;
   bool use_graphs = true;
   bool lam_valid = false;  // Ctrl::lam_now holds the current state's maximum
 };
@@ -63,12 +63,10 @@ int mfail(mmf_mesh *m, int code, const std::string &msg) {
   } while (0)
 
 void drop_graphs(mmf_mesh *m) {
-  for (int i = 0; i < 2; ++i) {
-    if (m->exec[i]) (void)hipGraphExecDestroy(m->exec[i]);
-    if (m->graph[i]) (void)hipGraphDestroy(m->graph[i]);
-    m->exec[i] = nullptr;
-    m->graph[i] = nullptr;
-  }
+  if (m->exec) (void)hipGraphExecDestroy(m->exec);
+  if (m->graph) (void)hipGraphDestroy(m->graph);
+  m->exec = nullptr;
+  m->graph = nullptr;
 }
 
 int read_ctrl(mmf_mesh *m) {
@@ -153,7 +151,7 @@ int ensure_lam(mmf_mesh *m) {
 
 constexpr int GRAPH_STEPS = 16;
 
-int capture(mmf_mesh *m, int slot, int64_t n) {
+int capture(mmf_mesh *m, int64_t n) {
   MCHK(m, hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
   int rc = enqueue_steps(m, n);
   hipGraph_t g = nullptr;
@@ -163,8 +161,8 @@ int capture(mmf_mesh *m, int slot, int64_t n) {
     return rc;
   }
   if (e != hipSuccess) return mfail(m, MMF_ERR_HIP, std::string("end of step capture: ") + hipGetErrorString(e));
-  m->graph[slot] = g;
-  MCHK(m, hipGraphInstantiate(&m->exec[slot], g, nullptr, nullptr, 0));
+  m->graph = g;
+  MCHK(m, hipGraphInstantiate(&m->exec, g, nullptr, nullptr, 0));
   return MMF_OK;
 }
 
@@ -477,19 +475,19 @@ int mmf_mesh_advance(mmf_mesh *m, int64_t nsteps) {
   const int rc0 = ensure_lam(m);
   if (rc0 != MMF_OK) return rc0;
   if (m->timing || !m->use_graphs || nsteps == 0) return enqueue_steps(m, nsteps);
-  while (nsteps > 0) {
-    const int slot = (nsteps >= GRAPH_STEPS) ? 1 : 0;
-    if (!m->exec[slot]) {
-      int rc = capture(m, slot, slot ? GRAPH_STEPS : 1);
+  // whole graphs, then the remainder by launches (three a step: less host time
+  // than a graph of one step, and no capture on a first short call)
+  for (; nsteps >= GRAPH_STEPS; nsteps -= GRAPH_STEPS) {
+    if (!m->exec) {
+      int rc = capture(m, GRAPH_STEPS);
       if (rc != MMF_OK) {
         drop_graphs(m);
         return rc;
       }
     }
-    MCHK(m, hipGraphLaunch(m->exec[slot], m->stream));
-    nsteps -= slot ? GRAPH_STEPS : 1;
+    MCHK(m, hipGraphLaunch(m->exec, m->stream));
   }
-  return MMF_OK;
+  return enqueue_steps(m, nsteps);
 }
 
 int mmf_mesh_set_step_graphs(mmf_mesh *m, int32_t on) {
