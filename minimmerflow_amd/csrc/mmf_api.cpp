@@ -935,6 +935,14 @@ int ensure_lam(mmf_ctx *ctx) {
 }
 
 int enqueue_steps(mmf_ctx *ctx, int64_t nsteps) {
+  // small 2D grids: a launch per step, by pairs (the state returns to its
+  // buffer); the launches that are timed each stay one stage's
+  if (ctx->timing != 1 && kernel_used(ctx) == mmf::KERNEL_BRICK && mmf::step_brick_supported(ctx->g))
+    for (; nsteps >= 2; nsteps -= 2) {
+      hipError_t e = mmf::launch_step_brick(ctx->g, ctx->dU, ctx->dW, ctx->dctrl, ctx->stream);
+      if (e == hipSuccess) e = mmf::launch_step_brick(ctx->g, ctx->dW, ctx->dU, ctx->dctrl, ctx->stream);
+      if (e != hipSuccess) return hip_fail(ctx, e, "step kernel launch");
+    }
   for (int64_t s = 0; s < nsteps; ++s) {
     for (int stage = 1; stage <= 3; ++stage) {
       int rc = launch_stage_timed(ctx, stage, mmf::MODE_STEP);

@@ -22,6 +22,8 @@
 // the gather kernel's and the oracle's bit for bit.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "mmf_device.hpp"
 #include "mmf_batch.hpp"
 #include "mmf_internal.hpp"
@@ -344,6 +346,228 @@ __global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X
   const int bz = (DIM == 3) ? tile / (nbx * nby) : 0;
   brick_stage<DIM, BX, BY, BZ, STAGE, MASK, P2>(g, X, U, out, ctrl, mode, tile % nbx, (tile / nbx) % nby, bz, blockIdx.x,
                                                 gridDim.x);
+}
+
+// ---- one launch per step: small 2D grids without a body ------------------------
+// A block advances O x O cells (O = R - 6) by a whole step: it loads the R x R
+// cells around them, one per thread, and forms W1, W2 and the new state on
+// regions that shrink by a ring per stage, so that only dt crosses blocks, and
+// that is known before the step.  A slot one cell outside a border that is not
+// periodic holds the virtual state of its inner cell: its thread rebuilds it
+// at every stage from the inner cell's state.  A block repeats its neighbours'
+// rings (2.0 tuples and 1.5 cell updates per cell and stage), which costs
+// less than the launches, the loads and the stores of two more stages do while
+// the grid does not fill the chip.  The new state goes to another buffer: the
+// neighbours still read the old one.
+// 16 x 16 regions: us per step of one grid alone / of three on three streams,
+// three launches a step and this one:
+//   64 x 64 periodic     16.3 / 8.0    11.5 / 5.7
+//   64 x 64 reflecting   17.5 / 8.3    15.3 / 6.8
+//   128 x 128 inflow     16.7 / 7.8    12.0 / 6.0
+//   256 x 200 inflow     18.7 / 9.0    15.9 / 8.3
+//   255 x 256 reflecting 21.1 / 10.1   18.4 / 10.4
+//   300 x 300 inflow     22.3 / 11.1   21.9 / 12.9
+// so up to 2^16 cells, where a chip of blocks is about full.  What is left is
+// one launch's latency and the step's close, and where a flow front leaves
+// momenta below 2^-900 the division sequences of its blocks.
+template <int R, bool P2>
+__global__ __launch_bounds__(R *R) void k_brick_step(GridDev g, const double *X, double *out, Ctrl *ctrl, int nbx) {
+  constexpr int NT = R * R, O = R - 6, NW = NT / 64;
+  __shared__ double lds[2][NTUP * NT];
+  __shared__ unsigned int sneg[3][NW];
+  __shared__ unsigned long long red[3][NW];
+
+  const int tid = threadIdx.x, lx = tid % R, ly = tid / R;
+  const int tile = xcd_range((int)blockIdx.x, (int)gridDim.x);
+  const int x0 = (tile % nbx) * O, y0 = (tile / nbx) * O;
+  const int n[2] = {(int)g.n[0], (int)g.n[1]};
+  auto owned = [&](int x, int y) {  // unwrapped
+    return x >= x0 && x < x0 + O && x < n[0] && y >= y0 && y < y0 + O && y < n[1];
+  };
+  int q[2] = {x0 - 3 + lx, y0 - 3 + ly};
+  const bool own = owned(q[0], q[1]);
+  // the slot's cell, or the inner cell of the virtual state it holds
+  int side = -1, inner = tid;
+  bool alive = true, own_inner = false;
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    if (g.periodic[a]) continue;
+    if (q[a] < -1 || q[a] > n[a]) alive = false;
+    else if (q[a] < 0 || q[a] == n[a]) {
+      if (side >= 0) alive = false;  // outside two borders
+      const int in = (q[a] < 0) ? 1 : -1;
+      side = 2 * a + (in < 0);
+      q[a] += in;
+      inner = tid + in * (a ? R : 1);
+    }
+  }
+  if (side >= 0 && alive) own_inner = owned(q[0], q[1]);
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    if (!g.periodic[a]) continue;
+    while (q[a] < 0) q[a] += n[a];
+    while (q[a] >= n[a]) q[a] -= n[a];
+  }
+  const uint32_t idx = alive ? (uint32_t)q[0] + (uint32_t)n[0] * (uint32_t)q[1] : (uint32_t)x0 + (uint32_t)n[0] * (uint32_t)y0;
+  const int64_t fs = g.fs;
+  double U[NF], S[NF];
+#pragma unroll
+  for (int k = 0; k < NF; ++k) S[k] = U[k] = X[k * fs + idx];
+  const bool run = ctrl->t < ctrl->tmax;  // main.cpp:377 loop guard
+  if (!run) {                             // uniform; the state stays, in the buffer that is then the current one
+    if (own) {
+#pragma unroll
+      for (int k = 0; k < NF; ++k) out[k * fs + idx] = U[k];
+    }
+    return;
+  }
+  const double dt = step_dt_early(ctrl);
+  const bool borders = (!g.periodic[0] && (x0 <= 3 || x0 + O + 3 > n[0])) || (!g.periodic[1] && (y0 <= 3 || y0 + O + 3 > n[1]));
+
+  NegCount neg;
+  unsigned int anyneg = 0;
+  double lam[3] = {0.0, 0.0, 0.0};  // maxima of stages 2 and 3, and of the new state
+
+  auto stage = [&](auto STAGE_) {
+    constexpr int STAGE = decltype(STAGE_)::value;
+    double *buf = lds[(STAGE - 1) & 1], *nxt = lds[STAGE & 1];
+    Tup T;
+    bool neg_here = false;
+    if (alive && lx >= STAGE - 1 && lx <= R - STAGE && ly >= STAGE - 1 && ly <= R - STAGE) {
+      if (side >= 0) {
+        double v[NF];
+        if (STAGE > 1) {
+#pragma unroll
+          for (int k = 0; k < NF; ++k) S[k] = buf[k * NT + inner];
+        }
+        border_state(g, side, side >> 1, S, v);  // euler.cpp:261-376
+#pragma unroll
+        for (int k = 0; k < NF; ++k) S[k] = v[k];
+      }
+      // one tuple for both kinds of slots: a wave holds some of each
+      make_tup_fast(S, T);
+      double ls = 0.0;
+      if (own) ls = lam_acc(fabs(T.vel[0]), fabs(T.vel[1])) + T.a;
+      if (own_inner) ls = fabs((side & 2) ? T.vel[1] : T.vel[0]) + T.a;
+      if (STAGE > 1) lam[STAGE - 2] = ls;
+      neg_here = tup_negative(T);
+      put_tup<NT>(buf, tid, T);
+    }
+    const unsigned long long nb = __ballot(neg_here);
+    if ((tid & 63) == 0) sneg[STAGE - 1][tid >> 6] = nb != 0;
+    __syncthreads();
+    unsigned int an = 0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) an |= sneg[STAGE - 1][i];
+    anyneg |= an;
+
+    if (alive && side < 0 && lx >= STAGE && lx < R - STAGE && ly >= STAGE && ly < R - STAGE) {
+      const int off[2] = {1, R};
+      const double halfA = P2 ? 1.0 : g.halfA;
+      double rhs[NF] = {0., 0., 0., 0., 0.};  // euler.cpp:142-148
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        double Fm[NF], Fp[NF];
+        Tup N;
+        get_tup<NT>(buf, tid - off[a], N);
+        face_flux_area(N, T, a, P2, g.A, halfA, Fm);
+        get_tup<NT>(buf, tid + off[a], N);
+        face_flux_area(T, N, a, P2, g.A, halfA, Fp);
+        if (g.periodic[a] && q[a] == n[a] - 1) {
+          // the wrap face is first in the reference-order face list
+#pragma unroll
+          for (int k = 0; k < NF; ++k) { rhs[k] -= Fp[k]; rhs[k] += Fm[k]; }
+        } else {
+#pragma unroll
+          for (int k = 0; k < NF; ++k) { rhs[k] += Fm[k]; rhs[k] -= Fp[k]; }
+        }
+      }
+      if (an && own) {
+        // once per face: every upper face, and the lower ones on a border
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          Tup N;
+          if (!g.periodic[a] && q[a] == 0) {
+            get_tup<NT>(buf, tid - off[a], N);
+            neg.add(N, T);
+          }
+          get_tup<NT>(buf, tid + off[a], N);
+          neg.add(T, N);
+        }
+      }
+      double x[NF], dq[NF];
+#pragma unroll
+      for (int k = 0; k < NF; ++k) x[k] = dt * (P2 ? g.halfA * rhs[k] : rhs[k]);
+      div_vol5<P2>(g, x, dq);
+#pragma unroll
+      for (int k = 0; k < NF; ++k) S[k] = rk_update_q<STAGE>(U[k], T.c[k], dq[k]);
+      if (STAGE < 3 && borders) {  // for the virtual states of the next stage
+#pragma unroll
+        for (int k = 0; k < NF; ++k) nxt[k * NT + tid] = S[k];
+      }
+      if (STAGE == 3 && own) {
+#pragma unroll
+        for (int k = 0; k < NF; ++k) out[k * fs + idx] = S[k];
+        // the next step's stage-1 maximum: this cell's, and the virtual states
+        // its border faces will have
+        double l = cell_max_eig<2>(S);
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          bool refl = false;
+#pragma unroll
+          for (int s = 0; s < 2; ++s) {
+            if (g.periodic[a] || q[a] != (s ? n[a] - 1 : 0)) continue;
+            const int bc = g.bc[2 * a + s], slot = s ? tid + off[a] : tid - off[a];
+            refl = refl || bc == BC_REFLECTING || bc == BC_WALL;
+            if (bc == BC_DIRICHLET) l = lam_acc(l, fabs(buf[(5 + a) * NT + slot]) + buf[9 * NT + slot]);
+          }
+          if (refl) {
+            double v[NF];
+            Tup V;
+            reflect_axis(S, a, v);
+            make_tup_fast(v, V);
+            l = lam_acc(l, fabs(V.vel[a]) + V.a);
+          }
+        }
+        lam[2] = l;
+      }
+    }
+    if (STAGE < 3 && borders) __syncthreads();
+  };
+  stage(std::integral_constant<int, 1>{});
+  stage(std::integral_constant<int, 2>{});
+  stage(std::integral_constant<int, 3>{});
+
+  if (anyneg) neg.flush(ctrl, tid);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const unsigned long long m = wave_max_u64(dbits(lam[i]));
+    if ((tid & 63) == 0) red[i][tid >> 6] = m;
+  }
+  __syncthreads();
+  if (tid < 3) {
+    unsigned long long m = red[tid][0];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) m = (red[tid][i] > m) ? red[tid][i] : m;
+    if (tid < 2) stage_max_put(ctrl, tid + 1, m, blockIdx.x);
+    else lam_put(ctrl, m, blockIdx.x);
+  }
+  close_step<true>(ctrl, tid, blockIdx.x, gridDim.x);
+}
+
+constexpr int STEP_R = 16;
+
+hipError_t launch_step_brick(const GridDev &g, const double *in, double *out, Ctrl *ctrl, hipStream_t s) {
+  constexpr int O = STEP_R - 6;
+  const int nbx = (int)((g.n[0] + O - 1) / O), nby = (int)((g.n[1] + O - 1) / O);
+  const dim3 grid((unsigned)nbx * nby), block(STEP_R * STEP_R);
+  if (g.pow2A && g.pow2V) hipLaunchKernelGGL((k_brick_step<STEP_R, true>), grid, block, 0, s, g, in, out, ctrl, nbx);
+  else hipLaunchKernelGGL((k_brick_step<STEP_R, false>), grid, block, 0, s, g, in, out, ctrl, nbx);
+  return hipGetLastError();
+}
+
+bool step_brick_supported(const GridDev &g) {
+  return brick_supported(g) && g.dim == 2 && g.flags == nullptr && g.N < STEP_BRICK_MAX_CELLS;
 }
 
 // ---- batches: one block per brick of every case --------------------------------

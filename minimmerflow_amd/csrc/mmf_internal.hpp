@@ -152,6 +152,12 @@ bool brick_supported(const GridDev &g);
 hipError_t launch_stage_brick(const GridDev &g, int stage, int mode, const double *U, const double *R, const double *W,
                               double *oR, double *oW, double *oU, Ctrl *ctrl, hipStream_t s);
 
+// A whole step per launch (mmf_brick.hip): 2D bricks without a body, from one
+// buffer to another; dt is Ctrl::lam_now's, as for the brick kernel.
+constexpr int64_t STEP_BRICK_MAX_CELLS = (int64_t)1 << 16;
+bool step_brick_supported(const GridDev &g);
+hipError_t launch_step_brick(const GridDev &g, const double *in, double *out, Ctrl *ctrl, hipStream_t s);
+
 // Order-2 brick kernel (mmf_brick_o2.hip): without bodies or per-face
 // conditions, 32-bit cell indices.
 bool brick_o2_supported(const GridDev &g);

@@ -98,6 +98,60 @@ def check(mmf, name, dim, n, bc, body, negative, order):
         assert a[4] == b[4], "positivity counts"
 
 
+STEP_CASES = [
+    ("one cell", (1, 1), [3, 0, 1, 2]),
+    ("two cells per axis, periodic", (2, 2), [4] * 4),
+    ("wraps several times", (2, 3), [4, 4, 4, 4]),
+    ("one tile", (10, 10), [1, 3, 2, 0]),
+    ("one past a tile", (11, 21), [4, 4, 3, 1]),
+    ("borders in the last ring", (12, 13), [0, 1, 3, 2]),
+    ("one row", (129, 1), [0, 2, 1, 3]),
+    ("largest, ragged", (257, 255), [3, 0, 1, 2]),
+    ("periodic", (64, 50), [4] * 4),
+]
+
+
+@pytest.mark.parametrize("name,n,bc", STEP_CASES, ids=[c[0] for c in STEP_CASES])
+@pytest.mark.parametrize("negative", [False, True])
+def test_steps_in_one_launch_equal_gather(mmf, name, n, bc, negative):
+    """Pairs of steps, each one launch on a small 2D grid, and a final time
+    reached by the first step of a pair (the other one then only moves the
+    state back)."""
+    info = np.tile([1.0, 0.3, -0.1, 0.0, 1.0], (6, 1))
+    s, U = build(mmf, 2, list(n), bc, info, None, order=1, seed=len(name))
+    if negative:
+        k = np.random.default_rng(3).integers(0, len(U), max(1, len(U) // 50))
+        U = U.copy()
+        U[k, 0] *= -1.0
+        U[k, 4] *= -1.0
+    s.set_kernel(mmf.KERNEL_GATHER)
+    s.set_state(U)
+    s.set_time(0.0, 10.0, 0.5)
+    s.advance(1)
+    try:
+        ends = [10.0] if negative else [10.0, 2.5 * s.time()[1]]
+    except mmf.MMFError:
+        ends = [10.0]
+    for end in ends:
+        out = []
+        for kind in (mmf.KERNEL_GATHER, mmf.KERNEL_AUTO):
+            s.set_kernel(kind)
+            s.set_state(U)
+            s.set_time(0.0, end, 0.5)
+            s.reset_positivity_counters()
+            s.advance(2 if negative else 4)
+            try:
+                t, dt, step, stages = s.time()
+                time = (t, dt, step, tuple(stages))
+            except mmf.MMFError:
+                time = s.nonfinite_steps()
+            out.append((s.get_state(), time, s.positivity_counters()))
+        a, b = out
+        assert np.array_equal(a[0], b[0], equal_nan=True), "state"
+        assert a[1] == b[1], "time control and stage maxima"
+        assert a[2] == b[2], "positivity counts"
+
+
 def test_brick_steps_against_the_oracle(mmf, orc):
     """64^2 and 20 x 18 x 12, reflecting and Dirichlet sides, orders 1 and 2, four steps each."""
     for dim, n, bc, order in ((2, [64, 64], [1, 1, 1, 1, 0, 0], 1), (3, [20, 18, 12], [3, 0, 1, 2, 0, 1], 1),
