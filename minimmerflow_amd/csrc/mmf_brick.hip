@@ -362,14 +362,14 @@ __global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X
 // 16 x 16 regions: us per step of one grid alone / of three on three streams,
 // three launches a step and this one:
 //   64 x 64 periodic     16.3 / 8.0    11.5 / 5.7
-//   64 x 64 reflecting   17.5 / 8.3    15.3 / 6.8
+//   64 x 64 reflecting   17.5 / 8.3    14.6 / 6.1 (15.3 / 6.4 with division
+//                        sequences in the reflected states)
 //   128 x 128 inflow     16.7 / 7.8    12.0 / 6.0
 //   256 x 200 inflow     18.7 / 9.0    15.9 / 8.3
 //   255 x 256 reflecting 21.1 / 10.1   18.4 / 10.4
 //   300 x 300 inflow     22.3 / 11.1   21.9 / 12.9
 // so up to 2^16 cells, where a chip of blocks is about full.  What is left is
-// one launch's latency and the step's close, and where a flow front leaves
-// momenta below 2^-900 the division sequences of its blocks.
+// one launch's latency, the chain of three stages and the step's close.
 template <int R, bool P2>
 __global__ __launch_bounds__(R *R) void k_brick_step(GridDev g, const double *X, double *out, Ctrl *ctrl, int nbx) {
   constexpr int NT = R * R, O = R - 6, NW = NT / 64;
@@ -440,7 +440,9 @@ __global__ __launch_bounds__(R *R) void k_brick_step(GridDev g, const double *X,
 #pragma unroll
           for (int k = 0; k < NF; ++k) S[k] = buf[k * NT + inner];
         }
-        border_state(g, side, side >> 1, S, v);  // euler.cpp:261-376
+        const int bc = g.bc[side];  // euler.cpp:261-376
+        if (bc == BC_REFLECTING || bc == BC_WALL) reflect_axis_quot(S, side >> 1, v);
+        else border_state(g, side, side >> 1, S, v);
 #pragma unroll
         for (int k = 0; k < NF; ++k) S[k] = v[k];
       }
@@ -524,7 +526,7 @@ __global__ __launch_bounds__(R *R) void k_brick_step(GridDev g, const double *X,
           if (refl) {
             double v[NF];
             Tup V;
-            reflect_axis(S, a, v);
+            reflect_axis_quot(S, a, v);
             make_tup_fast(v, V);
             l = lam_acc(l, fabs(V.vel[a]) + V.a);
           }
