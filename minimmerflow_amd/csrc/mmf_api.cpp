@@ -885,11 +885,22 @@ int ensure_tiles(mmf_ctx *ctx) {
   if (ctx->tiles_valid && ctx->g.march_tiles) return MMF_OK;
   // the segment table (3 * MARCH_SEGS entries per block) or the tile table
   // (one); a share that needs more segments than a block has: the chunks
-  const uint8_t *fl = ctx->hflags.empty() ? nullptr : ctx->hflags.data();
+  std::vector<uint8_t> ring;
+  if (ctx->g.flags && !ctx->hflags.empty()) {
+    ring.resize((size_t)mmf::march_tile_planes(ctx->g, ctx->shape));
+    uint8_t *d = nullptr;
+    HIPCHK(ctx, hipMalloc(&d, ring.size()));
+    hipError_t e = mmf::launch_tile_planes(ctx->g, ctx->shape, d, ctx->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(ring.data(), d, ring.size(), hipMemcpyDeviceToHost, ctx->stream);
+    const hipError_t es = hipStreamSynchronize(ctx->stream);
+    (void)hipFree(d);
+    if (e != hipSuccess || es != hipSuccess) return hip_fail(ctx, e != hipSuccess ? e : es, "tile planes");
+  }
+  const uint8_t *rg = ring.empty() ? nullptr : ring.data();
   std::vector<int32_t> t;
   if (segs) {
     t.resize((size_t)(ctx->shape.seg_blocks * 3 * mmf::MARCH_SEGS));
-    if (!mmf::build_march_segments(ctx->g, ctx->shape, fl, t.data())) {
+    if (!mmf::build_march_segments(ctx->g, ctx->shape, rg, t.data())) {
       ctx->shape.seg_blocks = 0;
       if (ctx->g.flags == nullptr || ctx->hflags.empty()) {
         ctx->g.march_tiles = nullptr;
@@ -900,7 +911,7 @@ int ensure_tiles(mmf_ctx *ctx) {
   }
   if (t.empty()) {
     t.resize((size_t)mmf::march_blocks(ctx->g, ctx->shape));
-    mmf::build_march_tiles(ctx->g, ctx->shape, fl, t.data());
+    mmf::build_march_tiles(ctx->g, ctx->shape, rg, t.data());
   }
   const int64_t nb = (int64_t)t.size();
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));

@@ -58,8 +58,8 @@ struct mmf_ctx {
   // marching kernel keeps it up to date from step to step; anything else
   // that changes the state, the time control or the kernel clears this)
   bool lam_valid = false;
-  // cell flags (cell order) kept on the host for the 3D marching kernel's
-  // tile table (empty when every cell is fluid and solved), and the table
+  // cell flags (cell order) on the host, empty when every cell is fluid and
+  // solved; the 3D marching kernel's tile table
   std::vector<uint8_t> hflags;
   int32_t *dtiles = nullptr;
   int64_t dtiles_n = 0;

@@ -174,16 +174,21 @@ bool march_shape_supported(const GridDev &g, const MarchShape &shape);
 // 3D order 2: the LDS-staged marching kernel (64 x 8 tiles), bodies included.
 hipError_t launch_stage_march3d_o2(const GridDev &g, int chunk, int stage, int mode, const double *U, const double *R,
                                    const double *W, double *oR, double *oW, double *oU, Ctrl *ctrl, hipStream_t s);
-// Tile table of the 3D marching kernel for cell flags 'flags' (cell order):
-// masked tiles first, the rest in the XCD-aware order.
-void build_march_tiles(const GridDev &g, const MarchShape &shape, const uint8_t *flags, int32_t *tiles);
+// Per tile plane of the 3D marching kernel (z fastest): whether the tile or the
+// ring around it holds a flag there; device array of march_tile_planes bytes.
+int64_t march_tile_planes(const GridDev &g, const MarchShape &shape);
+hipError_t launch_tile_planes(const GridDev &g, const MarchShape &shape, uint8_t *ring, hipStream_t s);
+// Tile table of the 3D marching kernel from those: masked tiles first, the
+// rest in the XCD-aware order.
+void build_march_tiles(const GridDev &g, const MarchShape &shape, const uint8_t *ring, int32_t *tiles);
 // The segment table of shape.seg_blocks blocks (3 * MARCH_SEGS entries
 // each): the tile planes split into shares of equal cost (a plane that needs
 // the masked code costs more), XCD-aware, each share cut into runs of one
 // tile and one code; per block its runs as (tile | MARCH_TILE_MASKED, first
-// plane, end plane), -1 after the last.  flags (cell order) or nullptr.
+// plane, end plane), -1 after the last.  ring: the tile planes with flags, or
+// nullptr for none.
 // False when a share would need more than MARCH_SEGS runs of different tiles.
-bool build_march_segments(const GridDev &g, const MarchShape &shape, const uint8_t *flags, int32_t *table);
+bool build_march_segments(const GridDev &g, const MarchShape &shape, const uint8_t *ring, int32_t *table);
 // Sets shape.seg_blocks where the chunks leave a partial round of blocks on
 // num_cus CUs and every share stays within a few tiles.
 void balance_march_shape(const GridDev &g, int num_cus, MarchShape &shape);

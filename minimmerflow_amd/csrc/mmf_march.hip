@@ -867,41 +867,57 @@ int64_t march_blocks(const GridDev &g, const MarchShape &sh) {
   return ntx * nty * ((g.n[2] + sh.chunk - 1) / sh.chunk);
 }
 
-void build_march_tiles(const GridDev &g, const MarchShape &sh, const uint8_t *flags, int32_t *tiles) {
-  const int64_t nx = g.n[0], ny = g.n[1], nz = g.n[2];
-  const int TX = sh.tx;
-  const int64_t ntx = (nx + TX - 1) / TX, nty = (ny + sh.ty - 1) / sh.ty;
+// ring[t * nz + z]: whether tile t's cells of plane z and the ring around them
+// hold a flag (wrapped across periodic sides).  One wave per tile plane: the
+// host read every flag for this one byte at a time, 6 ms of the first step of
+// a 192^3 grid with a body and as much after every change of one.
+__global__ __launch_bounds__(64) void k_tile_planes(GridDev g, int TX, int TY, int ntx, uint8_t *ring) {
+  const int nx = (int)g.n[0], ny = (int)g.n[1], nz = (int)g.n[2];
+  const int t = (int)(blockIdx.x / (unsigned)nz), z = (int)(blockIdx.x % (unsigned)nz);
+  const int x0 = (t % ntx) * TX, y0 = (t / ntx) * TY;
+  const int w = min(TX, nx - x0) + 2, h = min(TY, ny - y0) + 2;
+  bool m = false;
+  for (int p = threadIdx.x; p < w * h; p += 64) {
+    int x = x0 - 1 + p % w, y = y0 - 1 + p / w;
+    if (((x < 0 || x >= nx) && !g.periodic[0]) || ((y < 0 || y >= ny) && !g.periodic[1])) continue;
+    x = (x + nx) % nx;
+    y = (y + ny) % ny;
+    m = m || g.flags[(int64_t)x + (int64_t)nx * ((int64_t)y + (int64_t)ny * z)] != (CELL_FLUID | CELL_SOLVED);
+  }
+  const bool any = __ballot(m) != 0;
+  if (threadIdx.x == 0) ring[blockIdx.x] = any;
+}
+
+int64_t march_tile_planes(const GridDev &g, const MarchShape &sh) {
+  return ((g.n[0] + sh.tx - 1) / sh.tx) * ((g.n[1] + sh.ty - 1) / sh.ty) * g.n[2];
+}
+
+hipError_t launch_tile_planes(const GridDev &g, const MarchShape &sh, uint8_t *ring, hipStream_t s) {
+  const int ntx = (int)((g.n[0] + sh.tx - 1) / sh.tx);
+  hipLaunchKernelGGL(k_tile_planes, dim3((unsigned)march_tile_planes(g, sh)), dim3(64), 0, s, g, sh.tx, sh.ty, ntx, ring);
+  return hipGetLastError();
+}
+
+// Planes z0 .. z1 of a tile's ring flags, wrapped across a periodic z.
+static bool ring_any(const GridDev &g, const uint8_t *ring, int64_t z0, int64_t z1) {
+  const int64_t nz = g.n[2];
+  for (int64_t z = z0; z <= z1; ++z) {
+    if ((z < 0 || z >= nz) && !g.periodic[2]) continue;
+    if (ring[(z + nz) % nz]) return true;
+  }
+  return false;
+}
+
+void build_march_tiles(const GridDev &g, const MarchShape &sh, const uint8_t *ring, int32_t *tiles) {
+  const int64_t nz = g.n[2];
+  const int64_t ntiles = ((g.n[0] + sh.tx - 1) / sh.tx) * ((g.n[1] + sh.ty - 1) / sh.ty);
   const int nblk = (int)march_blocks(g, sh);
-  const uint8_t all = CELL_FLUID | CELL_SOLVED;
   // the cells a block reads: its tile and halo ring over its chunk and the
-  // planes below and above it, wrapped across periodic sides
-  auto wrap = [](int64_t i, int64_t n, bool per, int64_t &out) {
-    if (i >= 0 && i < n) { out = i; return true; }
-    if (!per) return false;
-    out = (i + n) % n;
-    return true;
-  };
+  // planes below and above it
   std::vector<uint8_t> masked((size_t)nblk, 0);
   for (int t = 0; t < nblk; ++t) {
-    const int64_t bx = t % ntx, by = (t / ntx) % nty, bz = t / (ntx * nty);
-    const int64_t x0 = bx * TX, y0 = by * sh.ty, m0 = bz * sh.chunk;
-    const int64_t x1 = std::min(x0 + TX, nx), y1 = std::min(y0 + sh.ty, ny), m1 = std::min(m0 + sh.chunk, nz);
-    bool m = false;
-    for (int64_t z = m0 - 1; z <= m1 && !m; ++z) {
-      int64_t zz;
-      if (!wrap(z, nz, g.periodic[2], zz)) continue;
-      for (int64_t y = y0 - 1; y <= y1 && !m; ++y) {
-        int64_t yy;
-        if (!wrap(y, ny, g.periodic[1], yy)) continue;
-        const uint8_t *row = flags + (yy + ny * zz) * nx;
-        for (int64_t x = x0 - 1; x <= x1; ++x) {
-          int64_t xx;
-          if (!wrap(x, nx, g.periodic[0], xx)) continue;
-          if (row[xx] != all) { m = true; break; }
-        }
-      }
-    }
-    masked[(size_t)t] = m;
+    const int64_t m0 = t / ntiles * sh.chunk, m1 = std::min(m0 + sh.chunk, nz);
+    masked[(size_t)t] = ring_any(g, ring + t % ntiles * nz, m0 - 1, m1);
   }
   // masked tiles on the first blocks of their XCD (the blocks b with the same
   // b % 8): they start in the first round and take longer, so their CUs are
@@ -920,62 +936,22 @@ void build_march_tiles(const GridDev &g, const MarchShape &sh, const uint8_t *fl
   }
 }
 
-// Per plane m of tile (bx, by): the tile's cells and halo ring in planes m -
-// 1, m and m + 1 (wrapped across periodic sides) are not all fluid and solved,
-// i.e. marching plane m needs the masked code.
-static void plane_masks(const GridDev &g, int TX, int TY, int64_t bx, int64_t by, const uint8_t *flags,
-                        std::vector<uint8_t> &pm) {
-  const int64_t nx = g.n[0], ny = g.n[1], nz = g.n[2];
-  pm.assign((size_t)nz, 0);
-  if (!flags) return;
-  const uint8_t all = CELL_FLUID | CELL_SOLVED;
-  auto wrap = [](int64_t i, int64_t n, bool per, int64_t &out) {
-    if (i >= 0 && i < n) { out = i; return true; }
-    if (!per) return false;
-    out = (i + n) % n;
-    return true;
-  };
-  const int64_t x0 = bx * TX, y0 = by * TY;
-  const int64_t x1 = std::min(x0 + TX, nx), y1 = std::min(y0 + TY, ny);
-  std::vector<uint8_t> ring((size_t)nz, 0);  // plane z's tile and ring
-  for (int64_t z = 0; z < nz; ++z) {
-    bool m = false;
-    for (int64_t y = y0 - 1; y <= y1 && !m; ++y) {
-      int64_t yy;
-      if (!wrap(y, ny, g.periodic[1], yy)) continue;
-      const uint8_t *row = flags + (yy + ny * z) * nx;
-      for (int64_t x = x0 - 1; x <= x1; ++x) {
-        int64_t xx;
-        if (!wrap(x, nx, g.periodic[0], xx)) continue;
-        if (row[xx] != all) { m = true; break; }
-      }
-    }
-    ring[(size_t)z] = m;
-  }
-  for (int64_t m = 0; m < nz; ++m)
-    for (int64_t z = m - 1; z <= m + 1; ++z) {
-      int64_t zz;
-      if (wrap(z, nz, g.periodic[2], zz) && ring[(size_t)zz]) pm[(size_t)m] = 1;
-    }
-}
-
 // Cost of a plane marched by the unmasked and by the masked code (flags,
 // body faces), in quarters of the former: on a 192^3 grid with a sphere the
 // stage time is lowest with masked planes at 2.5 to 3.5 times an unmasked one.
 constexpr int64_t PLANE_COST = 4, PLANE_COST_MASKED = 10;
 
-bool build_march_segments(const GridDev &g, const MarchShape &sh, const uint8_t *flags, int32_t *table) {
+bool build_march_segments(const GridDev &g, const MarchShape &sh, const uint8_t *ring, int32_t *table) {
   const int64_t nm = g.n[2];
   const int64_t ntx = (g.n[0] + sh.tx - 1) / sh.tx, nty = (g.n[1] + sh.ty - 1) / sh.ty;
   const int64_t W = ntx * nty * nm;  // tile planes, tile by tile
   const int B = sh.seg_blocks;
-  // masked planes and the cost prefix over the tile planes
-  std::vector<uint8_t> masked((size_t)W), pm;
+  // masked planes (a flag in the tile's ring over planes m - 1 .. m + 1) and
+  // the cost prefix over the tile planes
+  std::vector<uint8_t> masked((size_t)W, 0);
   std::vector<int64_t> pre((size_t)W + 1, 0);
-  for (int64_t t = 0; t < ntx * nty; ++t) {
-    plane_masks(g, sh.tx, sh.ty, t % ntx, t / ntx, flags, pm);
-    for (int64_t m = 0; m < nm; ++m) masked[(size_t)(t * nm + m)] = pm[(size_t)m];
-  }
+  if (ring)
+    for (int64_t i = 0; i < W; ++i) masked[(size_t)i] = ring_any(g, ring + i / nm * nm, i % nm - 1, i % nm + 1);
   for (int64_t i = 0; i < W; ++i) pre[(size_t)i + 1] = pre[(size_t)i] + (masked[(size_t)i] ? PLANE_COST_MASKED : PLANE_COST);
   const int64_t total = pre[(size_t)W];
   // first tile plane of block share L: the first whose cost prefix reaches L / B of the total
