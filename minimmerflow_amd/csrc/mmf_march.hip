@@ -937,9 +937,10 @@ void build_march_tiles(const GridDev &g, const MarchShape &sh, const uint8_t *ri
 }
 
 // Cost of a plane marched by the unmasked and by the masked code (flags,
-// body faces), in quarters of the former: on a 192^3 grid with a sphere the
-// stage time is lowest with masked planes at 2.5 to 3.5 times an unmasked one.
-constexpr int64_t PLANE_COST = 4, PLANE_COST_MASKED = 10;
+// body faces), in quarters of the former: priced at 2, 2.5, 3, 3.5 and 4 times
+// an unmasked one, a step of a 192^3 grid with a sphere takes 739, 668, 645,
+// 646 and 661 us, of a 224^3 one 1275, 1102, 1062, 1080 and 1090.
+constexpr int64_t PLANE_COST = 4, PLANE_COST_MASKED = 12;
 
 bool build_march_segments(const GridDev &g, const MarchShape &sh, const uint8_t *ring, int32_t *table) {
   const int64_t nm = g.n[2];
