@@ -191,7 +191,11 @@ int mmf_rk_update(mmf_ctx *ctx, int32_t stage, double dt);
 int mmf_pack_cells(mmf_ctx *ctx, int32_t state, const int64_t *cells, int64_t n, double *buf);
 int mmf_unpack_cells(mmf_ctx *ctx, int32_t state, const int64_t *cells, int64_t n, const double *buf);
 /* Device SoA view of a state (field k at ptr + k * field_stride, cell order),
- * for exchanges that stay on the device. */
+ * for exchanges that stay on the device: it may be read and written between
+ * calls, once the context's work is done (mmf_synchronize).  After STATE_U was
+ * handed out, mmf_advance and mmf_run take the eigenvalue maximum of the state
+ * they find instead of keeping the last call's (one pass over the state a
+ * call). */
 int mmf_get_device_state(mmf_ctx *ctx, int32_t state, double **ptr, int64_t *field_stride);
 
 /* ---- the same RHS, allocating nothing -------------------------------------- */

@@ -842,6 +842,7 @@ int mmf_get_device_state(mmf_ctx *ctx, int32_t state, double **ptr, int64_t *fie
   if (!ctx || !ptr || !state_ptr(ctx, state)) return MMF_ERR_INVALID;
   *ptr = state_ptr(ctx, state);
   if (field_stride) *field_stride = ctx->g.fs;
+  if (state == MMF_STATE_U) ctx->u_shared = true;
   return MMF_OK;
 }
 
@@ -938,7 +939,6 @@ int ensure_lam(mmf_ctx *ctx) {
     return MMF_OK;
   }
   if (ctx->lam_valid) return MMF_OK;
-  HIPCHK(ctx, hipMemsetAsync(&ctx->dctrl->lam_now, 0, sizeof(unsigned long long), ctx->stream));
   hipError_t e = mmf::launch_lam_init(ctx->g, ctx->dU, ctx->dctrl, ctx->stream);
   if (e != hipSuccess) return hip_fail(ctx, e, "early dt");
   ctx->lam_valid = true;
@@ -1043,8 +1043,7 @@ int replay_steps(mmf_ctx *ctx, int64_t nsteps) {
 
 // Steps are replayed from graphs, or launched one by one with per-launch
 // kernel timing on; region timing brackets the whole call with one event pair.
-int mmf_advance(mmf_ctx *ctx, int64_t nsteps) {
-  if (!ctx || nsteps < 0) return MMF_ERR_INVALID;
+static int advance_steps(mmf_ctx *ctx, int64_t nsteps) {
   int rct = ensure_tiles(ctx);
   if (rct != MMF_OK) return rct;
   int rc0 = ensure_lam(ctx);
@@ -1065,6 +1064,18 @@ int mmf_advance(mmf_ctx *ctx, int64_t nsteps) {
   return rc;
 }
 
+// The caller may have written the state through its device view since the last
+// call: its maximum is taken again.
+static void shared_state_changed(mmf_ctx *ctx) {
+  if (ctx->u_shared) ctx->lam_valid = false;
+}
+
+int mmf_advance(mmf_ctx *ctx, int64_t nsteps) {
+  if (!ctx || nsteps < 0) return MMF_ERR_INVALID;
+  shared_state_changed(ctx);
+  return advance_steps(ctx, nsteps);
+}
+
 int mmf_set_step_graphs(mmf_ctx *ctx, int32_t on) {
   if (!ctx) return MMF_ERR_INVALID;
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
@@ -1075,6 +1086,7 @@ int mmf_set_step_graphs(mmf_ctx *ctx, int32_t on) {
 
 int mmf_run(mmf_ctx *ctx, int64_t max_steps, int64_t *steps_done, double *t_final) {
   if (!ctx) return MMF_ERR_INVALID;
+  shared_state_changed(ctx);
   int rc = read_ctrl(ctx);
   if (rc != MMF_OK) return rc;
   const int64_t step0 = ctx->hctrl->step;
@@ -1090,7 +1102,7 @@ int mmf_run(mmf_ctx *ctx, int64_t max_steps, int64_t *steps_done, double *t_fina
       batch = (int64_t)std::min(std::max(rem, 1.0), 256.0);
     }
     if (max_steps >= 0) batch = std::min(batch, max_steps - done);
-    rc = mmf_advance(ctx, batch);
+    rc = advance_steps(ctx, batch);
     if (rc != MMF_OK) return rc;
     rc = read_ctrl(ctx);
     if (rc != MMF_OK) return rc;

@@ -607,7 +607,11 @@ __global__ __launch_bounds__(BATCH_BX *BATCH_BY) void k_batch_lam(const BatchCas
   const int64_t x = (int64_t)(b % nbx) * BATCH_BX + threadIdx.x % BATCH_BX;
   const int64_t y = (int64_t)(b / nbx) * BATCH_BY + threadIdx.x / BATCH_BX;
   double l = 0.0;
-  if (x < bc.g.n[0] && y < bc.g.n[1]) l = grid_cell_lam(bc.g, U + bc.offset, x + bc.g.n[0] * y);
+  if (x < bc.g.n[0] && y < bc.g.n[1]) {
+    uint32_t sides = 0;
+    l = grid_cell_lam<true>(bc.g, U + bc.offset, (uint32_t)(x + bc.g.n[0] * y), sides);
+    if (sides) l = lam_acc(l, dirichlet_lam(bc.g, sides));
+  }
   const unsigned long long m = wave_max_u64(dbits(l));
   if ((threadIdx.x & 63) == 0 && m) atomicMax(&bc.ctrl->lam_now, m);
 }

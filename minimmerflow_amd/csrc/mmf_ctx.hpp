@@ -54,10 +54,13 @@ struct mmf_ctx {
   hipGraphExec_t step_exec = nullptr;
   std::vector<char> graph_key;
   bool use_graphs = true;
-  // Ctrl::lam_now holds the early maximum of the current state (the 3D
-  // marching kernel keeps it up to date from step to step; anything else
-  // that changes the state, the time control or the kernel clears this)
+  // Ctrl::lam_now holds the early maximum of the current state (the steps of
+  // the brick and 3D marching kernels keep it up to date; anything else that
+  // changes the state, the time control or the kernel clears this)
   bool lam_valid = false;
+  // the state's device address was handed out: it may change between any two
+  // calls, so the maximum of one call's last state is not kept for the next
+  bool u_shared = false;
   // cell flags (cell order) on the host, empty when every cell is fluid and
   // solved; the 3D marching kernel's tile table
   std::vector<uint8_t> hflags;

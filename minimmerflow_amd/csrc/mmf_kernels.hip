@@ -201,22 +201,23 @@ __global__ __launch_bounds__(BLOCK) void k_stage(GridDev g, StageIn<STAGE> in, c
 // t += dt after stage 3 (main.cpp:505-506); resets the stage maxima.
 __global__ void k_advance(Ctrl *c) { advance_ctrl_wave(c, threadIdx.x); }
 
-// The early maximum of state U into Ctrl::lam_now, zero beforehand.
+// The early maximum of state U into Ctrl::lam_now.  VIRT: see grid_cell_lam.
+// Streams the state once, so HBM bounds it on large grids and its launch on
+// small ones; the first step after a new state, and every call once the
+// state's address was handed out, pays for it.  us added to a call, with
+// division sequences, 64-bit index divisions and the value cleared by a
+// launch of its own / as it is: 256^3 258 / 130 (5.2 TB/s), 192^3 with a
+// sphere 222 / 87, 1000 x 600 22 / 4, 64 x 64 12 / 8.
+template <bool VIRT>
 __global__ __launch_bounds__(256) void k_lam_init(GridDev g, const double *U, Ctrl *ctrl) {
   double m = 0.0;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < g.N; i += stride) {
-    m = lam_acc(m, grid_cell_lam(g, U, i));
-  }
-  __shared__ unsigned long long red[4];
-  const unsigned long long b = wave_max_u64(dbits(m));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = b;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long r = red[0];
-    for (int w = 1; w < 4; ++w) r = (red[w] > r) ? red[w] : r;
-    if (r) atomicMax(&ctrl->lam_now, r);
-  }
+  const uint32_t N = (uint32_t)g.N, stride = gridDim.x * 256u;
+  uint32_t sides = 0;
+  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < N; i += stride)
+    m = lam_acc(m, grid_cell_lam<VIRT>(g, U, i, sides));
+  if (VIRT && sides) m = lam_acc(m, dirichlet_lam(g, sides));
+  block_lam_to<256>(ctrl, m, threadIdx.x);
+  last_block(ctrl, threadIdx.x, blockIdx.x, gridDim.x, [&] { set_lam_wave(ctrl, threadIdx.x); });
 }
 
 __global__ void k_zero_slot(Ctrl *c, int slot) {
@@ -268,7 +269,10 @@ hipError_t launch_stage(const GridDev &g, int stage, int mode, const double *U, 
 hipError_t launch_lam_init(const GridDev &g, const double *U, Ctrl *ctrl, hipStream_t s) {
   const int64_t want = (g.N + 255) / 256;
   const unsigned nb = (unsigned)(want < 2048 ? (want > 0 ? want : 1) : 2048);
-  hipLaunchKernelGGL(k_lam_init, dim3(nb), dim3(256), 0, s, g, U, ctrl);
+  bool virt = g.flags != nullptr;
+  for (int side = 0; side < 2 * g.dim; ++side) virt = virt || (!g.periodic[side / 2] && g.bc[side] != BC_FREE_FLOW);
+  if (virt) hipLaunchKernelGGL((k_lam_init<true>), dim3(nb), dim3(256), 0, s, g, U, ctrl);
+  else hipLaunchKernelGGL((k_lam_init<false>), dim3(nb), dim3(256), 0, s, g, U, ctrl);
   return hipGetLastError();
 }
 

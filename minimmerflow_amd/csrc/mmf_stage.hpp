@@ -171,8 +171,8 @@ __device__ __forceinline__ void advance_ctrl_wave(Ctrl *c, int lane) {
 // block's maximum with its own atomics.  Only atomics carry the hand-over,
 // so no L2 write-back fence is needed.
 // blk of nb: this block's number among those that advance the control block.
-template <bool EARLY>
-__device__ __forceinline__ void close_step(Ctrl *ctrl, int tid, unsigned int blk, unsigned int nb) {
+template <typename Close>
+__device__ __forceinline__ void last_block(Ctrl *ctrl, int tid, unsigned int blk, unsigned int nb, Close close) {
   __shared__ int last;
   if (tid == 0) {
     const unsigned int k = blk % EIG_SPLIT;
@@ -187,9 +187,14 @@ __device__ __forceinline__ void close_step(Ctrl *ctrl, int tid, unsigned int blk
   }
   __syncthreads();
   if (last && tid < 64) {
-    advance_ctrl_wave<EARLY>(ctrl, tid);
+    close();
     if (tid <= EIG_SPLIT) atomicExch(&ctrl->done[tid][0], 0ull);
   }
+}
+
+template <bool EARLY>
+__device__ __forceinline__ void close_step(Ctrl *ctrl, int tid, unsigned int blk, unsigned int nb) {
+  last_block(ctrl, tid, blk, nb, [&] { advance_ctrl_wave<EARLY>(ctrl, tid); });
 }
 
 template <bool EARLY = false>
@@ -378,38 +383,53 @@ struct NegCount {
 // Cell i's part of the early maximum of state U: what the stage-1 faces of a
 // step starting from U give on a grid whose unsolved cells are all solid
 // (every face with a solved side takes the larger of its two sides' |u_a| + c,
-// euler.cpp:232-234): for a solved cell, every axis (it has faces along each);
-// along an axis with a wall face (a non-fluid neighbour) or a reflecting /
-// wall border, the reflected virtual state's (euler.cpp:318-356); at a
-// Dirichlet border, the border state's (euler.cpp:366-376).
-__device__ __forceinline__ double grid_cell_lam(const GridDev &g, const double *U, int64_t i) {
-  double m = 0.0;
-  if (g.flags && !(g.flags[i] & CELL_SOLVED)) return m;
+// euler.cpp:232-234): for a solved cell, every axis (it has faces along each).
+// VIRT: the grid has virtual states of their own speed: along an axis with a
+// wall face (a non-fluid neighbour) or a reflecting / wall border, the
+// reflected state's (euler.cpp:318-356); the Dirichlet sides that the cell
+// touches go into 'sides' (dirichlet_lam).  Fewer than 2^32 cells.
+template <bool VIRT>
+__device__ __forceinline__ double grid_cell_lam(const GridDev &g, const double *U, uint32_t i, uint32_t &sides) {
   double c[NF];
 #pragma unroll
   for (int k = 0; k < NF; ++k) c[k] = U[k * g.fs + i];
-  Tup T;
-  make_tup(c, T);
-  const int64_t q[3] = {i % g.n[0], (i / g.n[0]) % g.n[1], i / (g.n[0] * g.n[1])};
-  for (int a = 0; a < g.dim; ++a) {
-    m = lam_acc(m, fabs(T.vel[a]) + T.a);
-    bool refl = false;
-    for (int d = 0; d < 2; ++d) {
-      const int side = 2 * a + d;
-      int64_t nb;
-      if (neighbour(g, q, a, d ? 1 : -1, nb)) {
-        refl = refl || (g.flags && !(g.flags[nb] & CELL_FLUID));
-      } else if (g.bc[side] == BC_REFLECTING || g.bc[side] == BC_WALL) {
-        refl = true;
-      } else if (g.bc[side] == BC_DIRICHLET) {
-        double v[NF];
-        Tup V;
-        prim2cons(g.info[side], v);
-        make_tup(v, V);
-        m = lam_acc(m, fabs(V.vel[a]) + V.a);
+  if (!VIRT) return cell_max_eig_axes(c, g.dim == 3 ? 7u : 3u);
+  const uint32_t nx = (uint32_t)g.n[0], ny = (uint32_t)g.n[1], row = i / nx;
+  const uint32_t n[3] = {nx, ny, (uint32_t)g.n[2]}, st[3] = {1u, nx, nx * ny};
+  const uint32_t q[3] = {i - row * nx, g.dim == 3 ? row % ny : row, g.dim == 3 ? row / ny : 0u};
+  bool solved = true;
+  uint32_t refl = 0, dir = 0;
+  if (g.flags) {  // no load waits for another
+    uint8_t f[6], own = g.flags[i];
+#pragma unroll
+    for (int side = 0; side < 6; ++side) {
+      const int a = side / 2;
+      if (a >= g.dim) break;
+      const bool edge = q[a] == ((side & 1) ? n[a] - 1 : 0u);
+      const uint32_t o = edge ? (g.periodic[a] ? (n[a] - 1) * st[a] : 0u) : st[a];  // at a border: the cell itself
+      f[side] = g.flags[((side & 1) != 0) == edge ? i - o : i + o];
+    }
+    solved = own & CELL_SOLVED;
+#pragma unroll
+    for (int side = 0; side < 6; ++side) {
+      if (side / 2 >= g.dim) break;
+      if (!(f[side] & CELL_FLUID)) refl |= 1u << (side / 2);
+    }
+  }
+  double m = cell_max_eig_axes(c, g.dim == 3 ? 7u : 3u);
+  if (!solved) return 0.0;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    if (a >= g.dim) break;
+    if (!g.periodic[a]) {
+#pragma unroll
+      for (int side = 2 * a; side < 2 * a + 2; ++side) {
+        if (q[a] != ((side & 1) ? n[a] - 1 : 0u)) continue;
+        if (g.bc[side] == BC_REFLECTING || g.bc[side] == BC_WALL) refl |= 1u << a;
+        else if (g.bc[side] == BC_DIRICHLET) dir |= 1u << side;
       }
     }
-    if (refl) {
+    if (refl & (1u << a)) {
       double v[NF];
       Tup V;
       reflect_axis(c, a, v);
@@ -417,7 +437,31 @@ __device__ __forceinline__ double grid_cell_lam(const GridDev &g, const double *
       m = lam_acc(m, fabs(V.vel[a]) + V.a);
     }
   }
+  sides |= dir;
   return m;
+}
+
+// The border states' part (euler.cpp:366-376) at the Dirichlet sides touched.
+__device__ __forceinline__ double dirichlet_lam(const GridDev &g, uint32_t sides) {
+  double m = 0.0;
+  for (int side = 0; side < 2 * g.dim; ++side) {
+    if (!(sides & (1u << side))) continue;
+    const int a = side >> 1;
+    double v[NF];
+    Tup V;
+    prim2cons(g.info[side], v);
+    make_tup(v, V);
+    m = lam_acc(m, fabs((a == 0) ? V.vel[0] : (a == 1) ? V.vel[1] : V.vel[2]) + V.a);
+  }
+  return m;
+}
+
+// Ctrl::lam_now from the maxima that the blocks of this launch put into the
+// lam lines, by the first wave of the last block.
+__device__ __forceinline__ void set_lam_wave(Ctrl *c, int lane) {
+  unsigned long long v = (lane < EIG_SPLIT) ? atomicExch(&c->lam[lane][0], 0ull) : 0ull;
+  v = wave_max_u64(v);
+  if (lane == 0) c->lam_now = v;
 }
 
 // RK stage update of one field (main.cpp:421,457,493).
