@@ -174,11 +174,14 @@ __global__ __launch_bounds__(MB) void k_mesh_lam_axes(MeshDev m, uint8_t *lam_ax
   lam_axes[c] = plain ? (uint8_t)axes : 0;
 }
 
-// Stage 1 reads X = U and writes W1, stage 2 reads X = W1, stage 3 X = W2 and
-// writes U (out); RHS only: the residual of X = U.
+// Stage 1 reads X = U and writes W1 (out), stage 2 reads X = W1 and writes W2
+// to W, stage 3 reads X = W2 and writes U.  W is the reference's one stage
+// buffer: an unsolved cell keeps what it holds there (main.cpp:411-414,
+// 447-450), which stage 1 copies beside W1.  RHS only: the residual of X = U
+// as rows [cells][5], as the host takes them.
 template <int STAGE>
 __global__ __launch_bounds__(MB, 4) void k_mesh_stage(MeshDev m, const double *__restrict__ X, const double *U,
-                                                   double *out, Ctrl *ctrl, int mode) {
+                                                   const double *W, double *out, Ctrl *ctrl, int mode) {
   const bool step = mode == MODE_STEP;
   const int64_t c = (int64_t)blockIdx.x * MB + threadIdx.x;
   const int64_t fs = m.fs;
@@ -252,7 +255,7 @@ __global__ __launch_bounds__(MB, 4) void k_mesh_stage(MeshDev m, const double *_
     }
     if (!step) {
 #pragma unroll
-      for (int k = 0; k < NF; ++k) out[k * fs + c] = rhs[k];
+      for (int k = 0; k < NF; ++k) out[NF * c + k] = rhs[k];
     } else {
       double x[NF], q[NF], nu[NF];
 #pragma unroll
@@ -268,13 +271,12 @@ __global__ __launch_bounds__(MB, 4) void k_mesh_stage(MeshDev m, const double *_
       if (STAGE == 3) lam_nx = mesh_cell_lam(m, c, nu, U);
     }
   } else if (live && run) {
-    // unsolved cells keep their state (main.cpp:411-414); W2 has its own buffer
     if (!step) {
 #pragma unroll
-      for (int k = 0; k < NF; ++k) out[k * fs + c] = 0.0;
-    } else if (STAGE == 2) {
+      for (int k = 0; k < NF; ++k) out[NF * c + k] = 0.0;
+    } else if (STAGE == 1) {
 #pragma unroll
-      for (int k = 0; k < NF; ++k) out[k * fs + c] = X[k * fs + c];
+      for (int k = 0; k < NF; ++k) out[k * fs + c] = W[k * fs + c];
     }
   }
   if (!run) return;  // uniform over the grid
@@ -287,13 +289,13 @@ __global__ __launch_bounds__(MB, 4) void k_mesh_stage(MeshDev m, const double *_
   }
 }
 
-hipError_t launch_mesh_stage(const MeshDev &m, int stage, const double *X, const double *U, double *out, Ctrl *ctrl,
-                             int mode, hipStream_t s) {
+hipError_t launch_mesh_stage(const MeshDev &m, int stage, const double *X, const double *U, const double *W,
+                             double *out, Ctrl *ctrl, int mode, hipStream_t s) {
   const dim3 grid((unsigned)((m.N + MB - 1) / MB)), block(MB);
   switch (stage) {
-    case 1: hipLaunchKernelGGL(k_mesh_stage<1>, grid, block, 0, s, m, X, U, out, ctrl, mode); break;
-    case 2: hipLaunchKernelGGL(k_mesh_stage<2>, grid, block, 0, s, m, X, U, out, ctrl, mode); break;
-    default: hipLaunchKernelGGL(k_mesh_stage<3>, grid, block, 0, s, m, X, U, out, ctrl, mode);
+    case 1: hipLaunchKernelGGL(k_mesh_stage<1>, grid, block, 0, s, m, X, U, W, out, ctrl, mode); break;
+    case 2: hipLaunchKernelGGL(k_mesh_stage<2>, grid, block, 0, s, m, X, U, W, out, ctrl, mode); break;
+    default: hipLaunchKernelGGL(k_mesh_stage<3>, grid, block, 0, s, m, X, U, W, out, ctrl, mode);
   }
   return hipGetLastError();
 }

@@ -48,8 +48,8 @@ struct MeshDev {
   const int32_t *inc;     // incidences, per cell in increasing face index: face << 1 | (1 on the neighbour side)
 };
 
-hipError_t launch_mesh_stage(const MeshDev &m, int stage, const double *X, const double *U, double *out, Ctrl *ctrl,
-                             int mode, hipStream_t s);
+hipError_t launch_mesh_stage(const MeshDev &m, int stage, const double *X, const double *U, const double *W,
+                             double *out, Ctrl *ctrl, int mode, hipStream_t s);
 // Ctrl::lam_now of state U (zeroed beforehand).
 hipError_t launch_mesh_lam(const MeshDev &m, const double *U, Ctrl *ctrl, hipStream_t s);
 // adj, adj_kind (n incidences) and lam_axes from owner, neigh, kind, inc and flags.

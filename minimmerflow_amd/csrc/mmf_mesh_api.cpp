@@ -109,17 +109,19 @@ int refresh_adjacency(mmf_mesh *m) {
   return MMF_OK;
 }
 
-// W1 in dW, W2 in dR (the residual's buffer, free between the stages of a
-// step): a stage's cells read their neighbours' input while others are written.
+// W1 in dR (the residual's buffer, free between the stages of a step), W2 in
+// dW: a stage's cells read their neighbours' input while others are written.
+// dW changes in stage 2 and with the state only: a cell that turns unsolved
+// between steps keeps its last W2 there.
 int launch_stage(mmf_mesh *m, int stage, int mode) {
-  const double *X = (stage == 1) ? m->dU : (stage == 2) ? m->dW : m->dR;
-  double *out = (mode == mmf::MODE_RHS_ONLY) ? m->dR : (stage == 1) ? m->dW : (stage == 2) ? m->dR : m->dU;
+  const double *X = (stage == 1) ? m->dU : (stage == 2) ? m->dR : m->dW;
+  double *out = (stage == 1) ? m->dR : (stage == 2) ? m->dW : m->dU;
   hipEvent_t e[2] = {nullptr, nullptr};
   if (m->timing) {
     for (auto &x : e) MCHK(m, hipEventCreate(&x));
     MCHK(m, hipEventRecord(e[0], m->stream));
   }
-  const hipError_t r = mmf::launch_mesh_stage(m->m, stage, X, m->dU, out, m->dctrl, mode, m->stream);
+  const hipError_t r = mmf::launch_mesh_stage(m->m, stage, X, m->dU, m->dW, out, m->dctrl, mode, m->stream);
   if (r != hipSuccess) return mfail(m, MMF_ERR_HIP, std::string("stage kernel: ") + hipGetErrorString(r));
   if (m->timing) {
     MCHK(m, hipEventRecord(e[1], m->stream));
@@ -420,17 +422,12 @@ int mmf_mesh_set_state(mmf_mesh *m, const double *U) {
   return MMF_OK;
 }
 
-// Rows of the planes src through rows, a device buffer of their size.
-static int get_rows(mmf_mesh *m, const double *src, double *rows, double *U) {
-  const int64_t N = m->m.N, fs = m->m.fs;
-  MCHK(m, mmf::launch_soa_to_aos(src, nullptr, N, fs, rows, m->stream));
-  MCHK(m, mmf::copy_to_host(U, rows, sizeof(double) * 5 * (size_t)N, m->stream));
-  return MMF_OK;
-}
-
 int mmf_mesh_get_state(mmf_mesh *m, double *U) {
   if (!m || !U) return MMF_ERR_INVALID;
-  return get_rows(m, m->dU, m->dR, U);
+  const int64_t N = m->m.N;
+  MCHK(m, mmf::launch_soa_to_aos(m->dU, nullptr, N, m->m.fs, m->dR, m->stream));
+  MCHK(m, mmf::copy_to_host(U, m->dR, sizeof(double) * 5 * (size_t)N, m->stream));
+  return MMF_OK;
 }
 
 int mmf_mesh_compute_rhs(mmf_mesh *m, double *rhs, double *max_eig) {
@@ -439,12 +436,7 @@ int mmf_mesh_compute_rhs(mmf_mesh *m, double *rhs, double *max_eig) {
   if (e != hipSuccess) return mfail(m, MMF_ERR_HIP, "zero slot");
   int rc = launch_stage(m, 1, mmf::MODE_RHS_ONLY);
   if (rc != MMF_OK) return rc;
-  if (rhs) {
-    // through W, dead between steps but for the copy of U it then holds again
-    rc = get_rows(m, m->dR, m->dW, rhs);
-    if (rc != MMF_OK) return rc;
-    MCHK(m, hipMemcpyAsync(m->dW, m->dU, sizeof(double) * 5 * (size_t)m->m.fs, hipMemcpyDeviceToDevice, m->stream));
-  }
+  if (rhs) MCHK(m, mmf::copy_to_host(rhs, m->dR, sizeof(double) * 5 * (size_t)m->m.N, m->stream));
   rc = read_ctrl(m);
   if (rc != MMF_OK) return rc;
   if (max_eig) *max_eig = mmf::ctrl_stage_max(*m->hctrl, 3);

@@ -170,3 +170,33 @@ def test_mesh_nan_stops_the_run(mmf, orc):
     assert e.value.status == mmf.ERR_STATE
     assert g.counters()[2] >= 1
     g.close()
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+def test_cells_turned_unsolved_between_steps(mmf, orc, dim):
+    """The solved flags change between steps (ghost cells, main.cpp:231-235),
+    with read-backs in between: an unsolved cell keeps what the one stage
+    buffer of the serial loop holds there (main.cpp:411-414), bit for bit."""
+    fm = (meshes.refined(2, [24, 20], [0.0] * 3, 0.5, ([3.0, 2.0, 0], [7.5, 6.0, 0]), [0, 1, 3, 0], INFO) if dim == 2 else
+          meshes.refined(3, [10, 9, 8], [0.0] * 3, 0.5, ([1.0] * 3, [3.0, 2.5, 2.6]), [0, 1, 3, 0, 2, 0], INFO))
+    rng = np.random.default_rng(dim)
+    N = fm.ncells
+    o = face_solver(orc, orc.problem(orc.RADSOD, dim), fm)
+    g = mmf.Mesh(fm)
+    U0 = random_state(orc, rng, N, dim)
+    g.set_state(U0)
+    g.set_time(0.0, 1e30, 0.5)
+    Uo, Wo, t = U0.copy(), U0.copy(), 0.0
+    ones = np.ones(N, dtype=np.uint8)
+    for solved in (ones, (rng.uniform(size=N) > 0.1).astype(np.uint8), (rng.uniform(size=N) > 0.3).astype(np.uint8), ones):
+        g.set_cell_flags(ones, solved)
+        o.set_solved(solved)
+        for _ in range(2):
+            g.advance(1)
+            dt, eig = o.rk3_step(Uo, Wo, 0.5, t, 1e30)
+            t += dt
+            tg, dtg, _, eg = g.time()
+            assert (tg, dtg) == (t, dt) and np.array_equal(eg, eig)
+            assert np.array_equal(g.get_state(), Uo)
+            assert np.array_equal(g.compute_rhs()[0], o.compute_rhs(Uo)[0])
+    g.close()
