@@ -719,6 +719,7 @@ def main():
                   else "k_march tile %dx%d, the planes split over one block per CU in shares of equal cost" % (args.cols or 64,
                                                                                                kinfo[1])))
                 if kinfo[0] == mmf.KERNEL_MARCH
+                else "bricks (mmf_brick.hip, mmf_brick_o2.hip)" if kinfo[0] == mmf.KERNEL_BRICK
                 else "k_stage (per-cell gather)"),
             "algorithmic_bytes_per_launch": bytes_per_cell * N,
             "avg_launch_ms": avg_ms,

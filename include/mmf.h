@@ -83,22 +83,25 @@ const char *mmf_status_string(int status);
 int mmf_get_sizes(const mmf_ctx *ctx, int64_t *ncells, int64_t *ninterfaces);
 
 /* ---- stage-kernel selection ------------------------------------------------ */
-enum { MMF_KERNEL_AUTO = 0, MMF_KERNEL_GATHER = 1, MMF_KERNEL_MARCH = 2, MMF_KERNEL_TILE = 3 };
+enum { MMF_KERNEL_AUTO = 0, MMF_KERNEL_GATHER = 1, MMF_KERNEL_MARCH = 2, MMF_KERNEL_TILE = 3, MMF_KERNEL_BRICK = 4 };
 /* GATHER: per-cell kernel, any grid.  MARCH: the marching LDS-tile kernels
- * (order 1; order 2 in 2D without bodies).  TILE: the 8x8 LDS tile kernels of
- * 2D order-2 grids without bodies (each face once, the step's time advance
- * in its last stage; also the learned reconstruction's kernel).  AUTO: TILE
- * for 2D order-2 grids without bodies; MARCH where it applies from 2^18 cells
- * (2D order 1) or 2^20 cells (3D); else GATHER, which AUTO runs as LDS bricks
- * (a thread per cell, every flux tuple once per brick) where they apply: 3D
- * order 2 without bodies at any size, order 1 where every fluid cell is solved
- * and border conditions are per side, in 2D instead of MARCH below 2^24 cells,
- * in 3D from 2^20 cells only where MARCH's 64 x 8 tiles would be partly empty.  mmf_set_kernel refuses MARCH or TILE on a grid they do not
- * apply to; bodies set afterwards make them fall back to GATHER.  tile_rows (3D: 4 or 8) and chunk (planes per block along the last axis)
- * shape the marching kernel; <= 0 keeps the default (3D order 1, 64 x 8
+ * (order 1; order 2 in 2D without bodies, and in 3D).  TILE: the 8x8 LDS tile
+ * kernels of 2D order-2 grids without bodies (each face once, the step's time
+ * advance in its last stage; also the learned reconstruction's kernel).
+ * BRICK: LDS bricks, a thread per cell, every flux tuple once per brick (order
+ * 1 where every fluid cell is solved, order 2 in 3D without bodies; border
+ * conditions per side; fewer than 2^28 cells); small 2D grids advance a whole
+ * step per launch.  AUTO: TILE for 2D order-2 grids without bodies; BRICK for
+ * 3D order 2 without bodies at any size, for order 1 in 2D below 2^24 cells
+ * and in 3D below 2^20 cells, from there only where MARCH's 64 x 8 tiles would
+ * be partly empty; else MARCH where it applies from 2^18 cells (2D order 1) or
+ * 2^20 cells; else GATHER.  mmf_set_kernel refuses MARCH, TILE or BRICK on a
+ * grid they do not apply to; bodies set afterwards make them fall back to
+ * GATHER.  tile_rows (3D: 4 or 8) and chunk (planes per block along the last
+ * axis) shape the marching kernel; <= 0 keeps the default (3D order 1, 64 x 8
  * tiles: where the chunks would leave a partial round of blocks, the planes
  * of all tiles split over one block per CU in shares of equal cost, a plane
- * that needs the masked code near a body counting 2.5 times).  Every variant
+ * that needs the masked code near a body counting three times).  Every variant
  * gives bit-identical results. */
 int mmf_set_kernel(mmf_ctx *ctx, int32_t kind, int32_t tile_rows, int32_t chunk);
 /* 3D order 1, 64 x 8 tiles: the planes of all tiles split over 'blocks'
@@ -106,8 +109,9 @@ int mmf_set_kernel(mmf_ctx *ctx, int32_t kind, int32_t tile_rows, int32_t chunk)
  * count and the tile planes; a block marches up to four segments, each of
  * one tile and one code, masked or not); 0 restores the default. */
 int mmf_set_march_blocks(mmf_ctx *ctx, int32_t blocks);
-/* kind actually used for the next launches, and the marching shape (chunk 0:
- * the planes split over the blocks in shares of equal cost) */
+/* kind actually used for the next launches (mmf_set_kernel with it keeps
+ * them), and the marching shape (chunk 0: the planes split over the blocks in
+ * shares of equal cost) */
 int mmf_get_kernel(const mmf_ctx *ctx, int32_t *kind, int32_t *tile_rows, int32_t *chunk);
 /* The 3D marching kernel's tile (tile_x x tile_y cells: 64 x 4, 64 x 8,
  * 32 x 8 or 32 x 16) and chunk; <= 0 keeps the default of that field.  Does

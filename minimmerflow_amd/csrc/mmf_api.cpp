@@ -108,11 +108,18 @@ bool prefer_bricks(const GridDev &g) {
   return padded * (refl ? 10 : 7) > g.N * 13;
 }
 
+// The brick kind: order 1, or order 2 in 3D (2D order 2 has its bricks under
+// the tile kind).
+bool bricks_apply(const GridDev &g) {
+  return mmf::brick_supported(g) || (g.dim == 3 && mmf::brick_o2_supported(g));
+}
+
 // The stage kernel of the next launches.  With the learned reconstruction on:
 // the tile kernel, or (GATHER) the face-state + flux kernel pair.
 int kernel_used(const mmf_ctx *ctx) {
   if (ctx->learn_on) return ctx->kernel == mmf::KERNEL_GATHER ? mmf::KERNEL_GATHER : mmf::KERNEL_TILE;
   if (ctx->kernel == mmf::KERNEL_TILE) return tile_applies(ctx) ? mmf::KERNEL_TILE : mmf::KERNEL_GATHER;
+  if (ctx->kernel == mmf::KERNEL_BRICK) return bricks_apply(ctx->g) ? mmf::KERNEL_BRICK : mmf::KERNEL_GATHER;
   if (ctx->kernel == mmf::KERNEL_AUTO && tile_applies(ctx)) return mmf::KERNEL_TILE;
   if (ctx->kernel == mmf::KERNEL_AUTO && ctx->g.dim == 3 && mmf::brick_o2_supported(ctx->g)) return mmf::KERNEL_BRICK;
   if (ctx->kernel == mmf::KERNEL_AUTO && mmf::brick_supported(ctx->g) && prefer_bricks(ctx->g))
@@ -356,9 +363,11 @@ int mmf_set_kernel(mmf_ctx *ctx, int32_t kind, int32_t tile_rows, int32_t chunk)
   if (!ctx) return MMF_ERR_INVALID;
   ctx->lam_valid = false;
   ctx->tiles_valid = false;
-  if (kind < mmf::KERNEL_AUTO || kind > mmf::KERNEL_TILE) return fail(ctx, MMF_ERR_INVALID, "unknown kernel kind");
+  if (kind < mmf::KERNEL_AUTO || kind > mmf::KERNEL_BRICK) return fail(ctx, MMF_ERR_INVALID, "unknown kernel kind");
   if (kind == mmf::KERNEL_TILE && !tile_applies(ctx))
     return fail(ctx, MMF_ERR_INVALID, "tile kernel: order 2 in 2D without bodies");
+  if (kind == mmf::KERNEL_BRICK && !bricks_apply(ctx->g))
+    return fail(ctx, MMF_ERR_INVALID, "brick kernel: order 1 where every fluid cell is solved, or order 2 in 3D without bodies; border conditions per side; fewer than 2^28 cells");
   mmf::MarchShape sh = mmf::default_march_shape(ctx->g, ctx->num_cus);
   if (tile_rows > 0) sh.ty = tile_rows;
   if (chunk > 0) sh.chunk = chunk;
@@ -412,7 +421,7 @@ int mmf_set_march_blocks(mmf_ctx *ctx, int32_t blocks) {
 
 int mmf_get_kernel(const mmf_ctx *ctx, int32_t *kind, int32_t *tile_rows, int32_t *chunk) {
   if (!ctx) return MMF_ERR_INVALID;
-  if (kind) *kind = (kernel_used(ctx) == mmf::KERNEL_BRICK) ? (int)mmf::KERNEL_GATHER : kernel_used(ctx);
+  if (kind) *kind = kernel_used(ctx);
   if (tile_rows) *tile_rows = ctx->shape.ty;
   // 0: the planes of all tiles spread evenly over the blocks (3D order 1)
   if (chunk) *chunk = (ctx->shape.seg_blocks > 0 && ctx->g.dim == 3 && ctx->g.order == 1) ? 0 : ctx->shape.chunk;

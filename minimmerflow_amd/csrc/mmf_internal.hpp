@@ -60,7 +60,6 @@ __host__ __device__ inline int march_tile_of_block(int b, int nblk) {
 }
 
 // Stage-kernel variants.
-// KERNEL_BRICK is AUTO's choice only; at the C-ABI it reports as GATHER.
 enum KernelKind { KERNEL_AUTO = 0, KERNEL_GATHER = 1, KERNEL_MARCH = 2, KERNEL_TILE = 3, KERNEL_BRICK = 4 };
 
 // Launch shape of the marching kernel (tile rows and march chunk).
