@@ -367,7 +367,7 @@ int mmf_set_kernel(mmf_ctx *ctx, int32_t kind, int32_t tile_rows, int32_t chunk)
   if (kind == mmf::KERNEL_TILE && !tile_applies(ctx))
     return fail(ctx, MMF_ERR_INVALID, "tile kernel: order 2 in 2D without bodies");
   if (kind == mmf::KERNEL_BRICK && !bricks_apply(ctx->g))
-    return fail(ctx, MMF_ERR_INVALID, "brick kernel: order 1 where every fluid cell is solved, or order 2 in 3D without bodies; border conditions per side; fewer than 2^28 cells");
+    return fail(ctx, MMF_ERR_INVALID, "brick kernel: order 1 where every fluid cell is solved, or order 2 in 3D without bodies; border conditions per side; fewer than 2^28 cells, and than 2^32 with those that fill the bricks up");
   mmf::MarchShape sh = mmf::default_march_shape(ctx->g, ctx->num_cus);
   if (tile_rows > 0) sh.ty = tile_rows;
   if (chunk > 0) sh.chunk = chunk;

@@ -659,7 +659,10 @@ static hipError_t launch_brick_p(const GridDev &g, int stage, int mode, const do
 }
 
 bool brick_supported(const GridDev &g) {
-  return g.order == 1 && !g.bslot && (g.flags == nullptr || g.ghost_free) && g.N < BRICK_MAX_CELLS;
+  // a thread per cell of the bricks, up to 64 times the cells of a thin grid
+  const int64_t threads = (g.dim == 3) ? padded_cells(g, 8, 8, 4) : padded_cells(g, 16, 16, 1);
+  return g.order == 1 && !g.bslot && (g.flags == nullptr || g.ghost_free) && g.N < BRICK_MAX_CELLS &&
+         threads < LAUNCH_THREADS;
 }
 
 template <int DIM, int BX, int BY, int BZ>

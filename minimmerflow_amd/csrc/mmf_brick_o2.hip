@@ -346,7 +346,10 @@ static hipError_t launch_brick_o2_p(const GridDev &g, int stage, int mode, const
   return hipGetLastError();
 }
 
-bool brick_o2_supported(const GridDev &g) { return g.order == 2 && !g.bslot && !g.flags && g.N < BRICK_MAX_CELLS; }
+bool brick_o2_supported(const GridDev &g) {
+  return g.order == 2 && !g.bslot && !g.flags && g.N < BRICK_MAX_CELLS &&
+         padded_cells(g, 8, 8, g.dim == 3 ? 4 : 1) < LAUNCH_THREADS;
+}
 
 hipError_t launch_stage_brick_o2(const GridDev &g, int stage, int mode, const double *U, const double *R,
                                  const double *W, double *oR, double *oW, double *oU, Ctrl *ctrl, hipStream_t s) {

@@ -144,6 +144,15 @@ inline OutputLayout output_layout(int64_t N) {
 // cells rounded up to 64.
 int grid_from_desc(const mmf_grid_desc *d, GridDev &g);
 
+// Cells of the bricks of bx x by x bz cells that cover the grid.
+inline int64_t padded_cells(const GridDev &g, int64_t bx, int64_t by, int64_t bz) {
+  return (g.n[0] + bx - 1) / bx * bx * ((g.n[1] + by - 1) / by * by) * ((g.n[2] + bz - 1) / bz * bz);
+}
+
+// Threads of a launch stay below this: a larger launch runs modulo 2^32
+// threads, and no error tells.
+constexpr int64_t LAUNCH_THREADS = (int64_t)1 << 32;
+
 // Order-1 brick kernel (mmf_brick.hip): without per-face conditions, every
 // fluid cell solved, 32-bit cell indices.
 constexpr int64_t BRICK_MAX_CELLS = (int64_t)1 << 28;

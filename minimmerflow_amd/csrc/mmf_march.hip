@@ -871,21 +871,23 @@ int64_t march_blocks(const GridDev &g, const MarchShape &sh) {
 // hold a flag (wrapped across periodic sides).  One wave per tile plane: the
 // host read every flag for this one byte at a time, 6 ms of the first step of
 // a 192^3 grid with a body and as much after every change of one.
-__global__ __launch_bounds__(64) void k_tile_planes(GridDev g, int TX, int TY, int ntx, uint8_t *ring) {
+__global__ __launch_bounds__(64) void k_tile_planes(GridDev g, int TX, int TY, int ntx, int64_t planes, uint8_t *ring) {
   const int nx = (int)g.n[0], ny = (int)g.n[1], nz = (int)g.n[2];
-  const int t = (int)(blockIdx.x / (unsigned)nz), z = (int)(blockIdx.x % (unsigned)nz);
-  const int x0 = (t % ntx) * TX, y0 = (t / ntx) * TY;
-  const int w = min(TX, nx - x0) + 2, h = min(TY, ny - y0) + 2;
-  bool m = false;
-  for (int p = threadIdx.x; p < w * h; p += 64) {
-    int x = x0 - 1 + p % w, y = y0 - 1 + p / w;
-    if (((x < 0 || x >= nx) && !g.periodic[0]) || ((y < 0 || y >= ny) && !g.periodic[1])) continue;
-    x = (x + nx) % nx;
-    y = (y + ny) % ny;
-    m = m || g.flags[(int64_t)x + (int64_t)nx * ((int64_t)y + (int64_t)ny * z)] != (CELL_FLUID | CELL_SOLVED);
+  for (int64_t i = blockIdx.x; i < planes; i += gridDim.x) {
+    const int t = (int)(i / nz), z = (int)(i % nz);
+    const int x0 = (t % ntx) * TX, y0 = (t / ntx) * TY;
+    const int w = min(TX, nx - x0) + 2, h = min(TY, ny - y0) + 2;
+    bool m = false;
+    for (int p = threadIdx.x; p < w * h; p += 64) {
+      int x = x0 - 1 + p % w, y = y0 - 1 + p / w;
+      if (((x < 0 || x >= nx) && !g.periodic[0]) || ((y < 0 || y >= ny) && !g.periodic[1])) continue;
+      x = (x + nx) % nx;
+      y = (y + ny) % ny;
+      m = m || g.flags[(int64_t)x + (int64_t)nx * ((int64_t)y + (int64_t)ny * z)] != (CELL_FLUID | CELL_SOLVED);
+    }
+    const bool any = __ballot(m) != 0;
+    if (threadIdx.x == 0) ring[i] = any;
   }
-  const bool any = __ballot(m) != 0;
-  if (threadIdx.x == 0) ring[blockIdx.x] = any;
 }
 
 int64_t march_tile_planes(const GridDev &g, const MarchShape &sh) {
@@ -894,7 +896,10 @@ int64_t march_tile_planes(const GridDev &g, const MarchShape &sh) {
 
 hipError_t launch_tile_planes(const GridDev &g, const MarchShape &sh, uint8_t *ring, hipStream_t s) {
   const int ntx = (int)((g.n[0] + sh.tx - 1) / sh.tx);
-  hipLaunchKernelGGL(k_tile_planes, dim3((unsigned)march_tile_planes(g, sh)), dim3(64), 0, s, g, sh.tx, sh.ty, ntx, ring);
+  const int64_t planes = march_tile_planes(g, sh);
+  // a wave each; a thin grid's, as many as its cells, in turns
+  const unsigned nb = (unsigned)std::min(planes, LAUNCH_THREADS / 128);
+  hipLaunchKernelGGL(k_tile_planes, dim3(nb), dim3(64), 0, s, g, sh.tx, sh.ty, ntx, planes, ring);
   return hipGetLastError();
 }
 
