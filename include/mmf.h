@@ -91,8 +91,9 @@ enum { MMF_KERNEL_AUTO = 0, MMF_KERNEL_GATHER = 1, MMF_KERNEL_MARCH = 2, MMF_KER
  * BRICK: LDS bricks, a thread per cell, every flux tuple once per brick (order
  * 1 where every fluid cell is solved, order 2 in 3D without bodies; border
  * conditions per side; fewer than 2^28 cells, and than 2^32 with those that
- * fill the bricks up); small 2D grids advance a whole step per launch.  AUTO: TILE for 2D order-2 grids without bodies; BRICK for
- * 3D order 2 without bodies at any size, for order 1 in 2D below 2^24 cells
+ * fill the bricks up); small 2D grids advance a whole step per launch.  AUTO:
+ * TILE for 2D order-2 grids without bodies below 2^28 cells; BRICK for 3D
+ * order 2 without bodies below 2^28 cells, for order 1 in 2D below 2^24 cells
  * and in 3D below 2^20 cells, from there only where MARCH's 64 x 8 tiles would
  * be partly empty; else MARCH where it applies from 2^18 cells (2D order 1) or
  * 2^20 cells; else GATHER.  mmf_set_kernel refuses MARCH, TILE or BRICK on a

@@ -78,7 +78,8 @@ bool tile_applies(const mmf_ctx *ctx) {
 // 10.5, 128^2 25.7 / 11.3 and 27.7 / 11.1, 192^2 35 / 20 and 30 / 12, 256^2 48 /
 // 33 and 33 / 14; 512^2 128 (gather) and 69, 2048^2 1343 (strips) and 664.
 // 3D order 2 always takes the bricks: 32^3 66 (gather) and 37, 144^3 1357
-// (marching) and 594, 256^3 5207 and 3282.
+// (marching) and 594, 256^3 5207 and 3282.  Where the bricks do not apply, from
+// 2^28 cells, the six waves are no alternative (2048^2 2.0 ms): AUTO marches.
 constexpr int64_t TILE_SIX_WAVES_MAX_N = (int64_t)1 << 14;
 
 bool o2_bricks(const GridDev &g) {
@@ -120,7 +121,8 @@ int kernel_used(const mmf_ctx *ctx) {
   if (ctx->learn_on) return ctx->kernel == mmf::KERNEL_GATHER ? mmf::KERNEL_GATHER : mmf::KERNEL_TILE;
   if (ctx->kernel == mmf::KERNEL_TILE) return tile_applies(ctx) ? mmf::KERNEL_TILE : mmf::KERNEL_GATHER;
   if (ctx->kernel == mmf::KERNEL_BRICK) return bricks_apply(ctx->g) ? mmf::KERNEL_BRICK : mmf::KERNEL_GATHER;
-  if (ctx->kernel == mmf::KERNEL_AUTO && tile_applies(ctx)) return mmf::KERNEL_TILE;
+  if (ctx->kernel == mmf::KERNEL_AUTO && tile_applies(ctx) && (ctx->g.N <= TILE_SIX_WAVES_MAX_N || o2_bricks(ctx->g)))
+    return mmf::KERNEL_TILE;
   if (ctx->kernel == mmf::KERNEL_AUTO && ctx->g.dim == 3 && mmf::brick_o2_supported(ctx->g)) return mmf::KERNEL_BRICK;
   if (ctx->kernel == mmf::KERNEL_AUTO && mmf::brick_supported(ctx->g) && prefer_bricks(ctx->g))
     return mmf::KERNEL_BRICK;

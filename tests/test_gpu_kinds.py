@@ -36,6 +36,8 @@ AUTO_KINDS = [
     (3, (256, 128, 64), 1, "MARCH"),
     (2, (100, 100), 2, "TILE"),
     (2, (600, 500), 2, "TILE"),
+    (2, ((1 << 14) - 1, 1 << 14), 2, "TILE"),
+    (2, (1 << 14, 1 << 14), 2, "MARCH"),  # beyond the bricks' cells
     (3, (32, 32, 32), 2, "BRICK"),
     (3, (144, 144, 144), 2, "BRICK"),
 ]
