@@ -96,8 +96,10 @@ enum { MMF_KERNEL_AUTO = 0, MMF_KERNEL_GATHER = 1, MMF_KERNEL_MARCH = 2, MMF_KER
  * order 2 without bodies below 2^28 cells, for order 1 in 2D below 2^24 cells
  * and in 3D below 2^20 cells, from there only where MARCH's 64 x 8 tiles would
  * be partly empty; else MARCH where it applies from 2^18 cells (2D order 1) or
- * 2^20 cells; else GATHER.  mmf_set_kernel refuses MARCH, TILE or BRICK on a
- * grid they do not apply to; bodies set afterwards make them fall back to
+ * 2^20 cells; else GATHER.  Grids a few cells across, which leave bricks mostly
+ * empty, run the cheapest of the three by their padding (large ones: tubes
+ * GATHER, sheets MARCH or GATHER).  mmf_set_kernel refuses MARCH, TILE or BRICK
+ * on a grid they do not apply to; bodies set afterwards make them fall back to
  * GATHER.  tile_rows (3D: 4 or 8) and chunk (planes per block along the last
  * axis) shape the marching kernel; <= 0 keeps the default (3D order 1, 64 x 8
  * tiles: where the chunks would leave a partial round of blocks, the planes

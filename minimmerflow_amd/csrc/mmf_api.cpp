@@ -55,9 +55,8 @@ bool valid_bc(int b) { return b >= MMF_BC_FREE_FLOW && b <= MMF_BC_PERIODIC; }
 // it a grid gives the marching kernels too few blocks or rows to march):
 // 2D order 1 from 2^18 cells (64^2 56 vs 28 us per step, 512^2 equal, 1024^2
 // 137 vs 188), 3D order 1 from 2^20 (32^3 273 vs 37 us, 96^3 319 vs 193,
-// 128^3 271 vs 379), 3D order 2 (with bodies) from 2^20.  Order-1 grids without
-// ghost cells or per-face conditions go to the brick kernel where prefer_bricks
-// says so, order-2 grids without bodies to the tile kind and the bricks.
+// 128^3 271 vs 379), order 2 from 2^20.  Where the bricks apply, fit_order1 and
+// fit_order2 choose.
 bool use_march(const mmf_ctx *ctx) {
   if (ctx->kernel == mmf::KERNEL_GATHER || !mmf::march_shape_supported(ctx->g, ctx->shape)) return false;
   if (ctx->kernel == mmf::KERNEL_AUTO) {
@@ -77,7 +76,7 @@ bool tile_applies(const mmf_ctx *ctx) {
 // in flight, six waves against one (MI355X, vortex): 64^2 25.5 / 9.8 and 27.9 /
 // 10.5, 128^2 25.7 / 11.3 and 27.7 / 11.1, 192^2 35 / 20 and 30 / 12, 256^2 48 /
 // 33 and 33 / 14; 512^2 128 (gather) and 69, 2048^2 1343 (strips) and 664.
-// 3D order 2 always takes the bricks: 32^3 66 (gather) and 37, 144^3 1357
+// 3D order 2 takes the bricks at any size: 32^3 66 (gather) and 37, 144^3 1357
 // (marching) and 594, 256^3 5207 and 3282.  Where the bricks do not apply, from
 // 2^28 cells, the six waves are no alternative (2048^2 2.0 ms): AUTO marches.
 constexpr int64_t TILE_SIX_WAVES_MAX_N = (int64_t)1 << 14;
@@ -86,7 +85,7 @@ bool o2_bricks(const GridDev &g) {
   return mmf::brick_o2_supported(g) && (g.dim == 3 || g.N > TILE_SIX_WAVES_MAX_N);
 }
 
-// AUTO's choice between the brick and the marching kernel for order 1 (us per
+// Order-1 bricks or the marching kernel, on grids that fill their bricks (us per
 // step alone / with three grids in flight, marching against brick; MI355X).
 // 2D: bricks; 400 x 300 50 / 25 and 21 / 17, 1000 x 600 70 / 42 and 53 / 39,
 // 1200 x 1000 periodic 115 / 86 and 84 / 91, 1500 x 1400 reflecting 333 / 167
@@ -99,14 +98,66 @@ bool o2_bricks(const GridDev &g) {
 // partly empty go to the bricks (40 x 40 x 900 202 / 188 and 144 / 164): where
 // the padded cells exceed 1.3 times the grid's, or 1.86 times without
 // reflected states, whose full tiles march the cheaper flat pass.
-bool prefer_bricks(const GridDev &g) {
-  if (g.dim == 2) return g.N < ((int64_t)1 << 24);
-  if (g.N < ((int64_t)1 << 20)) return true;
+//
+// Thin grids (a few cells across) leave most of a brick empty.  Its empty cells
+// cost two thirds of a full one in 3D and half of one in 2D, the gather kernel
+// needs no padding but 1.9 times a full brick's time per cell (twice in 2D), and
+// the marching tiles and strips have their own: the cheapest by these estimates
+// runs.  us per step, gather / marching / bricks:
+//   2D 200,000 x 1 46 / 39 / 148, 500,000 x 2 155 / 91 / 356, 4 x 250,000 159 /
+//   718 / 227, 8 x 100,000 136 / 371 / 104
+//   3D 60,000 x 1 x 1 33 / 72 / 149, 400 x 2 x 400 95 / 125 / 121, 400,000 x 2 x 2
+//   310 / 569 / 970, 1100 x 1 x 1100 234 / 529 / 802, 550 x 4 x 550 255 / 166 /
+//   220, 4 x 550 x 550 250 / 3467 / 218, 1100 x 1100 x 1 235 / 227 / 363
+// Up to BRICK_CELLS_MIN cells of bricks their launches are as short as any (200
+// x 200 x 1 with 160,000 37 / 36 / 23 us, 8000 x 1 x 1 with 256,000 32 / 23 / 33).
+constexpr int64_t BRICK_CELLS_MIN = (int64_t)160 << 10;
+
+enum class Fit { BRICK, MARCH, GATHER };
+
+// Columns of tiles of w cells that cover n.
+int64_t padded_to(int64_t n, int64_t w) { return (n + w - 1) / w * w; }
+
+Fit fit_order1(const GridDev &g) {
+  const double N = (double)g.N;
+  if (g.dim == 2) {
+    if (g.N >= ((int64_t)1 << 24)) return Fit::MARCH;
+    const int64_t w = mmf::brick_width_2d(g), padded = mmf::padded_cells(g, w, w, 1);
+    if (padded <= BRICK_CELLS_MIN) return Fit::BRICK;
+    const double brick = (double)padded + N, gather = 4.0 * N;
+    // the strips are 62 cells wide, and there are enough of them from 2^18 cells
+    const double march = (g.N < ((int64_t)1 << 18)) ? HUGE_VAL : 2.2 * (double)(padded_to(g.n[0], 62) * g.n[1]);
+    return (brick <= march && brick <= gather) ? Fit::BRICK : (march <= gather) ? Fit::MARCH : Fit::GATHER;
+  }
+  const int64_t padded = mmf::padded_cells(g, 8, 8, 4);
+  if (g.N < ((int64_t)1 << 20)) return (padded <= BRICK_CELLS_MIN || 4 * padded <= 11 * g.N) ? Fit::BRICK : Fit::GATHER;
   bool refl = g.flags != nullptr;
   for (int s = 0; s < 6; ++s)
     refl = refl || (!g.periodic[s / 2] && (g.bc[s] == MMF_BC_REFLECTING || g.bc[s] == MMF_BC_WALL));
-  const int64_t padded = (g.n[0] + 63) / 64 * 64 * ((g.n[1] + 7) / 8 * 8) * g.n[2];
-  return padded * (refl ? 10 : 7) > g.N * 13;
+  const int64_t tiles = padded_to(g.n[0], 64) * padded_to(g.n[1], 8) * g.n[2];
+  if (2 * padded <= 3 * g.N) return tiles * (refl ? 10 : 7) > g.N * 13 ? Fit::BRICK : Fit::MARCH;
+  const double brick = (2.0 * (double)padded + N) / 3.0, gather = 1.9 * N;
+  // a marching tile reads a plane below and above its own
+  const double march = (double)tiles * (1.0 + 2.0 / (double)g.n[2]) / (refl ? 1.3 : 13.0 / 7.0);
+  return (brick <= march && brick <= gather) ? Fit::BRICK : (march <= gather) ? Fit::MARCH : Fit::GATHER;
+}
+
+// The same for order 2 without bodies (us per step, gather / marching or strips /
+// bricks): 2D 200,000 x 1 90 / 80 / 253, 100,000 x 3 139 / 90 / 144, 100,000 x 4
+// 184 / 112 / 145, 3 x 100,000 143 / 1693 / 144, 500,000 x 4 719 / 415 / 607,
+// 500,000 x 6 1125 / 604 / 628; 3D 60,000 x 1 x 1 52 / 132 / 323, 300 x 3 x 300
+// 206 / 252 / 163, 400 x 2 x 400 205 / 458 / 259, 800 x 2 x 800 663 / 1638 / 954,
+// 650 x 3 x 650 677 / 914 / 650, 1100 x 1100 x 1 589 / 528 / 815.
+Fit fit_order2(const GridDev &g) {
+  const bool large = g.N >= ((int64_t)1 << 20);
+  if (g.dim == 2) {
+    const int64_t padded = mmf::padded_cells(g, 8, 8, 1), strips = padded_to(g.n[0], 60) * g.n[1];
+    if (padded <= BRICK_CELLS_MIN || (2 * padded <= 5 * g.N && (!large || 20 * padded <= 27 * strips))) return Fit::BRICK;
+    return (large && 10 * strips <= 13 * g.N) ? Fit::MARCH : Fit::GATHER;
+  }
+  const int64_t padded = mmf::padded_cells(g, 8, 8, 4);
+  if (padded <= BRICK_CELLS_MIN || padded <= 3 * g.N) return Fit::BRICK;
+  return (large && 4 * padded_to(g.n[0], 64) * padded_to(g.n[1], 8) * g.n[2] <= 5 * g.N) ? Fit::MARCH : Fit::GATHER;
 }
 
 // The brick kind: order 1, or order 2 in 3D (2D order 2 has its bricks under
@@ -121,11 +172,14 @@ int kernel_used(const mmf_ctx *ctx) {
   if (ctx->learn_on) return ctx->kernel == mmf::KERNEL_GATHER ? mmf::KERNEL_GATHER : mmf::KERNEL_TILE;
   if (ctx->kernel == mmf::KERNEL_TILE) return tile_applies(ctx) ? mmf::KERNEL_TILE : mmf::KERNEL_GATHER;
   if (ctx->kernel == mmf::KERNEL_BRICK) return bricks_apply(ctx->g) ? mmf::KERNEL_BRICK : mmf::KERNEL_GATHER;
-  if (ctx->kernel == mmf::KERNEL_AUTO && tile_applies(ctx) && (ctx->g.N <= TILE_SIX_WAVES_MAX_N || o2_bricks(ctx->g)))
-    return mmf::KERNEL_TILE;
-  if (ctx->kernel == mmf::KERNEL_AUTO && ctx->g.dim == 3 && mmf::brick_o2_supported(ctx->g)) return mmf::KERNEL_BRICK;
-  if (ctx->kernel == mmf::KERNEL_AUTO && mmf::brick_supported(ctx->g) && prefer_bricks(ctx->g))
-    return mmf::KERNEL_BRICK;
+  if (ctx->kernel == mmf::KERNEL_AUTO) {
+    const GridDev &g = ctx->g;
+    if (tile_applies(ctx) && g.N <= TILE_SIX_WAVES_MAX_N) return mmf::KERNEL_TILE;
+    const bool bricks2 = o2_bricks(g), bricks = bricks2 || mmf::brick_supported(g);
+    const Fit fit = bricks2 ? fit_order2(g) : bricks ? fit_order1(g) : Fit::MARCH;
+    if (fit == Fit::BRICK) return (g.dim == 2 && bricks2) ? mmf::KERNEL_TILE : mmf::KERNEL_BRICK;
+    if (fit == Fit::GATHER) return mmf::KERNEL_GATHER;
+  }
   return use_march(ctx) ? mmf::KERNEL_MARCH : mmf::KERNEL_GATHER;
 }
 

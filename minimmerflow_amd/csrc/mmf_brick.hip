@@ -368,8 +368,11 @@ __global__ __launch_bounds__(BX *BY *BZ) void k_brick(GridDev g, const double *X
 //   256 x 200 inflow     18.7 / 9.0    15.9 / 8.3
 //   255 x 256 reflecting 21.1 / 10.1   18.4 / 10.4
 //   300 x 300 inflow     22.3 / 11.1   21.9 / 12.9
-// so up to 2^16 cells, where a chip of blocks is about full.  What is left is
-// one launch's latency, the chain of three stages and the step's close.
+// so up to 2^16 cells, where a chip of blocks is about full (three fit a CU:
+// 768).  Thin grids reach that earlier and then wait for blocks of mostly empty
+// regions: 12,000 x 1 (1200 blocks) 21.8 / 9.0 and 19.1 / 12.7, 60,000 x 1 44 / 29
+// and 66 / 61; so up to 768 blocks.  What is left is one launch's latency, the
+// chain of three stages and the step's close.
 template <int R, bool P2>
 __global__ __launch_bounds__(R *R) void k_brick_step(GridDev g, const double *X, double *out, Ctrl *ctrl, int nbx) {
   constexpr int NT = R * R, O = R - 6, NW = NT / 64;
@@ -569,7 +572,8 @@ hipError_t launch_step_brick(const GridDev &g, const double *in, double *out, Ct
 }
 
 bool step_brick_supported(const GridDev &g) {
-  return brick_supported(g) && g.dim == 2 && g.flags == nullptr && g.N < STEP_BRICK_MAX_CELLS;
+  return brick_supported(g) && g.dim == 2 && g.flags == nullptr && g.N < STEP_BRICK_MAX_CELLS &&
+         padded_cells(g, STEP_R - 6, STEP_R - 6, 1) <= STEP_BRICK_MAX_BLOCKS * (STEP_R - 6) * (STEP_R - 6);
 }
 
 // ---- batches: one block per brick of every case --------------------------------
@@ -686,7 +690,7 @@ static hipError_t launch_brick_s(const GridDev &g, int stage, int mode, const do
 hipError_t launch_stage_brick(const GridDev &g, int stage, int mode, const double *U, const double *R, const double *W,
                               double *oR, double *oW, double *oU, Ctrl *ctrl, hipStream_t s) {
   if (g.dim == 3) return launch_brick_s<3, 8, 8, 4>(g, stage, mode, U, R, W, oR, oW, oU, ctrl, s);
-  if (g.N >= (1 << 16)) return launch_brick_s<2, 16, 16, 1>(g, stage, mode, U, R, W, oR, oW, oU, ctrl, s);
+  if (brick_width_2d(g) == 16) return launch_brick_s<2, 16, 16, 1>(g, stage, mode, U, R, W, oR, oW, oU, ctrl, s);
   return launch_brick_s<2, 8, 8, 1>(g, stage, mode, U, R, W, oR, oW, oU, ctrl, s);
 }
 

@@ -157,12 +157,14 @@ constexpr int64_t LAUNCH_THREADS = (int64_t)1 << 32;
 // fluid cell solved, 32-bit cell indices.
 constexpr int64_t BRICK_MAX_CELLS = (int64_t)1 << 28;
 bool brick_supported(const GridDev &g);
+// Width of a 2D brick: 16 x 16 cells once that gives every CU a block.
+inline int64_t brick_width_2d(const GridDev &g) { return g.N >= ((int64_t)1 << 16) ? 16 : 8; }
 hipError_t launch_stage_brick(const GridDev &g, int stage, int mode, const double *U, const double *R, const double *W,
                               double *oR, double *oW, double *oU, Ctrl *ctrl, hipStream_t s);
 
 // A whole step per launch (mmf_brick.hip): 2D bricks without a body, from one
 // buffer to another; dt is Ctrl::lam_now's, as for the brick kernel.
-constexpr int64_t STEP_BRICK_MAX_CELLS = (int64_t)1 << 16;
+constexpr int64_t STEP_BRICK_MAX_CELLS = (int64_t)1 << 16, STEP_BRICK_MAX_BLOCKS = 768;
 bool step_brick_supported(const GridDev &g);
 hipError_t launch_step_brick(const GridDev &g, const double *in, double *out, Ctrl *ctrl, hipStream_t s);
 

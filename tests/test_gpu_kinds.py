@@ -38,6 +38,28 @@ AUTO_KINDS = [
     (2, (600, 500), 2, "TILE"),
     (2, ((1 << 14) - 1, 1 << 14), 2, "TILE"),
     (2, (1 << 14, 1 << 14), 2, "MARCH"),  # beyond the bricks' cells
+    # a few cells across: not to bricks of mostly padding, unless they are few
+    (2, (7680, 1), 1, "BRICK"),
+    (2, (60000, 1), 1, "GATHER"),
+    (2, (1, 200000), 1, "GATHER"),
+    (2, (500000, 2), 1, "MARCH"),
+    (2, (2, 500000), 1, "GATHER"),
+    (2, (8, 100000), 1, "BRICK"),
+    (3, (1000, 1, 1), 1, "BRICK"),
+    (3, (60000, 1, 1), 1, "GATHER"),
+    (3, (1, 1, 400000), 1, "GATHER"),
+    (3, (60000, 4, 4), 1, "BRICK"),
+    (3, (1100, 1, 1100), 1, "GATHER"),
+    (3, (1100, 1100, 1), 1, "MARCH"),
+    (3, (550, 4, 550), 1, "MARCH"),
+    (3, (4, 550, 550), 1, "BRICK"),
+    (2, (200000, 1), 2, "GATHER"),
+    (2, (500000, 4), 2, "MARCH"),
+    (2, (100000, 4), 2, "TILE"),
+    (3, (60000, 1, 1), 2, "GATHER"),
+    (3, (300, 3, 300), 2, "BRICK"),
+    (3, (800, 2, 800), 2, "GATHER"),
+    (3, (1100, 1100, 1), 2, "MARCH"),
     (3, (32, 32, 32), 2, "BRICK"),
     (3, (144, 144, 144), 2, "BRICK"),
 ]
