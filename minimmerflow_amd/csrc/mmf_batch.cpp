@@ -133,16 +133,29 @@ int build_items(mmf_batch *b) {
   return MMF_OK;
 }
 
-// Batches below this many cells run as bricks, one block each, larger ones as
-// the persistent strips, which issue a little less per cell but march their
-// rows one after another (us per step, strips / bricks, MI355X: 8 cases of
-// 316,416 cells 164 / 41, 60 of 1,728,000 217 / 129, 512 of 13,116,160 1012 /
-// 1064).
-constexpr int64_t BATCH_BRICKS_MAX_CELLS = (int64_t)1 << 23;
+// Bricks, one block each, or the persistent strips, which cost less per cell but
+// start slowly and march their rows one after another: the cheaper by what a
+// step of them takes in us (MI355X; P cells of the bricks, S cells of the strips
+// of 62 with a row below and above, N cells, all in millions): bricks 10 + 46 P +
+// 40 N, strips 115 + 39 S + 22 N.  us per step, strips / bricks: 8 cases of
+// 316,416 cells 164 / 41, 60 of 1,728,000 217 / 129, 512 of 100 x 100 482 / 540,
+// 32 of 500 x 500 647 / 727, 512 of 13,116,160 cells 1012 / 1064; thin cases: 64
+// of 1000 x 1 116 / 68, 64 of 8000 x 1 185 / 391, 16 of 20,000 x 4 190 / 266, 16
+// of 1 x 20,000 905 / 300.
+bool prefer_bricks(const mmf_batch *b) {
+  double P = 0.0, S = 0.0, N = 0.0;
+  for (const BatchCase &c : b->hcases) {
+    const GridDev &g = c.g;
+    P += 1e-6 * (double)mmf::padded_cells(g, 16, 16, 1);
+    S += 1e-6 * (double)((g.n[0] + 61) / 62 * 62 * (g.n[1] + 2));
+    N += 1e-6 * (double)g.N;
+  }
+  return 10.0 + 46.0 * P + 40.0 * N <= 115.0 + 39.0 * S + 22.0 * N;
+}
 
 // The blocks of the brick stages, in case order.
 int build_bricks(mmf_batch *b) {
-  b->bricks = b->total_cells < BATCH_BRICKS_MAX_CELLS;
+  b->bricks = prefer_bricks(b);
   if (!b->bricks) return MMF_OK;
   std::vector<int> v;
   for (int i = 0; i < b->ncases; ++i) {

@@ -220,3 +220,61 @@ def test_batch_problem_setup_and_error(mmf, orc):
         eo, _ = o.error(U, tend[i])
         assert so == steps[i] and to == t[i], i
         assert abs(l1[i] - eo) <= 1e-12 * eo, (i, l1[i], eo)
+
+
+def small_steps_equal_single(mmf, shapes):
+    """Three steps of a batch against each grid alone with the gather kernel."""
+    rng = np.random.default_rng(5)
+    states = []
+    for n in shapes:
+        U = np.zeros((n[0] * n[1], 5))
+        U[:, 0] = rng.uniform(0.8, 1.2, len(U))
+        U[:, 1:3] = rng.uniform(-0.2, 0.2, (len(U), 2))
+        U[:, 4] = rng.uniform(2.0, 3.0, len(U))
+        states.append(U)
+    b = mmf.Batch([mmf.grid_desc(2, list(n), [0.0] * 3, 0.01, [0] * 4) for n in shapes])
+    for i, U in enumerate(states):
+        b.set_state(i, U)
+    b.set_time(0.0, 1e30, 0.4)
+    b.advance(3)
+    for i, n in enumerate(shapes):
+        s = mmf.Solver(2, list(n), [0.0] * 3, 0.01, [0] * 4)
+        s.set_kernel(mmf.KERNEL_GATHER)
+        s.set_state(states[i])
+        s.set_time(0.0, 1e30, 0.4)
+        s.advance(3)
+        assert b.times()[0][i] == s.time()[0]
+        assert np.array_equal(b.get_state(i), s.get_state()), n
+        s.close()
+    b.close()
+
+
+@pytest.mark.parametrize("shapes", [
+    [(1000, 1), (1, 1000), (3, 700)],  # few bricks
+    [(60000, 1)] * 4 + [(1, 3000)],  # strips
+    [(1, 60000), (2, 40000), (9, 20000)],  # bricks
+    [(50000, 3)] * 8,  # strips
+    [(500, 500)] * 20,  # strips
+], ids=lambda v: "%dx%d" % v[0])
+def test_thin_and_large_batches_equal_single_grids(mmf, shapes):
+    small_steps_equal_single(mmf, shapes)
+
+
+@pytest.mark.parametrize("chunk,blocks,tail", [(1, 1, 0), (3, 7, 0), (64, 2048, 0), (8, 3, 1)])
+def test_strip_shapes(mmf, chunk, blocks, tail):
+    """Every shape of the strips (a large idle case keeps the batch off the
+    bricks) against the bricks of the same cases."""
+    cs, states = setup(mmf)
+    ref = make_batch(mmf, cs, states)
+    ref.advance(STEPS)
+    b = mmf.Batch([c[0] for c in cs] + [mmf.grid_desc(2, [2900, 2897], [-1.0, -1.0, 0.0], 1e-3, [4] * 4 + [0, 0])])
+    b.set_shape(chunk, blocks)
+    if tail:
+        b.set_tail(tail)
+    for i, U in enumerate(states):
+        b.set_state(i, U)
+    b.set_time(0.0, [c[3] for c in cs] + [0.0], [c[2] for c in cs] + [0.5])
+    b.advance(STEPS)
+    assert np.array_equal(b.times()[0][:len(cs)], ref.times()[0])
+    for i in range(len(cs)):
+        assert np.array_equal(b.get_state(i), ref.get_state(i)), i
