@@ -14,7 +14,7 @@
 // writing A*F for a cell kernel to sum halves the fluxes, but the 40 bytes per
 // face it writes and the cell kernel reads twice cost more (us per step, with a
 // face kernel / without: 491,520 octree cells 188 / 116, 61,440 66 / 41, 7,680
-// 39 / 42; 3.9 million cells 1341 / 858).  What bounds it now is FP64 issue: 215
+// 39 / 33; 3.9 million cells 1341 / 858).  What bounds it now is FP64 issue: 215
 // instructions per incidence, a third of them the other cell's tuple.
 //
 // dt is known before stage 1 (Ctrl::lam_now): stage 3 gathers the maximum of
@@ -30,7 +30,12 @@
 
 namespace mmf {
 
-constexpr int MB = 256;
+// Cells per block: one wave.  Small meshes do not fill the chip, and their waves
+// wait for the chain of their cells' faces; blocks of four waves leave three
+// CUs of four idle (us per step, four waves / one: octree of 2,512 cells 38.4 /
+// 33.7, with reflecting borders 44.2 / 38.4, 7,680 40.5 / 33.2 and 47.6 / 37.1,
+// 15,000 38.8 / 33.4; 61,440 and 491,520 39.2 and 124, both).
+constexpr int MB = 64;
 
 __device__ __forceinline__ bool mesh_solved(const MeshDev &m, int64_t c) {
   return m.flags == nullptr || (m.flags[c] & CELL_SOLVED);
