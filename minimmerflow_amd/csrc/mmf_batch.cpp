@@ -381,14 +381,9 @@ int mmf_batch_set_state(mmf_batch *b, int32_t ci, const double *U) {
   const BatchCase &c = b->hcases[(size_t)ci];
   const int64_t N = c.g.N, fs = c.g.fs;
   b->lam_valid = false;
-  // the rows cross as they are; the planes are formed on the device, through
-  // the residual's buffer (dead between steps)
-  BCHK(b, hipStreamSynchronize(b->stream));
-  BCHK(b, hipMemcpy(b->dR + c.offset, U, sizeof(double) * 5 * (size_t)N, hipMemcpyHostToDevice));
-  BCHK(b, mmf::launch_aos_to_soa(b->dR + c.offset, nullptr, N, fs, b->dU + c.offset, b->stream));
-  BCHK(b, hipMemcpyAsync(b->dW + c.offset, b->dU + c.offset, sizeof(double) * 5 * (size_t)fs, hipMemcpyDeviceToDevice,
-                         b->stream));
-  BCHK(b, hipStreamSynchronize(b->stream));
+  // through the residual's buffer (dead between steps, as W: stage 2 writes
+  // every cell of it)
+  BCHK(b, mmf::rows_to_planes(U, b->dU + c.offset, nullptr, N, fs, b->dR + c.offset, b->stream));
   return MMF_OK;
 }
 
@@ -396,8 +391,7 @@ int mmf_batch_get_state(mmf_batch *b, int32_t ci, double *U) {
   if (!b || !U || ci < 0 || ci >= b->ncases) return MMF_ERR_INVALID;
   const BatchCase &c = b->hcases[(size_t)ci];
   const int64_t N = c.g.N, fs = c.g.fs;
-  BCHK(b, mmf::launch_soa_to_aos(b->dU + c.offset, nullptr, N, fs, b->dR + c.offset, b->stream));
-  BCHK(b, mmf::copy_to_host(U, b->dR + c.offset, sizeof(double) * 5 * (size_t)N, b->stream));
+  BCHK(b, mmf::planes_to_rows(U, b->dU + c.offset, N, fs, b->dR + c.offset, b->stream));
   return MMF_OK;
 }
 

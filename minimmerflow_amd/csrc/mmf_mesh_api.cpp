@@ -411,22 +411,16 @@ int mmf_mesh_set_cell_flags(mmf_mesh *m, const uint8_t *fluid, const uint8_t *so
 int mmf_mesh_set_state(mmf_mesh *m, const double *U) {
   if (!m || !U) return MMF_ERR_INVALID;
   const int64_t N = m->m.N, fs = m->m.fs;
-  // the rows cross as they are; the planes are formed on the device, through
-  // dR (dead between steps)
-  MCHK(m, hipStreamSynchronize(m->stream));
-  MCHK(m, hipMemcpy(m->dR, U, sizeof(double) * 5 * (size_t)N, hipMemcpyHostToDevice));
-  MCHK(m, mmf::launch_aos_to_soa(m->dR, nullptr, N, fs, m->dU, m->stream));
   m->lam_valid = false;
-  // the stage buffer starts as a copy: cells never solved keep their state in it
-  MCHK(m, hipMemcpyAsync(m->dW, m->dU, sizeof(double) * 5 * (size_t)fs, hipMemcpyDeviceToDevice, m->stream));
+  // through dR (dead between steps); the stage buffer starts as a copy: cells
+  // never solved keep their state in it
+  MCHK(m, mmf::rows_to_planes(U, m->dU, m->dW, N, fs, m->dR, m->stream));
   return MMF_OK;
 }
 
 int mmf_mesh_get_state(mmf_mesh *m, double *U) {
   if (!m || !U) return MMF_ERR_INVALID;
-  const int64_t N = m->m.N;
-  MCHK(m, mmf::launch_soa_to_aos(m->dU, nullptr, N, m->m.fs, m->dR, m->stream));
-  MCHK(m, mmf::copy_to_host(U, m->dR, sizeof(double) * 5 * (size_t)N, m->stream));
+  MCHK(m, mmf::planes_to_rows(U, m->dU, m->m.N, m->m.fs, m->dR, m->stream));
   return MMF_OK;
 }
 

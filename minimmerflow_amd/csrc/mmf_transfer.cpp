@@ -14,6 +14,9 @@
 #include <mutex>
 #include <system_error>
 #include <thread>
+#include <vector>
+
+#include "mmf_internal.hpp"
 
 namespace mmf {
 
@@ -127,6 +130,43 @@ hipError_t copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t s)
     e = nullptr;
   }
   return err;
+}
+
+// Cells below which the host forms the rows, and the planes (us per read-back of
+// one batch case / face list, host and device rows: 1024 cells 26 / 37, 4096 19 /
+// 28, 10,000 32 / 37, 15,000 47 / 46, 40,000 131 / 97; per upload 448 cells 20 / 24,
+// 2512 26 / 27, 7168 40 / 32).
+constexpr int64_t HOST_ROWS_MAX = 12 << 10, HOST_PLANES_MAX = 5 << 10;
+
+hipError_t planes_to_rows(double *rows, const double *soa, int64_t N, int64_t fs, double *scratch, hipStream_t s) {
+  if (N >= HOST_ROWS_MAX) {
+    const hipError_t e = launch_soa_to_aos(soa, nullptr, N, fs, scratch, s);
+    return e != hipSuccess ? e : copy_to_host(rows, scratch, sizeof(double) * 5 * (size_t)N, s);
+  }
+  std::vector<double> planes((size_t)(5 * fs));
+  hipError_t e = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = hipMemcpy(planes.data(), soa, sizeof(double) * planes.size(), hipMemcpyDeviceToHost);
+  if (e != hipSuccess) return e;
+  for (int64_t i = 0; i < N; ++i)
+    for (int k = 0; k < 5; ++k) rows[5 * i + k] = planes[(size_t)(k * fs + i)];
+  return hipSuccess;
+}
+
+hipError_t rows_to_planes(const double *rows, double *soa, double *copy, int64_t N, int64_t fs, double *scratch,
+                          hipStream_t s) {
+  const size_t bytes = sizeof(double) * 5 * (size_t)fs;
+  hipError_t e = hipStreamSynchronize(s);
+  if (e != hipSuccess) return e;
+  if (N >= HOST_PLANES_MAX) {
+    e = hipMemcpy(scratch, rows, sizeof(double) * 5 * (size_t)N, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = launch_aos_to_soa(scratch, nullptr, N, fs, soa, s);
+    return (e != hipSuccess || !copy) ? e : hipMemcpyAsync(copy, soa, bytes, hipMemcpyDeviceToDevice, s);
+  }
+  std::vector<double> planes((size_t)(5 * fs), 0.0);
+  for (int64_t i = 0; i < N; ++i)
+    for (int k = 0; k < 5; ++k) planes[(size_t)(k * fs + i)] = rows[5 * i + k];
+  e = hipMemcpy(soa, planes.data(), bytes, hipMemcpyHostToDevice);
+  return (e != hipSuccess || !copy) ? e : hipMemcpy(copy, planes.data(), bytes, hipMemcpyHostToDevice);
 }
 
 void transfer_attach() {
