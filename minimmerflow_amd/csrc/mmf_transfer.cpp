@@ -12,7 +12,7 @@
 #include <atomic>
 #include <cstring>
 #include <mutex>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <vector>
 
@@ -99,7 +99,7 @@ hipError_t copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t s)
   if (err == hipSuccess) {
     try {
       for (; started < WORKERS; ++started) workers[started] = std::thread([&c] { c.work(); });
-    } catch (const std::system_error &) {  // fewer of them, or this thread alone
+    } catch (const std::exception &) {  // fewer of them, or this thread alone
     }
   }
   size_t issued = 0;
