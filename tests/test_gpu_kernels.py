@@ -341,3 +341,25 @@ def test_early_dt_dirichlet_side_behind_a_body(mmf, covered):
     assert d1g == d1m
     assert tg[:3] == tm[:3] and np.array_equal(tg[3], tm[3]), (tg, tm)
     assert np.array_equal(Ug, Um)
+
+
+@pytest.mark.parametrize("bc", [[0] * 4, [4] * 4, [1, 3, 4, 4]])
+@pytest.mark.parametrize("n", [(59, 30), (60, 33), (61, 41), (121, 40), (185, 70)])
+def test_march2d_order2_counts_each_face_once(mmf, n, bc):
+    """Negative states everywhere: the faces that two strips or two chunks share
+    are evaluated by both and counted once, as the gather kernel counts them."""
+    s, U = build(mmf, 2, list(n), bc, np.tile([1.0, 0.3, -0.1, 0.0, 1.0], (6, 1)), None, order=2, seed=5)
+    U[::3, 0] *= -1.0
+    U[::3, 4] *= -1.0
+    U[1::7, 4] = 0.01
+    out = []
+    for kind, chunk in ((mmf.KERNEL_GATHER, 0), (mmf.KERNEL_MARCH, 8), (mmf.KERNEL_MARCH, 128)):
+        s.set_kernel(kind, 0, chunk)
+        s.set_state(U)
+        s.reset_positivity_counters()
+        rhs, _ = s.compute_rhs()
+        out.append((rhs, s.positivity_counters()))
+    assert out[0][1][0] > 0 and out[0][1][1] > 0
+    for rhs, counts in out[1:]:
+        assert counts == out[0][1]
+        assert np.array_equal(rhs, out[0][0], equal_nan=True)
