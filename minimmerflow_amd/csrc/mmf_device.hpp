@@ -148,7 +148,10 @@ __device__ __forceinline__ void make_tup(const double *c, Tup &t) {
 // range, so inside it a further quotient by the same divisor is three
 // instructions, the same operations on the same operands: the same double
 // (compared with a / b, K / b^2, sqrt and the two constants on 10^9 operands
-// each, mantissas at both ends of their range among them).  The stage kernels
+// each, mantissas at both ends of their range among them; the tests add
+// quotients next to the middle of two doubles and operands at every bound
+// below).  The methods are Newton's for the reciprocal, Markstein's correction
+// of a quotient by its remainder, and Goldschmidt's square root.  The stage kernels
 // issue FP64 instructions three quarters of the time, and a flux tuple's seven
 // divisions were two thirds of it (145 issue slots, 85 this way).
 // ---------------------------------------------------------------------------
