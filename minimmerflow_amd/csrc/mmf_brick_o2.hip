@@ -26,6 +26,7 @@
 // results equal the gather kernel's and the oracle's bit for bit.
 #include <hip/hip_runtime.h>
 
+#include "mmf_brick.hpp"
 #include "mmf_device.hpp"
 #include "mmf_internal.hpp"
 #include "mmf_stage.hpp"
@@ -33,30 +34,6 @@
 namespace mmf {
 
 namespace {
-
-constexpr int NTUP = 11;  // c[5], vel[3], p, a, H
-
-template <int NS>
-__device__ __forceinline__ void put_tup(double *lds, int slot, const Tup &t) {
-#pragma unroll
-  for (int k = 0; k < NF; ++k) lds[k * NS + slot] = t.c[k];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) lds[(5 + a) * NS + slot] = t.vel[a];
-  lds[8 * NS + slot] = t.p;
-  lds[9 * NS + slot] = t.a;
-  lds[10 * NS + slot] = t.H;
-}
-
-template <int NS>
-__device__ __forceinline__ void get_tup(const double *lds, int slot, Tup &t) {
-#pragma unroll
-  for (int k = 0; k < NF; ++k) t.c[k] = lds[k * NS + slot];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) t.vel[a] = lds[(5 + a) * NS + slot];
-  t.p = lds[8 * NS + slot];
-  t.a = lds[9 * NS + slot];
-  t.H = lds[10 * NS + slot];
-}
 
 // LDS written by the lanes of a wave, then read by them: the hardware keeps a
 // wave's LDS operations in order; this keeps the compiler from moving them.
