@@ -576,8 +576,9 @@ class Solver:
         self._c(lib().mmf_reset_positivity_counters(self.ctx))
 
     def enable_timing(self, on=True):
-        """on: True or 1, an event pair per stage launch (steps launched one
-        by one); 2, one pair per advance call with the steps graph-replayed."""
+        """on: True or 1, an event pair per stage launch (steps launched one by
+        one, stage by stage); 2, one pair per advance call with the steps
+        graph-replayed, three stages counted per step."""
         self._c(lib().mmf_enable_timing(self.ctx, int(on)))
 
     def read_timing(self):

@@ -936,8 +936,6 @@ namespace {
 
 constexpr int GRAPH_STEPS = 16;
 
-// Before steps of the 3D marching kernel with early dt: the maximum of the
-// current state, unless the previous steps left it (outside any capture).
 // The 3D marching kernel's tile table on grids with flags (the masked tiles
 // first; the others run the unmasked code).
 int ensure_tiles(mmf_ctx *ctx) {
@@ -995,6 +993,8 @@ int ensure_tiles(mmf_ctx *ctx) {
   return MMF_OK;
 }
 
+// Before steps of a kernel with early dt: the maximum of the current state,
+// unless the previous steps left it (outside any capture).
 int ensure_lam(mmf_ctx *ctx) {
   const int used = kernel_used(ctx);
   const bool early = (used == mmf::KERNEL_MARCH && mmf::march_early(ctx->g)) ||

@@ -8,12 +8,14 @@
 //   - the brick's outer faces need the facing value of the cell beyond, two
 //     per line of cells: 256 lines in 3D (32 in 2D), one per lane, each lane
 //     holding its line's two outer cells, so that all of them take one pass.
-// That is 7 tuples and 3 faces per 3D cell (5 and 2 in 2D).  The gather kernel
-// builds 12 (8) and the marching kernel, which it replaces, 10 on 5 faces.
+// That is 7 tuples and 3 faces per 3D cell (5 and 2 in 2D), the faces above the
+// brick in a second evaluation per axis that fills 8 to 32 lanes of a wave.  The
+// gather kernel builds 12 (8) and the marching kernel, which it replaces, 10 on 5
+// faces.
 // The tuple of a cell's upper face value goes to the next cell, and that
 // cell's lower face flux back, through LDS.  Along x and y both ends are lanes
 // of one wave, whose LDS operations execute in order, so only the z axis has
-// block barriers (two, and one after the states are stored).
+// block barriers (three, and one after the states are stored).
 //
 // Border faces: beyond a non-periodic border the outer cell's slot holds the
 // border cell's own state, so the one-sided difference is zero and with it the

@@ -39,7 +39,7 @@ struct mmf_ctx {
   int timing = 0;
   struct TimedSpan {
     hipEvent_t start, end;
-    int64_t launches;  // stage launches between the two events
+    int64_t launches;  // stages between the two events (three a step)
   };
   std::vector<TimedSpan> events;
   double timed_ms = 0.0;

@@ -24,7 +24,7 @@ struct GridDev {
   double info[6][5];   // Dirichlet primitives per side
   const uint8_t *flags;  // MMF_CELL_* bits per cell, or nullptr (all fluid+solved)
   int32_t ghost_free;    // with flags: every fluid cell is solved (no ghost cells)
-  double invV;         // 1/V, used only when V is a power of two (x/V == x*invV exactly)
+  double invV;         // 1/V: x/V == x*invV exactly where V is a power of two, else quot()'s reciprocal of V
   int32_t pow2V;
   int32_t quotV;       // invV and V are inside the range of quot() (mmf_device.hpp)
   int32_t pow2A;       // A is a power of two: A*(0.5*x) == (0.5*A)*x exactly
@@ -95,10 +95,11 @@ struct Ctrl {
   // holds a NaN or infinity; such a step leaves t, dt and the step count
   // unchanged
   unsigned long long nonfinite;
-  // Early dt (the 3D marching kernel on grids without a body or a reflected
-  // border): the stage-1 maximum of a step, max over cells and axes of
-  // |u_a| + c, known before the step from the state it starts from (bits).
-  // The step's stage-3 launch gathers the next one into lam[k][0].
+  // Early dt (the order-1 brick kernels, the 3D marching kernel where every
+  // fluid cell is solved, the interface list): the stage-1 maximum of a step,
+  // the largest |u_n| + c of both sides of every face, known before the step
+  // from the state it starts from (bits).  The step's stage-3 launch gathers
+  // the next one into lam[k][0].
   unsigned long long lam_now;
   // running stage maxima (bits) in entry [s][k][0], s = 3: compute_rhs; the
   // stage maximum is the largest over k
